@@ -329,12 +329,23 @@ size_t mi355_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int in_dtype,
 }
 
 int mi355_quantize_e4m3(const void* x, int x_dtype, int64_t n, void* x_q, float* scale_amax, void* stream) {
+  return mi355_quantize_e4m3_scratch(x, x_dtype, n, x_q, scale_amax, nullptr, 0, stream);
+}
+
+size_t mi355_quantize_e4m3_scratch_bytes(int64_t n) {
+  return n <= 0 || (double)n > kMaxElements ? 0 : (size_t)mi355::quantize_e4m3_partials(n) * sizeof(float);
+}
+
+int mi355_quantize_e4m3_scratch(const void* x, int x_dtype, int64_t n, void* x_q, float* scale_amax, void* scratch,
+                                size_t scratch_bytes, void* stream) {
   if (x_dtype != MI355_BF16 && x_dtype != MI355_F16 && x_dtype != MI355_F32) return MI355_ERR_DTYPE;
   if (n < 0 || (double)n > kMaxElements) return MI355_ERR_SHAPE;
   if (!scale_amax || (n > 0 && (!x || !x_q))) return MI355_ERR_NULL;
-  if ((uintptr_t)x % 16 != 0 || (uintptr_t)x_q % 8 != 0 || (uintptr_t)scale_amax % 4 != 0) return MI355_ERR_ALIGN;
-  return mi355::launch_quantize_e4m3(x, x_dtype, n, x_q, scale_amax, (hipStream_t)stream) == 0 ? MI355_OK
-                                                                                              : MI355_ERR_LAUNCH;
+  if ((uintptr_t)x % 16 != 0 || (uintptr_t)x_q % 8 != 0 || (uintptr_t)scale_amax % 4 != 0 || (uintptr_t)scratch % 4 != 0)
+    return MI355_ERR_ALIGN;
+  return mi355::launch_quantize_e4m3(x, x_dtype, n, x_q, scale_amax, (float*)scratch,
+                                     scratch ? (int64_t)(scratch_bytes / sizeof(float)) : 0, (hipStream_t)stream) == 0
+             ? MI355_OK : MI355_ERR_LAUNCH;
 }
 
 size_t mi355_mx_shuffled_bytes(int64_t rows, int64_t K) {

@@ -94,8 +94,11 @@ int stream_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx = fal
 int stream_tile_cols(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx = false);  // rows of W per workgroup: 64 or 128
 int launch_stream_mx(const GemmArgs& g, int out_dtype, int splits, void* workspace, hipStream_t stream);
 int launch_stream(const GemmArgs& g, int in_dtype, int out_dtype, int splits, void* workspace, hipStream_t stream);
-// Per-tensor e4m3 quantisation (amax -> scale -> cast); scale_amax points to two floats.
-int launch_quantize_e4m3(const void* x, int in_dtype, int64_t n, void* q, float* scale_amax, hipStream_t stream);
+// Per-tensor e4m3 quantisation (amax -> scale -> cast); scale_amax points to two floats.  partial: scratch memory of
+// `partials` floats, or null; quantize_e4m3_partials(n) is how many the quantiser would like.
+int64_t quantize_e4m3_partials(int64_t n);
+int launch_quantize_e4m3(const void* x, int in_dtype, int64_t n, void* q, float* scale_amax, float* partial, int64_t partials,
+                         hipStream_t stream);
 int launch_simple(const GemmArgs& g, int in_dtype, int out_dtype, hipStream_t stream);
 // Repacking for problems the tiled kernels cannot address (gemm_tn_simple.hip): rows of `row_bytes`
 // bytes with stride src_ld bytes -> 16-byte aligned rows with stride dst_ld bytes, the tail of every

@@ -6,6 +6,7 @@ namespace mi355 {
 
 template <class In> struct Load8;  // 8 consecutive elements -> 8 floats
 template <> struct Load8<float> {
+  typedef float Element;
   static __device__ __forceinline__ void run(const void* p, int64_t i, float* v) {
     const f32x4 a = ((const f32x4*)((const float*)p + i))[0], b = ((const f32x4*)((const float*)p + i))[1];
     v[0] = a[0]; v[1] = a[1]; v[2] = a[2]; v[3] = a[3]; v[4] = b[0]; v[5] = b[1]; v[6] = b[2]; v[7] = b[3];
@@ -13,6 +14,7 @@ template <> struct Load8<float> {
   static __device__ __forceinline__ float one(const void* p, int64_t i) { return ((const float*)p)[i]; }
 };
 template <> struct Load8<BF16> {
+  typedef uint16_t Element;
   static __device__ __forceinline__ void run(const void* p, int64_t i, float* v) {
     const u32x4 a = *(const u32x4*)((const uint16_t*)p + i);
 #pragma unroll
@@ -24,6 +26,7 @@ template <> struct Load8<BF16> {
   static __device__ __forceinline__ float one(const void* p, int64_t i) { return Decode<BF16>::run(p, i); }
 };
 template <> struct Load8<F16> {
+  typedef uint16_t Element;
   static __device__ __forceinline__ void run(const void* p, int64_t i, float* v) {
     const f16x8 a = *(const f16x8*)((const _Float16*)p + i);
 #pragma unroll
@@ -50,20 +53,26 @@ __device__ __forceinline__ uint32_t to_e4m3(float f) {
   return sign | code;
 }
 
-// Four fp32 -> four e4m3 codes in one word (a in the lowest byte), bit for bit what to_e4m3 gives: the hardware
-// conversion (v_cvt_pk_fp8_f32, OCP e4m3 on this GPU, round to nearest even) behind an explicit clamp to +-448.  A NaN
-// is carried around the clamp, which would turn it into a number, and comes out of the conversion as a code whose
-// low seven bits are all ones, as no number does; the sign of such codes is cleared afterwards.
+// Four fp32 of magnitude 448 or a little more (below 464, which is where rounding would pass 448), or NaN, -> four e4m3
+// codes in one word (a in the lowest byte): the hardware conversion (v_cvt_pk_fp8_f32, OCP e4m3 on this GPU, round to
+// nearest even).  A NaN comes out of it as a code whose low seven bits are all ones, as no number does; the sign of such
+// codes is cleared.
+__device__ __forceinline__ uint32_t to_e4m3x4_bounded(float a, float b, float c, float d) {
+  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
+  w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
+  const uint32_t u = (uint32_t)w;
+  const uint32_t nan_sign = ((u & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u;   // bit 7 of the bytes that hold 0x7f or 0xff
+  return u & ~nan_sign;
+}
+
+// Four fp32 -> four e4m3 codes in one word (a in the lowest byte), bit for bit what to_e4m3 gives: the
+// conversion above behind an explicit clamp to +-448.  A NaN is carried around the clamp, which would turn it into a number.
 __device__ __forceinline__ uint32_t to_e4m3x4(float a, float b, float c, float d) {
   const auto clamped = [](float f) __attribute__((always_inline)) {
     const float inside = __builtin_amdgcn_fmed3f(f, -448.0f, 448.0f);
     return f != f ? f : inside;
   };
-  int w = __builtin_amdgcn_cvt_pk_fp8_f32(clamped(a), clamped(b), 0, false);
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(clamped(c), clamped(d), w, true);
-  const uint32_t u = (uint32_t)w;
-  const uint32_t nan_sign = ((u & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u;   // bit 7 of the bytes that hold 0x7f or 0xff
-  return u & ~nan_sign;
+  return to_e4m3x4_bounded(clamped(a), clamped(b), clamped(c), clamped(d));
 }
 
 }  // namespace mi355

@@ -159,9 +159,12 @@ std::pair<torch::Tensor, torch::Tensor> quantize_e4m3(const torch::Tensor x) {
   c10::DeviceGuard guard(x.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
   torch::Tensor q = torch::empty(x.sizes(), x.options().dtype(at::kFloat8_e4m3fn));
-  torch::Tensor sa = torch::empty({2}, x.options().dtype(at::kFloat));
-  int st = mi355_quantize_e4m3(x.const_data_ptr(), dt, x.numel(), q.mutable_data_ptr(), sa.data_ptr<float>(),
-                               (void*)stream);
+  // scale, amax, and behind them the quantiser's scratch memory
+  const size_t scratch = mi355_quantize_e4m3_scratch_bytes(x.numel());
+  torch::Tensor sa = torch::empty({2 + (int64_t)(scratch / sizeof(float))}, x.options().dtype(at::kFloat));
+  float* sa_ptr = sa.data_ptr<float>();
+  int st = mi355_quantize_e4m3_scratch(x.const_data_ptr(), dt, x.numel(), q.mutable_data_ptr(), sa_ptr,
+                                       scratch ? sa_ptr + 2 : nullptr, scratch, (void*)stream);
   TORCH_CHECK(st == MI355_OK, "gemm_kernels: ", mi355_gemm_strerror(st));
   return {q, sa[0]};
 }

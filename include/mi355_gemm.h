@@ -146,12 +146,19 @@ int mi355_gemm_tn_noalloc(const void *A, const void *B, void *C,
  *   x_q        device pointer, n bytes (e4m3), 8-byte aligned
  *   scale_amax device pointer to two floats: [0] receives scale, [1] is scratch (receives amax)
  *
- * Asynchronous on `stream` (three launches, no host synchronisation).  Counterpart in the
- * reference: none; the contract is the fp8 benchmark configuration's (per-tensor fp32 scales
- * amax/448).
+ * Asynchronous on `stream` (one launch for small tensors, otherwise three; no host synchronisation).
+ * Counterpart in the reference: none; the contract is the fp8 benchmark configuration's
+ * (per-tensor fp32 scales amax/448).
+ *
+ * mi355_quantize_e4m3_scratch is the same with scratch memory (4-byte aligned, contents need not be
+ * initialised, not shared with calls that may overlap) of mi355_quantize_e4m3_scratch_bytes(n) bytes,
+ * which spares one of the three launches; with less, or NULL, it runs as mi355_quantize_e4m3 does.
  */
 int mi355_quantize_e4m3(const void *x, int x_dtype, int64_t n, void *x_q,
                         float *scale_amax, void *stream);
+size_t mi355_quantize_e4m3_scratch_bytes(int64_t n);
+int mi355_quantize_e4m3_scratch(const void *x, int x_dtype, int64_t n, void *x_q, float *scale_amax,
+                                void *scratch, size_t scratch_bytes, void *stream);
 
 /*
  * OCP MX block scaling (MXFP8): C = A · B^T where every block of 32 consecutive elements of a row
