@@ -16,7 +16,7 @@ struct GemmArgs {
   float scale;
   // K split: with splits > 1 every (tile, split) pair is a work item that covers k-steps
   // [split*steps/splits, (split+1)*steps/splits) and writes its unscaled fp32 partial tile to
-  // partial[split][M][N]; launch_splitk_reduce then adds the splits in order, scales and rounds.
+  // partial[split][M][partial_columns(N)]; launch_splitk_reduce then adds the splits in order, scales and rounds.
   int32_t splits;
   float* partial;
   // Tail split (single-group tile kernel only, splits == 1): the last tail_tiles tiles in tile-map
@@ -31,10 +31,18 @@ struct GemmArgs {
   // Non-zero when operands and output together exceed what the Infinity Cache holds: the tile kernels then write C
   // with non-temporal stores (tile_store.h).
   int32_t c_streams;
+  // Non-zero when C is to be stored through store_ragged_quad / store_ragged_octet: its rows are aligned by nothing but its
+  // element type, or by less than 64 bytes and this is the faster way (rows_want_plain_stores in gemm_api.hip).  Single-group
+  // tile kernel and streaming kernel only, and not with block scales.
+  int32_t c_ragged;
   // Block scales (MX) of A and of B in the shuffled layout, or null.
   const uint8_t* mx_a;
   const uint8_t* mx_b;
 };
+
+// Columns of a row of fp32 partial sums: planes are [M][N rounded up to 4], so that four sums are one aligned load.  (Rows
+// of B past N read as zeros, so the added columns hold zeros.)
+inline __host__ __device__ int64_t partial_columns(int64_t N) { return (N + 3) / 4 * 4; }
 
 // Effective output scale; wave-uniform, read once per workgroup.
 #if defined(__HIPCC__)
@@ -69,7 +77,7 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
-// C = rne(scale * sum_s partial[s]) for partial laid out [splits][M][N] in fp32.
+// C = rne(scale * sum_s partial[s]) for partial laid out [splits][M][partial_columns(N)] in fp32.
 int launch_splitk_reduce(const float* partial, const GemmArgs& g, int out_dtype, hipStream_t stream);
 int launch_tile_ring(const GemmArgs& g, int in_dtype, int out_dtype, int tile, hipStream_t stream);
 // Tail split the single-group kernel would use for this problem (pure host heuristic): returns the
@@ -80,6 +88,10 @@ int launch_tile_ring_mx(const GemmArgs& g, int out_dtype, int tile, hipStream_t 
 int launch_tile_ring_bf16(const GemmArgs& g, int out_dtype, int tile, hipStream_t stream);
 int launch_tile_ring_f16(const GemmArgs& g, int out_dtype, int tile, hipStream_t stream);
 int launch_tile_ring_e4m3(const GemmArgs& g, int out_dtype, int tile, hipStream_t stream);
+// The same with g.c_ragged set.
+int launch_tile_ring_bf16_ragged(const GemmArgs& g, int out_dtype, int tile, hipStream_t stream);
+int launch_tile_ring_f16_ragged(const GemmArgs& g, int out_dtype, int tile, hipStream_t stream);
+int launch_tile_ring_e4m3_ragged(const GemmArgs& g, int out_dtype, int tile, hipStream_t stream);
 // Block scales: bytes of the shuffled layout for `rows` rows and K elements per row; the shuffle
 // itself (natural (rows, K/32) row-major bytes -> shuffled); and the MX quantiser
 // (x (rows, K) -> e4m3 elements + natural-layout E8M0 scales).
@@ -100,13 +112,15 @@ int64_t quantize_e4m3_partials(int64_t n);
 int launch_quantize_e4m3(const void* x, int in_dtype, int64_t n, void* q, float* scale_amax, float* partial, int64_t partials,
                          hipStream_t stream);
 int launch_simple(const GemmArgs& g, int in_dtype, int out_dtype, hipStream_t stream);
-// Repacking for problems the tiled kernels cannot address (gemm_tn_simple.hip): rows of `row_bytes`
-// bytes with stride src_ld bytes -> 16-byte aligned rows with stride dst_ld bytes, the tail of every
-// row and the rows from `rows` up to dst_rows zero-filled; and a (rows x cols) block of 16-bit
-// elements with row stride src_ld elements -> row stride dst_ld elements at any 2-byte alignment.
-int launch_repack_rows(const void* src, int64_t rows, int64_t row_bytes, int64_t src_ld, void* dst, int64_t dst_rows,
-                       int64_t dst_ld, int elem_bytes, hipStream_t stream);
-int launch_copy_out(const void* src, int64_t rows, int64_t cols, int64_t src_ld, void* dst, int64_t dst_ld,
-                    hipStream_t stream);
+// Repacking for problems the tiled kernels cannot address (gemm_tn_simple.hip): rows of `row_bytes` bytes with stride
+// src_ld bytes -> 16-byte aligned rows with stride dst_ld bytes, the tail of every row filled with zeros.  One or two
+// operands in one launch (second.rows == 0: only the first).
+struct RepackOperand {
+  const uint8_t* src;
+  int64_t rows, src_ld;
+  uint8_t* dst;
+  int64_t dst_ld;
+};
+int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, int64_t row_bytes, int elem_bytes, hipStream_t stream);
 
 }  // namespace mi355

@@ -43,7 +43,8 @@
 // (TMA producer warpgroup, mbarrier full/empty ring of 3 stages, two consumer warpgroups); here
 // every wave is loader and math at once because direct-to-LDS loads need no registers.
 //
-// This header holds the kernel and its launch templates; gemm_tn_ring_{bf16,f16,e4m3,mx}.hip
+// This header holds the kernel and its launch templates; gemm_tn_ring_{bf16,f16,e4m3,mx}.hip and,
+// for rows of C without alignment, gemm_tn_ring_{bf16,f16,e4m3}_ragged.hip
 // instantiate them per input type, one translation unit each so that they compile in parallel.
 #pragma once
 #include "gemm_launch.h"
@@ -91,7 +92,7 @@ constexpr uint32_t kMxUnitBytes = 512;
 // before the barrier that waits for it (a third of a microsecond on the small tile), with d = 4
 // about three.
 template <class T, class OutT, bool kRaggedK, int kTileT, int kWavesN = 2, int kTileNT = kTileT, int kAhead = 2,
-          bool kRotateT = (kAhead > 2)>
+          bool kRotateT = (kAhead > 2), bool kRaggedC = false>
 __global__ __launch_bounds__(threads_of(kWavesN), (kTileT == 256 || kAhead > 2) ? 1 : 2) void gemm_tn_tile_ring(GemmArgs g) {
   constexpr int kSlots = 2 * kAhead + 1;          // shadows the five of ring_common.h
   constexpr int kTile = kTileT;                   // rows of A per workgroup
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(threads_of(kWavesN), (kTileT == 256 || kAhead > 2) 
   const float scale = output_scale(g);
   constexpr bool kAsmMfma = kTile == 256 || kMx;  // see mfma_u; the scaled MFMA is always inline assembly
   auto epilogue = [&](int64_t m0, int64_t n0) __attribute__((always_inline)) {
-    store_output_tile<G, OutT, kNbM, kNbN, kAsmMfma>(acc, g, m0, n0, kTile, kTileN, wm * kWaveTileM, wn * kWaveTileN, lane, scale);
+    store_output_tile<G, OutT, kNbM, kNbN, kAsmMfma, kRaggedC>(acc, g, m0, n0, kTile, kTileN, wm * kWaveTileM, wn * kWaveTileN, lane, scale);
   };
   auto store_partial = [&](int64_t m0, int64_t n0, uint32_t split, uint32_t tile_no) __attribute__((always_inline)) {
     if (tail_tiles) {
@@ -380,11 +381,11 @@ __global__ __launch_bounds__(threads_of(kWavesN), (kTileT == 256 || kAhead > 2) 
       float* base = g.partial + ((int64_t)split * tail_tiles + (tile_no - whole_tiles)) * (kTile * kTileN);
       store_partial_tile<G, kNbM, kNbN, kAsmMfma>(acc, base, kTileN, kTile, kTileN, wm * kWaveTileM, wn * kWaveTileN, lane);
     } else {
-      // plane `split` of M x N floats, clipped at the matrix edge
-      const int64_t rows = g.M - m0 < kTile ? g.M - m0 : kTile;
-      const uint32_t cols = (uint32_t)(g.N - n0 < kTileN ? g.N - n0 : kTileN);
-      float* base = g.partial + ((int64_t)split * g.M + m0) * g.N + n0;
-      store_partial_tile<G, kNbM, kNbN, kAsmMfma>(acc, base, (uint32_t)g.N, rows, cols, wm * kWaveTileM, wn * kWaveTileN, lane);
+      // plane `split` of M x partial_columns(N) floats, clipped at the matrix edge
+      const int64_t rows = g.M - m0 < kTile ? g.M - m0 : kTile, ldp = partial_columns(g.N);
+      const uint32_t cols = (uint32_t)(ldp - n0 < kTileN ? ldp - n0 : kTileN);
+      float* base = g.partial + ((int64_t)split * g.M + m0) * ldp + n0;
+      store_partial_tile<G, kNbM, kNbN, kAsmMfma>(acc, base, (uint32_t)ldp, rows, cols, wm * kWaveTileM, wn * kWaveTileN, lane);
     }
   };
 
@@ -594,16 +595,19 @@ __global__ __launch_bounds__(256) void tail_reduce(GemmArgs g) {
   tile_coord_t<uint32_t>((uint32_t)(g.tiles_m * g.tiles_n) - (uint32_t)g.tail_tiles + t, (uint32_t)g.tiles_m,
                          (uint32_t)g.tiles_n, &tile_m, &tile_n);
   const int64_t m = (int64_t)tile_m * kTileT + r, n = (int64_t)tile_n * kTileNT + c;
-  if (m >= g.M || n >= g.N) return;  // N % 4 == 0: a quad is in or out as a whole
+  if (m >= g.M || n >= g.N) return;
   const float* p = g.partial + (int64_t)t * (kTileT * kTileNT) + r * kTileNT + c;
   const int64_t split_stride = (int64_t)g.tail_tiles * (kTileT * kTileNT);
   f32x4 sum = *(const f32x4*)p;
   for (int s = 1; s < g.tail_splits; ++s) sum += *(const f32x4*)(p + s * split_stride);
   const float scale = output_scale(g);
-  *(u32x2*)((uint16_t*)g.C + m * g.ldc + n) = Pack4<OutT>::run(sum[0] * scale, sum[1] * scale, sum[2] * scale, sum[3] * scale);
+  const u32x2 out = Pack4<OutT>::run(sum[0] * scale, sum[1] * scale, sum[2] * scale, sum[3] * scale);
+  uint16_t* dst = (uint16_t*)g.C + m * g.ldc + n;
+  if (g.c_ragged) store_ragged_quad(dst, out, g.N - n);
+  else *(u32x2*)dst = out;   // N % 4 == 0: a quad is in or out as a whole
 }
 
-template <class T, class OutT, int kTileT, int kTileNT = kTileT, int kAhead = 2, int kWavesN = 2, bool kRotateT = (kAhead > 2)>
+template <class T, class OutT, bool kRaggedC, int kTileT, int kTileNT = kTileT, int kAhead = 2, int kWavesN = 2, bool kRotateT = (kAhead > 2)>
 int launch_tile(const GemmArgs& g, hipStream_t stream) {
   const int64_t items = g.tail_tiles ? g.tiles_m * g.tiles_n + (int64_t)g.tail_tiles * (g.tail_splits - 1)
                                      : g.tiles_m * g.tiles_n * g.splits;
@@ -611,10 +615,10 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
   const int64_t slots = (int64_t)compute_units() * ((kTileT == 256 || kAhead > 2) ? 1 : 2);  // resident workgroups (LDS-bound)
   const int64_t blocks = items < slots ? items : slots;
   if ((g.K * T::kBytes) % kRowBytes == 0) {
-    hipLaunchKernelGGL((gemm_tn_tile_ring<T, OutT, false, kTileT, kWavesN, kTileNT, kAhead, kRotateT>), dim3((unsigned)blocks), dim3(threads_of(kWavesN)), 0, stream, g);
+    hipLaunchKernelGGL((gemm_tn_tile_ring<T, OutT, false, kTileT, kWavesN, kTileNT, kAhead, kRotateT, kRaggedC>), dim3((unsigned)blocks), dim3(threads_of(kWavesN)), 0, stream, g);
   } else {
     if constexpr (std::is_same<T, MxE4M3>::value) return -1;  // block scales need whole k-steps (host check)
-    else hipLaunchKernelGGL((gemm_tn_tile_ring<T, OutT, true, kTileT, kWavesN, kTileNT, kAhead, kRotateT>), dim3((unsigned)blocks), dim3(threads_of(kWavesN)), 0, stream, g);
+    else hipLaunchKernelGGL((gemm_tn_tile_ring<T, OutT, true, kTileT, kWavesN, kTileNT, kAhead, kRotateT, kRaggedC>), dim3((unsigned)blocks), dim3(threads_of(kWavesN)), 0, stream, g);
   }
   if (hipGetLastError() != hipSuccess) return -1;
   if (g.splits > 1)
@@ -627,16 +631,17 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
   return 0;
 }
 
-template <class T, class OutT>
+// kRaggedC: the form that stores rows of C at any 2-byte alignment (g.c_ragged).
+template <class T, class OutT, bool kRaggedC = false>
 int launch(const GemmArgs& g, int tile, hipStream_t stream) {
-  if (tile == kRingTile256x128) return launch_tile<T, OutT, 256, 128>(g, stream);
+  if (tile == kRingTile256x128) return launch_tile<T, OutT, kRaggedC, 256, 128>(g, stream);
   if (tile == kRingTile128Deep || tile == kRingTile128DeepPlain) {
     // the planner does not pick these with block scales (their registers are timed for five slots)
     if constexpr (std::is_same<T, MxE4M3>::value) return -1;
-    else if (tile == kRingTile128Deep) return launch_tile<T, OutT, 128, 128, 4>(g, stream);
-    else return launch_tile<T, OutT, 128, 128, 4, 2, false>(g, stream);
+    else if (tile == kRingTile128Deep) return launch_tile<T, OutT, kRaggedC, 128, 128, 4>(g, stream);
+    else return launch_tile<T, OutT, kRaggedC, 128, 128, 4, 2, false>(g, stream);
   }
-  return tile == 128 ? launch_tile<T, OutT, 128>(g, stream) : launch_tile<T, OutT, 256>(g, stream);
+  return tile == 128 ? launch_tile<T, OutT, kRaggedC, 128>(g, stream) : launch_tile<T, OutT, kRaggedC, 256>(g, stream);
 }
 
 }  // namespace

@@ -1,8 +1,8 @@
 // One thread per output element: C[m][n] = rne(scale * sum_k A[m][k] * B[n][k]) with a serial
 // fp32 fused-multiply-add chain over k.  Handles every shape, stride and dtype the ABI accepts;
 // it is the library's on-device cross-check for the MFMA kernels and the path for shapes they
-// reject.  Also here: the two copy kernels with which the library repacks such a problem into an
-// aligned one when the caller lends it the memory (gemm_api.hip).  Counterpart in the reference:
+// reject.  Also here: the copy kernel with which the library repacks the operands of such a problem
+// into aligned ones when the caller lends it the memory (gemm_api.hip).  Counterpart in the reference:
 // none (its only kernel rejects such shapes, kernels/gemm_kernels/sm90a/gemm_test.cu:33-41).
 #include "cdna4_primitives.h"
 #include "gemm_launch.h"
@@ -27,42 +27,48 @@ __global__ __launch_bounds__(256) void gemm_tn_simple(GemmArgs g) {
   }
 }
 
-// One thread per 16-byte chunk of the destination.  The source has only element alignment, so it is
-// read element by element (the loads of neighbouring threads still coalesce).
+// Sixteen source bytes of a row from byte `at` on, zeros from row_bytes on.  The source has only element alignment: the
+// compiler may use one wide load (global accesses need no alignment on this target).
 template <class E>
-__global__ __launch_bounds__(256) void repack_rows(const uint8_t* __restrict__ src, int64_t rows, int64_t row_bytes,
-                                                   int64_t src_ld, uint8_t* __restrict__ dst, int64_t dst_rows,
-                                                   int64_t dst_ld) {
-  constexpr int kPer = 16 / (int)sizeof(E);
-  const int64_t chunks_per_row = dst_ld / 16;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= dst_rows * chunks_per_row) return;
-  const int64_t row = id / chunks_per_row, at = (id % chunks_per_row) * 16;
-  E v[kPer];
+__device__ __forceinline__ u32x4 row_chunk(const uint8_t* row, uint32_t at, uint32_t row_bytes) {
+  u32x4 out = {0u, 0u, 0u, 0u};
+  if (at + 16 <= row_bytes) {
+    __builtin_memcpy(&out, row + at, 16);
+  } else if (at < row_bytes) {
+    E v[16 / sizeof(E)];
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    const int64_t byte = at + i * (int64_t)sizeof(E);
-    v[i] = row < rows && byte < row_bytes ? *(const E*)(src + row * src_ld + byte) : (E)0;
+    for (uint32_t i = 0; i < 16 / sizeof(E); ++i) {
+      const uint32_t byte = at + i * (uint32_t)sizeof(E);
+      v[i] = byte < row_bytes ? *(const E*)(row + byte) : (E)0;
+    }
+    __builtin_memcpy(&out, v, 16);
   }
-  u32x4 out;
-  __builtin_memcpy(&out, v, 16);
-  *(u32x4*)(dst + row * dst_ld + at) = out;
+  return out;
 }
 
-// One thread per four columns: the source rows are 8-byte aligned (src_ld % 4 == 0), the
-// destination has only element alignment.
-__global__ __launch_bounds__(256) void copy_out(const uint16_t* __restrict__ src, int64_t rows, int64_t cols,
-                                                int64_t src_ld, uint16_t* __restrict__ dst, int64_t dst_ld) {
-  const int64_t quads = (cols + 3) / 4;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= rows * quads) return;
-  const int64_t row = id / quads, col = (id % quads) * 4;
-  const u32x2 v = *(const u32x2*)(src + row * src_ld + col);
-  uint16_t* d = dst + row * dst_ld + col;
-  d[0] = (uint16_t)v[0];
-  if (col + 1 < cols) d[1] = (uint16_t)(v[0] >> 16);
-  if (col + 2 < cols) d[2] = (uint16_t)v[1];
-  if (col + 3 < cols) d[3] = (uint16_t)(v[1] >> 16);
+// Bound by its read and its write: kChunks 16-byte chunks of the destination per thread, all loads out before the first
+// store; one or two operands per launch.
+constexpr int kChunks = 4;
+template <class E>
+__global__ __launch_bounds__(256) void repack_rows(RepackOperand first, RepackOperand second, uint32_t row_bytes,
+                                                   uint32_t first_blocks) {
+  const bool is_second = blockIdx.x >= first_blocks;
+  const RepackOperand& op = is_second ? second : first;
+  const uint32_t per_row = (uint32_t)(op.dst_ld / 16);
+  const uint32_t begin = (is_second ? blockIdx.x - first_blocks : blockIdx.x) * (256 * kChunks) + threadIdx.x;
+  const uint32_t total = (uint32_t)op.rows * per_row;      // below 2^31 (host check)
+  u32x4 v[kChunks];
+  int64_t to[kChunks];
+#pragma unroll
+  for (int i = 0; i < kChunks; ++i) {
+    const uint32_t id = begin + i * 256;
+    const uint32_t row = id / per_row, at = (id % per_row) * 16;
+    to[i] = id < total ? (int64_t)row * op.dst_ld + at : -1;
+    if (id < total) v[i] = row_chunk<E>(op.src + (int64_t)row * op.src_ld, at, row_bytes);
+  }
+#pragma unroll
+  for (int i = 0; i < kChunks; ++i)
+    if (to[i] >= 0) *(u32x4*)(op.dst + to[i]) = v[i];
 }
 
 template <class T, class OutT>
@@ -75,29 +81,21 @@ int launch(const GemmArgs& g, hipStream_t stream) {
 
 }  // namespace
 
-int launch_repack_rows(const void* src, int64_t rows, int64_t row_bytes, int64_t src_ld, void* dst, int64_t dst_rows,
-                       int64_t dst_ld, int elem_bytes, hipStream_t stream) {
-  const int64_t chunks = dst_rows * (dst_ld / 16);
-  if (chunks == 0) return 0;
-  const int64_t blocks = (chunks + 255) / 256;
-  if (blocks >= ((int64_t)1 << 31) || dst_ld % 16 != 0) return -1;
-  if (elem_bytes == 2)
-    hipLaunchKernelGGL(repack_rows<uint16_t>, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint8_t*)src, rows,
-                       row_bytes, src_ld, (uint8_t*)dst, dst_rows, dst_ld);
-  else
-    hipLaunchKernelGGL(repack_rows<uint8_t>, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint8_t*)src, rows,
-                       row_bytes, src_ld, (uint8_t*)dst, dst_rows, dst_ld);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-int launch_copy_out(const void* src, int64_t rows, int64_t cols, int64_t src_ld, void* dst, int64_t dst_ld,
-                    hipStream_t stream) {
-  const int64_t n = rows * ((cols + 3) / 4);
-  if (n == 0) return 0;
-  const int64_t blocks = (n + 255) / 256;
-  if (blocks >= ((int64_t)1 << 31) || src_ld % 4 != 0 || (uintptr_t)src % 8 != 0) return -1;
-  hipLaunchKernelGGL(copy_out, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)src, rows, cols, src_ld,
-                     (uint16_t*)dst, dst_ld);
+int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, int64_t row_bytes, int elem_bytes, hipStream_t stream) {
+  uint32_t blocks[2];
+  const RepackOperand* ops[2] = {&first, &second};
+  for (int i = 0; i < 2; ++i) {
+    const RepackOperand& o = *ops[i];
+    if (o.rows == 0) {
+      blocks[i] = 0;
+      continue;
+    }
+    if (o.dst_ld % 16 != 0 || o.dst_ld >= ((int64_t)1 << 31) || o.rows >= ((int64_t)1 << 31) / (o.dst_ld / 16)) return -1;
+    blocks[i] = (uint32_t)((o.rows * (o.dst_ld / 16) + 256 * kChunks - 1) / (256 * kChunks));
+  }
+  if (blocks[0] + blocks[1] == 0) return 0;
+  const auto kernel = elem_bytes == 2 ? repack_rows<uint16_t> : repack_rows<uint8_t>;
+  hipLaunchKernelGGL(kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, stream, first, second, (uint32_t)row_bytes, blocks[0]);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

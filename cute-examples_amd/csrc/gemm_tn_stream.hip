@@ -16,7 +16,7 @@
 //     with four consecutive n of one m;
 //   * workgroups start their k-steps at different points and wrap around, so that they do not all
 //     read the same column of rows a power of two apart (the same memory channels) at once;
-//   * with K split S ways the partial tiles go to an fp32 workspace [S][M][N] and a second kernel
+//   * with K split S ways the partial tiles go to an fp32 workspace [S][M][N rounded up to 4] and a second kernel
 //     adds them in a fixed order (deterministic), scales and rounds; with S = 1 the tile is
 //     rounded and stored directly.
 //
@@ -77,6 +77,9 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_stream(GemmArgs g, float* pa
   const int64_t tile_m = blockIdx.x % tiles_m, tile_n = blockIdx.x / tiles_m;
   const int64_t m0 = tile_m * kTm, n0 = tile_n * kTn;
   const uint32_t split = blockIdx.y;
+  // Read here and not behind the k loop, where the wait for it would be a part of every call (bf16 16 x 14336 x 4096: 1 %).
+  const int c_ragged = __builtin_amdgcn_readfirstlane(g.c_ragged);
+  asm volatile("" ::"s"(c_ragged));
 
   const uint32_t ldx_b = (uint32_t)(g.lda * T::kBytes), ldw_b = (uint32_t)(g.ldb * T::kBytes);
   const uint32_t k_bytes = (uint32_t)(g.K * T::kBytes);
@@ -230,19 +233,21 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_stream(GemmArgs g, float* pa
 #pragma unroll
     for (int j = 0; j < kNB; ++j) {
       const int64_t n = n0 + (wn * kNB + j) * 16 + grp * 4;
-      if (n + 4 > g.N) continue;
+      if (n >= g.N) continue;      // N % 4 == 0 unless C is ragged
       // A wave has at most sixteen of these stores: each one's data registers are simply held over
       // the wait states a wide store wants before they may be rewritten (see hold_previous).
       if (partial) {
         u32x4 data = __builtin_bit_cast(u32x4, acc[i][j]);
         asm volatile("" : "+v"(data));
-        *(u32x4*)(partial + ((int64_t)split * g.M + m) * g.N + n) = data;
+        *(u32x4*)(partial + ((int64_t)split * g.M + m) * partial_columns(g.N) + n) = data;
         hold_last(data);
       } else {
         const float sc = output_scale(g);
         u32x2 data = Pack4<OutT>::run(acc[i][j][0] * sc, acc[i][j][1] * sc, acc[i][j][2] * sc, acc[i][j][3] * sc);
         asm volatile("" : "+v"(data));
-        *(u32x2*)((uint16_t*)g.C + m * g.ldc + n) = data;
+        uint16_t* c = (uint16_t*)g.C + m * g.ldc + n;
+        if (c_ragged) store_ragged_quad(c, data, g.N - n);
+        else *(u32x2*)c = data;
         hold_last(data);
       }
     }
@@ -253,9 +258,11 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_stream(GemmArgs g, float* pa
 template <class OutT>
 __global__ __launch_bounds__(256) void splitk_reduce(const float* partial, GemmArgs g) {
   uint16_t* C = (uint16_t*)g.C;
-  const int64_t M = g.M, N = g.N, ldc = g.ldc;
+  const int64_t M = g.M, N = partial_columns(g.N), ldc = g.ldc;
   const int splits = g.splits;
   const float scale = output_scale(g);
+  const int c_ragged = __builtin_amdgcn_readfirstlane(g.c_ragged);
+  asm volatile("" ::"s"(c_ragged));   // not at the end of the kernel, as in gemm_tn_stream
   const int64_t quads_per_row = N / 4;
   const int64_t q = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (q >= M * quads_per_row) return;
@@ -272,7 +279,9 @@ __global__ __launch_bounds__(256) void splitk_reduce(const float* partial, GemmA
 #pragma unroll
     for (int i = 0; i < 4; ++i) sum = s0 + i < splits ? sum + t[i] : sum;
   }
-  *(u32x2*)(C + m * ldc + n) = Pack4<OutT>::run(sum[0] * scale, sum[1] * scale, sum[2] * scale, sum[3] * scale);
+  const u32x2 out = Pack4<OutT>::run(sum[0] * scale, sum[1] * scale, sum[2] * scale, sum[3] * scale);
+  if (c_ragged) store_ragged_quad(C + m * ldc + n, out, g.N - n);
+  else *(u32x2*)(C + m * ldc + n) = out;
 }
 
 template <class T, class OutT, int kMB, int kNB, int kWM, int kWN, int kDepth>
@@ -422,7 +431,7 @@ int stream_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx) {
 }
 
 int launch_splitk_reduce(const float* partial, const GemmArgs& g, int out_dtype, hipStream_t stream) {
-  const int64_t quads = g.M * (g.N / 4);
+  const int64_t quads = g.M * (partial_columns(g.N) / 4);
   const dim3 grid((unsigned)((quads + 255) / 256));
   if (out_dtype == 0) hipLaunchKernelGGL((splitk_reduce<BF16>), grid, dim3(256), 0, stream, partial, g);
   else hipLaunchKernelGGL((splitk_reduce<F16>), grid, dim3(256), 0, stream, partial, g);

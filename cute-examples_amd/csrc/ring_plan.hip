@@ -274,9 +274,9 @@ size_t ring_tail(int64_t M, int64_t N, int64_t K, int elem_bytes, int* tail_tile
 
 int launch_tile_ring(const GemmArgs& g, int in_dtype, int out_dtype, int tile, hipStream_t stream) {
   switch (in_dtype) {
-    case 0: return launch_tile_ring_bf16(g, out_dtype, tile, stream);
-    case 1: return launch_tile_ring_f16(g, out_dtype, tile, stream);
-    case 2: return launch_tile_ring_e4m3(g, out_dtype, tile, stream);
+    case 0: return g.c_ragged ? launch_tile_ring_bf16_ragged(g, out_dtype, tile, stream) : launch_tile_ring_bf16(g, out_dtype, tile, stream);
+    case 1: return g.c_ragged ? launch_tile_ring_f16_ragged(g, out_dtype, tile, stream) : launch_tile_ring_f16(g, out_dtype, tile, stream);
+    case 2: return g.c_ragged ? launch_tile_ring_e4m3_ragged(g, out_dtype, tile, stream) : launch_tile_ring_e4m3(g, out_dtype, tile, stream);
   }
   return -1;
 }

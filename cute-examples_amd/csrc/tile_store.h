@@ -34,7 +34,9 @@ __device__ __forceinline__ void pin_acc_block(Acc& a) {
 
 // The wave's part of the output tile at (m0, n0), tile_rows x tile_cols at most.
 // wave_row / wave_col: first row / column of the wave inside the tile.
-template <class G, class OutT, int kNbM, int kNbN, bool kAsmRead>
+// kRaggedC: rows of C at any 2-byte alignment (g.c_ragged).  A form of its own and not a branch: with a third form of this
+// phase in one kernel the compiler lifts accumulator reads in front of the choice, into the last MFMAs.
+template <class G, class OutT, int kNbM, int kNbN, bool kAsmRead, bool kRaggedC = false>
 __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][kNbN], const GemmArgs& g,
                                                   int64_t m0, int64_t n0, int tile_rows, int tile_cols,
                                                   uint32_t wave_row, uint32_t wave_col, uint32_t lane, float scale) {
@@ -96,7 +98,54 @@ __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][k
       }
     });
   };
-  if (cols == (uint32_t)tile_cols) {
+  if constexpr (kRaggedC && !kAsmRead) {
+    // Rows at any alignment: global stores (a raw buffer store has to be dword-aligned), predicated by hand where the
+    // descriptor would have clipped, and without the write-through policy below: a 64-byte run that straddles cache lines is
+    // better put together in the L2 than written through in parts (figures at rows_want_plain_stores in gemm_api.hip).
+    uint8_t* tile = (uint8_t*)g.C + (m0 * g.ldc + n0) * 2;
+    convert([&](auto ic, auto colc, u32x2 x, u32x2 y) __attribute__((always_inline)) {
+      constexpr int i = decltype(ic)::value, col = decltype(colc)::value;
+      u32x4 data = {x[0], x[1], y[0], y[1]};
+      asm volatile("" : "+v"(data));
+      if ((int64_t)(wave_row + rblk + i * kBlk) < rows)
+        store_ragged_octet((uint16_t*)(tile + (v0 + i * block_step + col * 2)), data, (int64_t)cols - (col0 + col));
+      hold_last(data);   // eight of these per wave at most
+    });
+  } else if constexpr (kRaggedC) {
+    // The same through the descriptor and without a branch between the stores, which 256 live accumulator registers do not
+    // tolerate (the register allocator then moves some through vector registers in the k loop): 16 bytes at a time where rows
+    // are dword-aligned and the tile is whole, else one element at a time, lanes past N sent out of range.
+    u32x4 previous = {0u, 0u, 0u, 0u}, before = {0u, 0u, 0u, 0u};
+    if (cols == (uint32_t)tile_cols && ((ldc_b | (uint32_t)(uintptr_t)g.C) & 3u) == 0) {
+      asm volatile("; C in wide pieces" : "+v"(factor));
+      convert([&](auto ic, auto colc, u32x2 x, u32x2 y) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, col = decltype(colc)::value;
+        u32x4 data = {x[0], x[1], y[0], y[1]};
+        hold_previous(data, previous, before);
+        __builtin_amdgcn_raw_buffer_store_b128(data, rc, v0 + col * 2, i * block_step, 0);
+        MI355_FENCE();
+        before = previous;
+        previous = data;
+      });
+      hold_last(previous);
+    } else {
+      asm volatile("; C element by element" : "+v"(factor));
+      convert([&](auto ic, auto colc, u32x2 x, u32x2 y) __attribute__((always_inline)) {
+        constexpr int i = decltype(ic)::value, col = decltype(colc)::value;
+        u32x4 data = {x[0], x[1], y[0], y[1]};
+        hold_previous(data, previous, before);
+        static_for<8>([&](auto ec) __attribute__((always_inline)) {
+          constexpr int e = decltype(ec)::value;
+          const uint32_t v = col0 + col + e < cols ? v0 + (col + e) * 2 : kStoreOutOfRange;
+          __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(data[e / 2] >> (16 * (e % 2))), rc, v, i * block_step, 0);
+        });
+        MI355_FENCE();
+        before = previous;
+        previous = data;
+      });
+      hold_last(previous);
+    }
+  } else if (cols == (uint32_t)tile_cols) {
     auto whole_rows = [&](auto auxc) __attribute__((always_inline)) {
       // The two forms of this phase differ in one bit of their stores.  Each takes the scale through a statement of
       // its own, so that the compiler cannot lift the first conversions, which would otherwise be the same in both,

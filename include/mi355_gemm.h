@@ -72,9 +72,11 @@ enum mi355_status {
  *             variant needs it for its K split (MI355_ERR_WORKSPACE otherwise); the tiled variant
  *             runs without its K split or tail split, i.e. slower, when it is NULL or too small,
  *             and MI355_VARIANT_AUTO then uses the tiled variant also where it would stream.
- *             MI355_VARIANT_AUTO also uses it (256-byte aligned) to repack a large problem the
- *             tiled kernels cannot address (K*elem_bytes % 16, N % 4, strides, pointers) into
- *             an aligned one; without it such a problem runs on the slow generic kernel
+ *             MI355_VARIANT_AUTO also uses it (256-byte aligned) to repack the operands of a large
+ *             problem the tiled kernels cannot address (K*elem_bytes % 16, strides, pointers);
+ *             without it such a problem, or a large one with N or ldc % 4 != 0, runs on the slow
+ *             generic kernel.  With it, an output whose rows only its element type aligns is stored
+ *             by the tiled kernels directly (mi355_gemm_select_variant still reports SIMPLE)
  *   stream    hipStream_t on which the kernels are enqueued (NULL = the null stream)
  *
  * Replaces test::gemm_tn_test (kernels/gemm_kernels/sm90a/gemm_test.cu:12-92): same operand
