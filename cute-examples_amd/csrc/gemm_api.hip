@@ -147,11 +147,17 @@ struct Repack {
 
 size_t round_up(size_t x, size_t to) { return (x + to - 1) / to * to; }
 
+constexpr double kRepackMinFlops = 134217728.0;   // below, repacking is not worth its launches
+// From here on such a small problem runs on gemm_tn_small instead of the generic kernel.  Both timed at M = 1...2048 and 1 to 67
+// million products: K = 65 small 0.5-1.0 of the generic kernel's speed, K = 129 1.0-1.7, 257 2.0-3.5, 513 3.9-7.7, 1025 7-16
+// times (bf16 16 x 4025 x 1025 128 -> 13 us), 14335 51-157 times (bf16 16 x 287 x 14335 1808 -> 33 us).
+constexpr int64_t kSmallMinK = 128;
+
 bool repack_plan(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
                  int64_t ldb, int64_t ldc, int in_dtype, Repack* r) {
   const int64_t es = elem_bytes(in_dtype);
   if (M <= 0 || N <= 0 || K <= 0) return false;
-  if (2.0 * (double)M * (double)N * (double)K < 134217728.0) return false;   // under ~0.1 ms on the generic kernel
+  if (2.0 * (double)M * (double)N * (double)K < kRepackMinFlops) return false;
   const int64_t per16 = 16 / es;
   r->Kp = (K + per16 - 1) / per16 * per16;
   r->Np = (N + 3) / 4 * 4;
@@ -699,6 +705,18 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   if (ab_aligned && tile256_ok(M, Np, K, lda, ldb, ldc4, in_dtype)) {
     *handled = true;
     return product(A, B, K, lda, ldb, workspace, workspace_bytes);
+  }
+  if (!large && K >= kSmallMinK && (uintptr_t)A % es == 0 && (uintptr_t)B % es == 0 && 2.0 * (double)M * (double)N * (double)K < kRepackMinFlops) {
+    *handled = true;
+    if (mode == kStrictDry) return MI355_OK;
+    mi355::GemmArgs g = {};
+    g.A = A; g.B = B; g.C = C;
+    g.M = M; g.N = N; g.K = K;
+    g.lda = lda; g.ldb = ldb; g.ldc = ldc;
+    g.scale = scale;
+    g.scale_a = scale_a;
+    g.scale_b = scale_b;
+    return mi355::launch_small(g, in_dtype, out_dtype, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
   }
   if (!large || !(r.a || r.b)) return MI355_OK;
   if (!tile256_ok(M, r.Np, r.Kp, r.a ? r.ld_ab : lda, r.b ? r.ld_ab : ldb, ldc4, in_dtype)) return MI355_OK;

@@ -111,6 +111,8 @@ int launch_stream(const GemmArgs& g, int in_dtype, int out_dtype, int splits, vo
 int64_t quantize_e4m3_partials(int64_t n);
 int launch_quantize_e4m3(const void* x, int in_dtype, int64_t n, void* q, float* scale_amax, float* partial, int64_t partials,
                          hipStream_t stream);
+// Small products with rows of any alignment (gemm_tn_small.hip).
+int launch_small(const GemmArgs& g, int in_dtype, int out_dtype, hipStream_t stream);
 int launch_simple(const GemmArgs& g, int in_dtype, int out_dtype, hipStream_t stream);
 // Repacking for problems the tiled kernels cannot address (gemm_tn_simple.hip): rows of `row_bytes` bytes with stride
 // src_ld bytes -> 16-byte aligned rows with stride dst_ld bytes, the tail of every row filled with zeros.  One or two
