@@ -719,8 +719,11 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
     return mi355::launch_small(g, in_dtype, out_dtype, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
   }
   if (!large || !(r.a || r.b)) return MI355_OK;
-  if (!tile256_ok(M, r.Np, r.Kp, r.a ? r.ld_ab : lda, r.b ? r.ld_ab : ldb, ldc4, in_dtype)) return MI355_OK;
-  const bool copies_b = r.Kp != K || (ldb * es) % 16 != 0 || (uintptr_t)B % 16 != 0;   // not for N: rows past it read as zeros
+  // N alone is no reason to copy B (rows past N read as zeros), a row stride beyond the tiled kernels' 32-bit offsets is; what
+  // they are handed in the end has to pass their check.
+  const bool copies_b = r.b && (r.Kp != K || (uintptr_t)B % 16 != 0 || !tile256_ok(M, r.Np, r.Kp, r.ld_ab, ldb, r.Np, in_dtype));
+  const int64_t ld_a = r.a ? r.ld_ab : lda, ld_b = copies_b ? r.ld_ab : ldb;
+  if (!tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, ldc4, in_dtype)) return MI355_OK;
   const size_t bytes_b = copies_b ? r.bytes_b : 0, packed = r.bytes_a + bytes_b;
   if (r.bytes_a >= kMaxRepackBytes || bytes_b >= kMaxRepackBytes) return MI355_OK;
   // What the repacked (aligned) problem wants for its own splits.  The streaming kernel insists
@@ -742,8 +745,7 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   const mi355::RepackOperand pack_a = {(const uint8_t*)A, r.a ? M : 0, lda * es, wa, r.ld_ab * es};
   const mi355::RepackOperand pack_b = {(const uint8_t*)B, copies_b ? N : 0, ldb * es, wb, r.ld_ab * es};
   if (mi355::launch_repack_rows(pack_a, pack_b, K * es, (int)es, s) != 0) return MI355_ERR_LAUNCH;
-  return product(r.a ? wa : A, copies_b ? wb : B, r.Kp, r.a ? r.ld_ab : lda, copies_b ? r.ld_ab : ldb, rest_bytes ? rest : nullptr,
-                 rest_bytes);
+  return product(r.a ? wa : A, copies_b ? wb : B, r.Kp, ld_a, ld_b, rest_bytes ? rest : nullptr, rest_bytes);
 }
 
 int run_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

@@ -1,0 +1,94 @@
+"""What a call of the C ABI launches, looked at without a GPU: the built library's host code runs against a recorder in the
+place of the HIP runtime (launch_recorder.cpp), in a process of its own."""
+import json
+import os
+import subprocess
+import sys
+
+import pytest
+
+from tests import abi_ctypes as ac
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+A, B, C, WS = 1 << 44, 2 << 44, 3 << 44, 5 << 44      # addresses that nothing reads
+GEMM = ["M", "N", "K", "lda", "ldb", "ldc", "A", "B", "C", "c_ragged", "splits", "tail_tiles"]
+REPACK = ["rows", "src_ld", "src", "dst", "dst_ld", "blocks"]
+
+CHILD = """
+import ctypes, json, sys
+recorder = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+sys.path.insert(0, sys.argv[2])
+from tests import abi_ctypes as ac
+L = ac.load()
+recorder.recorded_name.restype = ctypes.c_char_p
+recorder.recorded_values.restype = ctypes.POINTER(ctypes.c_int64)
+out = []
+for c in json.load(sys.stdin):
+    recorder.forget()
+    args = [c["A"], c["B"], c["C"], c["M"], c["N"], c["K"], c["lda"], c["ldb"], c["ldc"], c["in_dt"], c["out_dt"], 1.0, c["variant"]]
+    need = L.mi355_gemm_workspace_bytes(c["M"], c["N"], c["K"], c["in_dt"], c["variant"])
+    room = need if c["room"] is None else c["room"]
+    st = L.mi355_gemm_tn_noalloc(*args, None) if c["noalloc"] else L.mi355_gemm_tn(*args, c["ws"] if room else None, room, None)
+    got = [(recorder.recorded_name(i).decode(), recorder.recorded_values(i)[:12]) for i in range(recorder.recorded())]
+    out.append((st, need, got))
+json.dump(out, sys.stdout)
+"""
+
+
+@pytest.fixture(scope="module")
+def launches(tmp_path_factory):
+    """launches(cases) -> [(status, workspace query, [(kernel, values)])]."""
+    so = str(tmp_path_factory.mktemp("recorder") / "recorder.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-isystem", "/opt/rocm/include",
+                    "-o", so, os.path.join(HERE, "launch_recorder.cpp")], check=True)
+
+    def ask(cases):
+        run = subprocess.run([sys.executable, "-c", CHILD, so, os.path.dirname(HERE)], input=json.dumps(cases), text=True,
+                             capture_output=True, check=True)
+        out = []
+        for st, need, got in json.loads(run.stdout):
+            shown = []
+            for name, v in got:
+                if "repack_rows" in name:
+                    v = [dict(zip(REPACK, v[:6])), dict(zip(REPACK, v[6:]))]
+                elif "gemm_tn_" in name:
+                    v = dict(zip(GEMM, v))
+                shown.append((name, v))
+            out.append((st, need, shown))
+        return out
+    return ask
+
+
+def case(M, N, K, in_dt=ac.BF16, lda=None, ldb=None, ldc=None, a=A, b=B, c=C, variant=ac.AUTO, room=None, noalloc=False, ws=WS):
+    """room: bytes of workspace, None for what the query asks."""
+    return dict(M=M, N=N, K=K, in_dt=in_dt, out_dt=ac.BF16 if in_dt == ac.E4M3 else in_dt, lda=lda or K, ldb=ldb or K, ldc=ldc or N,
+                A=a, B=b, C=c, variant=variant, room=room, noalloc=noalloc, ws=ws)
+
+
+def matrix_core(name):
+    return "gemm_tn_" in name and "gemm_tn_simple" not in name and "gemm_tn_small" not in name
+
+
+def panel_ok(v, es):
+    return 256 * v["lda"] * es < 1 << 31 and 256 * v["ldb"] * es < 1 << 31
+
+
+# 256 rows of B of 2 GiB and more, N not a multiple of 4: tile and streaming kernels, A aligned or not, K aligned or not.
+@pytest.mark.parametrize("in_dt", [ac.BF16, ac.F16, ac.E4M3])
+def test_no_kernel_gets_rows_of_b_it_cannot_address(launches, in_dt):
+    es = 1 if in_dt == ac.E4M3 else 2
+    limit = (1 << 31) // 256 // es
+    cases = [case(M, N, K, in_dt, ldb=ldb, a=a, b=b, room=None if a == A else 1 << 34)    # the query counts on aligned rows of A
+             for M, N, K in [(4096, 5, 4096), (1024, 257, 1024), (300, 130, 4096), (100, 1001, 2048), (17, 4099, 4096), (2048, 8191, 4100)]
+             for ldb in (limit - 16, limit, limit + 3, 1 << 26, 1 << 29)
+             for a, b in ((A, B), (A + es, B), (A, B + es))]
+    for c, (st, need, got) in zip(cases, launches(cases)):
+        assert st == ac.OK and got, c
+        for name, v in got:
+            if matrix_core(name):
+                assert panel_ok(v, es), (c, name, v)
+        # with that much workspace every one of these runs on the matrix cores
+        assert any(matrix_core(name) for name, _ in got), (c, got)
+        packed = [v for name, v in got if "repack_rows" in name]
+        if c["ldb"] >= limit:
+            assert packed and packed[0][1]["rows"] == c["N"] and packed[0][1]["src_ld"] == c["ldb"] * es

@@ -103,3 +103,19 @@ def test_repacked_operands(abi, dt, M, N, K):
         C, kept = run(abi, A, B, offset, N + offset, room=room)
         assert kept
         close(C, A, B)
+
+
+def test_rows_of_b_farther_apart_than_the_kernels_reach(abi):
+    """N % 4 != 0 and 256 rows of B beyond 2 GiB: B is copied to rows that the tiled kernels can address."""
+    M, N, K, ldb = 4096, 5, 4096, 1 << 29
+    A, B = operand(M, K, torch.bfloat16, 21), operand(N, K, torch.bfloat16, 22)
+    far = torch.empty((N - 1) * ldb + K, dtype=torch.bfloat16, device="cuda")
+    for n in range(N):
+        far[n * ldb:n * ldb + K] = B[n].cuda()
+    Ad, C = A.cuda(), torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
+    need = abi.mi355_gemm_workspace_bytes(M, N, K, ac.BF16, ac.AUTO)
+    ws = torch.empty(need, dtype=torch.uint8, device="cuda")
+    st = abi.mi355_gemm_tn(Ad.data_ptr(), far.data_ptr(), C.data_ptr(), M, N, K, K, ldb, N, ac.BF16, ac.BF16, 1.0, ac.AUTO,
+                           ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
+    assert st == ac.OK
+    close(C.cpu().double(), A, B)
