@@ -134,7 +134,6 @@ int resolve(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t l
 // passes over the operands.  The generic kernel takes about a millisecond per GFLOP; the repacked problem runs at the
 // tiled kernels' rate.  The plan also counts a padded copy of C where N or ldc is not a multiple of 4: the size of the
 // workspace includes it, though the kernels that store such a C directly leave that part unused.
-constexpr size_t kMaxRepackBytes = (size_t)1 << 34;   // the copy kernel counts 16-byte chunks in 32 bits
 struct Repack {
   bool a, b, c;
   int64_t Kp, Np;                 // padded K (elements) and N
@@ -725,7 +724,6 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   const int64_t ld_a = r.a ? r.ld_ab : lda, ld_b = copies_b ? r.ld_ab : ldb;
   if (!tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, ldc4, in_dtype)) return MI355_OK;
   const size_t bytes_b = copies_b ? r.bytes_b : 0, packed = r.bytes_a + bytes_b;
-  if (r.bytes_a >= kMaxRepackBytes || bytes_b >= kMaxRepackBytes) return MI355_OK;
   // What the repacked (aligned) problem wants for its own splits.  The streaming kernel insists
   // on the workspace of its K split, so a lenient call repacks only when the rest covers it.
   const size_t inner = mi355_gemm_workspace_bytes(M, r.Np, r.Kp, in_dtype, MI355_VARIANT_AUTO);

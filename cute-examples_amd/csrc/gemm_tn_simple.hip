@@ -56,7 +56,7 @@ __global__ __launch_bounds__(256) void repack_rows(RepackOperand first, RepackOp
   const RepackOperand& op = is_second ? second : first;
   const uint32_t per_row = (uint32_t)(op.dst_ld / 16);
   const uint32_t begin = (is_second ? blockIdx.x - first_blocks : blockIdx.x) * (256 * kChunks) + threadIdx.x;
-  const uint32_t total = (uint32_t)op.rows * per_row;      // below 2^31 (host check)
+  const uint32_t total = (uint32_t)op.rows * per_row;      // below 2^31 (launch_repack_rows)
   u32x4 v[kChunks];
   int64_t to[kChunks];
 #pragma unroll
@@ -82,21 +82,28 @@ int launch(const GemmArgs& g, hipStream_t stream) {
 }  // namespace
 
 int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, int64_t row_bytes, int elem_bytes, hipStream_t stream) {
-  uint32_t blocks[2];
-  const RepackOperand* ops[2] = {&first, &second};
-  for (int i = 0; i < 2; ++i) {
-    const RepackOperand& o = *ops[i];
-    if (o.rows == 0) {
-      blocks[i] = 0;
-      continue;
-    }
-    if (o.dst_ld % 16 != 0 || o.dst_ld >= ((int64_t)1 << 31) || o.rows >= ((int64_t)1 << 31) / (o.dst_ld / 16)) return -1;
-    blocks[i] = (uint32_t)((o.rows * (o.dst_ld / 16) + 256 * kChunks - 1) / (256 * kChunks));
-  }
-  if (blocks[0] + blocks[1] == 0) return 0;
   const auto kernel = elem_bytes == 2 ? repack_rows<uint16_t> : repack_rows<uint8_t>;
-  hipLaunchKernelGGL(kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, stream, first, second, (uint32_t)row_bytes, blocks[0]);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
+  constexpr int64_t kMaxChunks = ((int64_t)1 << 31) - 1;   // of a launch and operand; a larger copy goes in runs of rows
+  RepackOperand rest[2] = {first, second};
+  while (rest[0].rows > 0 || rest[1].rows > 0) {
+    RepackOperand part[2];
+    uint32_t blocks[2];
+    for (int i = 0; i < 2; ++i) {
+      part[i] = rest[i];
+      blocks[i] = 0;
+      if (rest[i].rows == 0) continue;
+      const int64_t per_row = rest[i].dst_ld / 16;
+      if (rest[i].dst_ld % 16 != 0 || per_row > kMaxChunks) return -1;
+      if (part[i].rows > kMaxChunks / per_row) part[i].rows = kMaxChunks / per_row;
+      blocks[i] = (uint32_t)((part[i].rows * per_row + 256 * kChunks - 1) / (256 * kChunks));
+      rest[i].rows -= part[i].rows;
+      rest[i].src += part[i].rows * rest[i].src_ld;
+      rest[i].dst += part[i].rows * rest[i].dst_ld;
+    }
+    hipLaunchKernelGGL(kernel, dim3(blocks[0] + blocks[1]), dim3(256), 0, stream, part[0], part[1], (uint32_t)row_bytes, blocks[0]);
+    if (hipGetLastError() != hipSuccess) return -1;
+  }
+  return 0;
 }
 
 int launch_simple(const GemmArgs& g, int in_dtype, int out_dtype, hipStream_t stream) {

@@ -92,3 +92,27 @@ def test_no_kernel_gets_rows_of_b_it_cannot_address(launches, in_dt):
         packed = [v for name, v in got if "repack_rows" in name]
         if c["ldb"] >= limit:
             assert packed and packed[0][1]["rows"] == c["N"] and packed[0][1]["src_ld"] == c["ldb"] * es
+
+
+# Copies of 17 GB and of 36 and 40 GB (two launches: one counts below 2^31 chunks of 16 bytes), of B and of A; 34 GB of fp8.
+@pytest.mark.parametrize("M,N,K,in_dt,copies", [(8192, 262144, 33001, ac.BF16, 1), (64, 600000, 33001, ac.BF16, 2), (550000, 40, 32801, ac.F16, 2),
+                                                (300, 530001, 65001, ac.E4M3, 2)])
+def test_copies_of_any_size_are_made(launches, M, N, K, in_dt, copies):
+    es = 1 if in_dt == ac.E4M3 else 2
+    cases = [case(M, N, K, in_dt), case(M, N, K, in_dt, noalloc=True)]
+    (st, need, got), (st_noalloc, _, got_noalloc) = launches(cases)
+    assert st == ac.OK and need > 17e9
+    packed = [v for name, v in got if "repack_rows" in name]
+    assert len(packed) == copies
+    for i, (src, rows) in enumerate(((A, M), (B, N))):
+        parts = [p[i] for p in packed if p[i]["rows"]]
+        assert sum(p["rows"] for p in parts) == rows
+        at, to = src, parts[0]["dst"]
+        for p in parts:      # one after the other, without a gap
+            chunks = p["rows"] * (p["dst_ld"] // 16)
+            assert (p["src"], p["dst"], p["src_ld"]) == (at, to, K * es)
+            assert chunks < 1 << 31 and p["blocks"] == -(-chunks // 1024)
+            at, to = at + p["rows"] * p["src_ld"], to + p["rows"] * p["dst_ld"]
+        assert WS <= parts[0]["dst"] and to <= WS + need
+    assert any(matrix_core(name) for name, _ in got) and not any("simple" in name for name, _ in got)
+    assert st_noalloc == ac.ERR_SCRATCH and not got_noalloc
