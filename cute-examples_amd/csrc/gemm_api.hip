@@ -132,8 +132,8 @@ int resolve(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t l
 // stride not a multiple of 16, misaligned A or B) into an aligned one in the caller's workspace -- A and B copied to
 // zero-padded 16-byte-aligned rows -- when the workspace is large enough and the problem is big enough to pay for the
 // passes over the operands.  The generic kernel takes about a millisecond per GFLOP; the repacked problem runs at the
-// tiled kernels' rate.  The plan also counts a padded copy of C where N or ldc is not a multiple of 4: the size of the
-// workspace includes it, though the kernels that store such a C directly leave that part unused.
+// tiled kernels' rate.  The plan also counts a copy of B where N is not a multiple of 4 and a padded copy of C where N or ldc
+// is not: so does the size of the workspace, though run_unaligned makes those only where their rows are out of reach.
 struct Repack {
   bool a, b, c;
   int64_t Kp, Np;                 // padded K (elements) and N
@@ -679,9 +679,10 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
 }
 
 // A problem that MI355_VARIANT_AUTO reports as SIMPLE, on the matrix cores all the same where that can be done: directly when
-// only C is in the way (N or ldc not a multiple of 4, C not 8-byte aligned), with A and B repacked when they are and the
-// workspace holds the copies.  *handled says whether it was done.  Measured, both sides: bf16 1000 x 50257 x 768 with a
-// padded copy of B and of C 174 us, direct 127 us; fp16 515 x 2050 x 4100 with padded C 40.0 us, without 29.5 us.
+// only C is in the way (N or ldc not a multiple of 4, C not 8-byte aligned), with A and B repacked when they are (and C padded
+// when its rows are out of reach) and the workspace holds the copies.  *handled says whether it was done.  Measured, both
+// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 127 us; fp16 515 x 2050 x 4100 with padded C
+// 40.0 us, without 29.5 us.
 int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                   int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, void* workspace,
                   size_t workspace_bytes, hipStream_t s, WorkspaceMode mode, bool* handled) {
@@ -693,17 +694,19 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   const bool large = repack_plan(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, &r);
   if (large && (!workspace || (uintptr_t)workspace % 256 != 0)) return MI355_OK;   // the contract: the generic kernel then
   const bool ab_aligned = (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
-  // The product on operands that the tiled kernels can address, with what is left of the workspace.
-  const auto product = [&](const void* a, const void* b, int64_t k, int64_t ld_a, int64_t ld_b, void* ws, size_t ws_bytes) {
-    const bool c_ragged = N % 4 != 0 || ldc % 4 != 0 || (uintptr_t)C % 8 != 0;
+  // The product on operands that the tiled kernels can address, with what is left of the workspace: into the caller's C, or
+  // (padded) into a copy of it whose rows are aligned and have room for Np columns.
+  const auto product = [&](const void* a, const void* b, int64_t k, int64_t ld_a, int64_t ld_b, void* c, int64_t ld_c, bool padded,
+                           void* ws, size_t ws_bytes) {
+    const bool c_ragged = !padded && (N % 4 != 0 || ldc % 4 != 0 || (uintptr_t)C % 8 != 0);
     int v = auto_variant(M, Np, k, in_dtype);
     if (c_ragged && v == MI355_VARIANT_ALTERNATE) v = MI355_VARIANT_BASIC;   // the two kernels that take such a C
-    return run_variant(a, b, C, M, N, k, ld_a, ld_b, ldc, in_dtype, out_dtype, scale, scale_a, scale_b, v, true, c_ragged, ws,
+    return run_variant(a, b, c, M, N, k, ld_a, ld_b, ld_c, in_dtype, out_dtype, scale, scale_a, scale_b, v, true, c_ragged, ws,
                        ws_bytes, s, mode);
   };
   if (ab_aligned && tile256_ok(M, Np, K, lda, ldb, ldc4, in_dtype)) {
     *handled = true;
-    return product(A, B, K, lda, ldb, workspace, workspace_bytes);
+    return product(A, B, K, lda, ldb, C, ldc, false, workspace, workspace_bytes);
   }
   if (!large && K >= kSmallMinK && (uintptr_t)A % es == 0 && (uintptr_t)B % es == 0 && 2.0 * (double)M * (double)N * (double)K < kRepackMinFlops) {
     *handled = true;
@@ -717,13 +720,14 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
     g.scale_b = scale_b;
     return mi355::launch_small(g, in_dtype, out_dtype, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
   }
-  if (!large || !(r.a || r.b)) return MI355_OK;
+  if (!large) return MI355_OK;
   // N alone is no reason to copy B (rows past N read as zeros), a row stride beyond the tiled kernels' 32-bit offsets is; what
-  // they are handed in the end has to pass their check.
+  // they are handed in the end has to pass their check.  So for C, whose padded copy is copied out afterwards.
   const bool copies_b = r.b && (r.Kp != K || (uintptr_t)B % 16 != 0 || !tile256_ok(M, r.Np, r.Kp, r.ld_ab, ldb, r.Np, in_dtype));
   const int64_t ld_a = r.a ? r.ld_ab : lda, ld_b = copies_b ? r.ld_ab : ldb;
-  if (!tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, ldc4, in_dtype)) return MI355_OK;
-  const size_t bytes_b = copies_b ? r.bytes_b : 0, packed = r.bytes_a + bytes_b;
+  const bool pads_c = r.c && !tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, ldc4, in_dtype);
+  if (!tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, pads_c ? r.ld_c : ldc4, in_dtype)) return MI355_OK;
+  const size_t bytes_b = copies_b ? r.bytes_b : 0, bytes_c = pads_c ? r.bytes_c : 0, packed = r.bytes_a + bytes_b + bytes_c;
   // What the repacked (aligned) problem wants for its own splits.  The streaming kernel insists
   // on the workspace of its K split, so a lenient call repacks only when the rest covers it.
   const size_t inner = mi355_gemm_workspace_bytes(M, r.Np, r.Kp, in_dtype, MI355_VARIANT_AUTO);
@@ -738,12 +742,16 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   if (mode == kStrictDry) return MI355_OK;
   uint8_t* wa = (uint8_t*)workspace;
   uint8_t* wb = wa + r.bytes_a;
-  uint8_t* rest = wb + bytes_b;
+  uint8_t* wc = wb + bytes_b;
+  uint8_t* rest = wc + bytes_c;
   const size_t rest_bytes = workspace_bytes - packed;
   const mi355::RepackOperand pack_a = {(const uint8_t*)A, r.a ? M : 0, lda * es, wa, r.ld_ab * es};
   const mi355::RepackOperand pack_b = {(const uint8_t*)B, copies_b ? N : 0, ldb * es, wb, r.ld_ab * es};
   if (mi355::launch_repack_rows(pack_a, pack_b, K * es, (int)es, s) != 0) return MI355_ERR_LAUNCH;
-  return product(r.a ? wa : A, copies_b ? wb : B, r.Kp, ld_a, ld_b, rest_bytes ? rest : nullptr, rest_bytes);
+  const int st = product(r.a ? wa : A, copies_b ? wb : B, r.Kp, ld_a, ld_b, pads_c ? (void*)wc : C, pads_c ? r.ld_c : ldc, pads_c,
+                         rest_bytes ? rest : nullptr, rest_bytes);
+  if (st != MI355_OK || !pads_c) return st;
+  return mi355::launch_copy_out(wc, M, N, r.ld_c, C, ldc, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
 }
 
 int run_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

@@ -33,7 +33,8 @@ struct GemmArgs {
   int32_t c_streams;
   // Non-zero when C is to be stored through store_ragged_quad / store_ragged_octet: its rows are aligned by nothing but its
   // element type, or by less than 64 bytes and this is the faster way (rows_want_plain_stores in gemm_api.hip).  Single-group
-  // tile kernel and streaming kernel only, and not with block scales.
+  // tile kernel and streaming kernel only, and not with block scales.  Zero otherwise: rows of C then have room for
+  // partial_columns(N) columns and are written four columns at a time.
   int32_t c_ragged;
   // Block scales (MX) of A and of B in the shuffled layout, or null.
   const uint8_t* mx_a;
@@ -42,7 +43,7 @@ struct GemmArgs {
 
 // Columns of a row of fp32 partial sums: planes are [M][N rounded up to 4], so that four sums are one aligned load.  (Rows
 // of B past N read as zeros, so the added columns hold zeros.)
-inline __host__ __device__ int64_t partial_columns(int64_t N) { return (N + 3) / 4 * 4; }
+inline __host__ __device__ int64_t partial_columns(int64_t N) { return (N + 3) & ~(int64_t)3; }
 
 // Effective output scale; wave-uniform, read once per workgroup.
 #if defined(__HIPCC__)
@@ -124,5 +125,8 @@ struct RepackOperand {
   int64_t dst_ld;
 };
 int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, int64_t row_bytes, int elem_bytes, hipStream_t stream);
+// A (rows x cols) block of 16-bit elements with row stride src_ld elements (a multiple of 4) -> row stride dst_ld elements at any
+// 2-byte alignment.
+int launch_copy_out(const void* src, int64_t rows, int64_t cols, int64_t src_ld, void* dst, int64_t dst_ld, hipStream_t stream);
 
 }  // namespace mi355

@@ -604,7 +604,7 @@ __global__ __launch_bounds__(256) void tail_reduce(GemmArgs g) {
   const u32x2 out = Pack4<OutT>::run(sum[0] * scale, sum[1] * scale, sum[2] * scale, sum[3] * scale);
   uint16_t* dst = (uint16_t*)g.C + m * g.ldc + n;
   if (g.c_ragged) store_ragged_quad(dst, out, g.N - n);
-  else *(u32x2*)dst = out;   // N % 4 == 0: a quad is in or out as a whole
+  else *(u32x2*)dst = out;   // rows of an aligned C have room for whole quads
 }
 
 template <class T, class OutT, bool kRaggedC, int kTileT, int kTileNT = kTileT, int kAhead = 2, int kWavesN = 2, bool kRotateT = (kAhead > 2)>

@@ -1,8 +1,8 @@
 // One thread per output element: C[m][n] = rne(scale * sum_k A[m][k] * B[n][k]) with a serial
 // fp32 fused-multiply-add chain over k.  Handles every shape, stride and dtype the ABI accepts;
 // it is the library's on-device cross-check for the MFMA kernels and the path for shapes they
-// reject.  Also here: the copy kernel with which the library repacks the operands of such a problem
-// into aligned ones when the caller lends it the memory (gemm_api.hip).  Counterpart in the reference:
+// reject.  Also here: the copy kernels with which the library repacks the operands of such a problem
+// into aligned ones, and its output out of an aligned one, when the caller lends it the memory (gemm_api.hip).  Counterpart in the reference:
 // none (its only kernel rejects such shapes, kernels/gemm_kernels/sm90a/gemm_test.cu:33-41).
 #include "cdna4_primitives.h"
 #include "gemm_launch.h"
@@ -71,6 +71,16 @@ __global__ __launch_bounds__(256) void repack_rows(RepackOperand first, RepackOp
     if (to[i] >= 0) *(u32x4*)(op.dst + to[i]) = v[i];
 }
 
+// One thread per four columns: the source rows are 8-byte aligned, the destination has only element alignment.
+__global__ __launch_bounds__(256) void copy_out(const uint16_t* __restrict__ src, int64_t rows, int64_t cols, int64_t src_ld,
+                                                uint16_t* __restrict__ dst, int64_t dst_ld) {
+  const int64_t quads = (cols + 3) / 4;
+  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (id >= rows * quads) return;
+  const int64_t row = id / quads, col = (id % quads) * 4;
+  store_ragged_quad(dst + row * dst_ld + col, *(const u32x2*)(src + row * src_ld + col), cols - col);
+}
+
 template <class T, class OutT>
 int launch(const GemmArgs& g, hipStream_t stream) {
   const int64_t blocks = ((g.N + 15) / 16) * ((g.M + 15) / 16);
@@ -104,6 +114,15 @@ int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, 
     if (hipGetLastError() != hipSuccess) return -1;
   }
   return 0;
+}
+
+int launch_copy_out(const void* src, int64_t rows, int64_t cols, int64_t src_ld, void* dst, int64_t dst_ld, hipStream_t stream) {
+  const int64_t n = rows * ((cols + 3) / 4), blocks = (n + 255) / 256;
+  if (n == 0) return 0;
+  if (blocks >= ((int64_t)1 << 31) || src_ld % 4 != 0 || (uintptr_t)src % 8 != 0) return -1;
+  hipLaunchKernelGGL(copy_out, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)src, rows, cols, src_ld, (uint16_t*)dst,
+                     dst_ld);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int launch_simple(const GemmArgs& g, int in_dtype, int out_dtype, hipStream_t stream) {

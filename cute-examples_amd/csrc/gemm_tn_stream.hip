@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_stream(GemmArgs g, float* pa
 #pragma unroll
     for (int j = 0; j < kNB; ++j) {
       const int64_t n = n0 + (wn * kNB + j) * 16 + grp * 4;
-      if (n >= g.N) continue;      // N % 4 == 0 unless C is ragged
+      if (n >= g.N) continue;      // rows of an aligned C have room for whole quads
       // A wave has at most sixteen of these stores: each one's data registers are simply held over
       // the wait states a wide store wants before they may be rewritten (see hold_previous).
       if (partial) {

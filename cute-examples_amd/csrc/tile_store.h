@@ -50,7 +50,8 @@ __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][k
   // side) and the 32-wide blocks do not (32 bytes: measured 3 % slower with sc1, 25 % with nt + sc1).
   const uint32_t rblk = lane & (kBlk - 1), grp = lane / kBlk;
   const int64_t rows = g.M - m0 < tile_rows ? g.M - m0 : tile_rows;
-  const uint32_t cols = (uint32_t)(g.N - n0 < tile_cols ? g.N - n0 : tile_cols);
+  const int64_t n_end = kRaggedC ? g.N : partial_columns(g.N);   // rows of an aligned C have room for whole quads
+  const uint32_t cols = (uint32_t)(n_end - n0 < tile_cols ? n_end - n0 : tile_cols);
   const uint32_t ldc_b = (uint32_t)g.ldc * 2;
   const __amdgpu_buffer_rsrc_t rc =
       make_raw_buffer((const uint16_t*)g.C + m0 * g.ldc + n0, (uint32_t)(((rows - 1) * g.ldc + cols) * 2));
@@ -169,7 +170,7 @@ __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][k
     else if (g.c_streams) whole_rows(std::integral_constant<int, 18>{});
     else whole_rows(std::integral_constant<int, 16>{});
   } else {
-    // N is a multiple of 4 (host check), so each half of the 8 columns is in or out as a whole.
+    // n_end is a multiple of 4, so each half of the 8 columns is in or out as a whole.
     u32x4 previous = {0u, 0u, 0u, 0u}, before = {0u, 0u, 0u, 0u};
     convert([&](auto ic, auto colc, u32x2 x, u32x2 y) __attribute__((always_inline)) {
       constexpr int i = decltype(ic)::value, col = decltype(colc)::value;

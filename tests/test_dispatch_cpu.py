@@ -116,3 +116,24 @@ def test_copies_of_any_size_are_made(launches, M, N, K, in_dt, copies):
         assert WS <= parts[0]["dst"] and to <= WS + need
     assert any(matrix_core(name) for name, _ in got) and not any("simple" in name for name, _ in got)
     assert st_noalloc == ac.ERR_SCRATCH and not got_noalloc
+
+
+# Rows of C of 2^21 elements and more: the tile kernels' 32-bit offsets do not reach them, a padded copy of C does.
+@pytest.mark.parametrize("in_dt", [ac.BF16, ac.E4M3])
+@pytest.mark.parametrize("M,N,K", [(300, 1003, 1024), (100, 4099, 4096), (4096, 5, 4096), (2048, 8190, 129), (8192, 16385, 128), (300, 1000, 1024)])
+def test_rows_of_c_out_of_reach(launches, in_dt, M, N, K):
+    limit = 1 << 21
+    strides = (limit - 3, limit - 1, limit + 1, limit + 6, 1 << 24)     # none aligned where N is
+    cases = [case(M, N, K, in_dt, ldc=ldc + (ldc % 4 == 0 and N % 4 == 0), room=1 << 31) for ldc in strides]
+    for c, (st, need, got) in zip(cases, launches(cases)):
+        assert st == ac.OK
+        products = [v for name, v in got if matrix_core(name)]
+        assert products and not any("simple" in name for name, _ in got), c
+        assert all(256 * v["ldc"] * 4 < 1 << 31 for v in products), c
+        out_of_reach = 256 * (-(-c["ldc"] // 4) * 4) * 4 >= 1 << 31
+        assert ("copy_out" in got[-1][0]) == out_of_reach, (c, got)
+        for v in products:
+            if out_of_reach:      # whole quads of columns fit in a padded row
+                assert WS <= v["C"] < WS + need + (1 << 31) and v["ldc"] >= -(-N // 4) * 4 and v["ldc"] % 64 == 0 and not v["c_ragged"]
+            else:
+                assert v["ldc"] == c["ldc"]

@@ -119,3 +119,13 @@ def test_rows_of_b_farther_apart_than_the_kernels_reach(abi):
                            ws.data_ptr(), need, torch.cuda.current_stream().cuda_stream)
     assert st == ac.OK
     close(C.cpu().double(), A, B)
+
+
+@pytest.mark.parametrize("M,N,K,dt", [(300, 1003, 1024, torch.bfloat16), (65, 514, 2055, torch.float16), (300, 130, 4096, torch.float8_e4m3fn),
+                                      (40, 2049, 2048, torch.bfloat16), (260, 1000, 264, torch.bfloat16)])
+def test_rows_of_c_farther_apart_than_the_kernels_reach(abi, M, N, K, dt):
+    """Computed into a padded copy of C and copied out, on the streaming kernel, the tile kernel and its K splits."""
+    A, B = operand(M, K, dt, 23), operand(N, K, dt, 24)
+    C, kept = run(abi, A, B, 1, (1 << 21) + 3)
+    assert kept
+    close(C, A, B)
