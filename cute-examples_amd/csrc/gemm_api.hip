@@ -147,9 +147,10 @@ struct Repack {
 size_t round_up(size_t x, size_t to) { return (x + to - 1) / to * to; }
 
 constexpr double kRepackMinFlops = 134217728.0;   // below, repacking is not worth its launches
-// From here on such a small problem runs on gemm_tn_small instead of the generic kernel.  Both timed at M = 1...2048 and 1 to 67
-// million products: K = 65 small 0.5-1.0 of the generic kernel's speed, K = 129 1.0-1.7, 257 2.0-3.5, 513 3.9-7.7, 1025 7-16
-// times (bf16 16 x 4025 x 1025 128 -> 13 us), 14335 51-157 times (bf16 16 x 287 x 14335 1808 -> 33 us).
+// From here on a small problem with unaligned operands, or an e4m3 one with any unaligned rows, runs on gemm_tn_small instead of
+// the generic kernel.  Both timed at M = 1...2048 and 1 to 67 million products: K = 65 small 0.5-1.0 of the generic kernel's
+// speed, K = 129 1.0-1.7, 257 2.0-3.5, 513 3.9-7.7, 1025 7-16 times (bf16 16 x 4025 x 1025 128 -> 13 us), 14335 51-157 times
+// (bf16 16 x 287 x 14335 1808 -> 33 us).
 constexpr int64_t kSmallMinK = 128;
 
 bool repack_plan(const void* A, const void* B, const void* C, int64_t M, int64_t N, int64_t K, int64_t lda,
@@ -326,7 +327,7 @@ size_t mi355_gemm_workspace_bytes(int64_t M, int64_t N, int64_t K, int in_dtype,
     Repack r;
     if (!repack_plan(nullptr, nullptr, nullptr, M, N, K, K, K, N, in_dtype, &r)) {
       const int64_t Np = mi355::partial_columns(N);
-      return Np != N && tile256_ok(M, Np, K, K, K, Np, in_dtype) ? mi355_gemm_workspace_bytes(M, Np, K, in_dtype, variant) : 0;
+      return Np != N && in_dtype != MI355_E4M3 && tile256_ok(M, Np, K, K, K, Np, in_dtype) ? mi355_gemm_workspace_bytes(M, Np, K, in_dtype, variant) : 0;
     }
     return r.bytes_a + r.bytes_b + r.bytes_c + mi355_gemm_workspace_bytes(M, r.Np, r.Kp, in_dtype, MI355_VARIANT_AUTO);
   }
@@ -704,7 +705,12 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
     return run_variant(a, b, c, M, N, k, ld_a, ld_b, ld_c, in_dtype, out_dtype, scale, scale_a, scale_b, v, true, c_ragged, ws,
                        ws_bytes, s, mode);
   };
-  if (ab_aligned && tile256_ok(M, Np, K, lda, ldb, ldc4, in_dtype)) {
+  // Small e4m3 products stay on fp32 sums (gemm_tn_small, the generic kernel): the matrix cores' fp8 sums are coarser.  Sums that
+  // cancel, relative error behind the rounding to fp16: 1.8e-4 with either of the two at every K, 1.8e-4 / 2.4e-4 / 4.0e-4 / 6.9e-4
+  // at K = 128 / 1024 / 4096 / 14336 on the matrix cores; bf16 and fp16 products are off by the same on all three.  16-bit
+  // products are faster here from the smallest on (M = 1...2048, 1 to 67 million products, us, generic kernel against this: K = 16
+  // 4.1...122 / 4.0...8.1, K = 128 13...120 / 4.2...6.0, K = 1024 106...146 / 7...13).
+  if (ab_aligned && (large || in_dtype != MI355_E4M3) && tile256_ok(M, Np, K, lda, ldb, ldc4, in_dtype)) {
     *handled = true;
     return product(A, B, K, lda, ldb, C, ldc, false, workspace, workspace_bytes);
   }

@@ -137,3 +137,15 @@ def test_rows_of_c_out_of_reach(launches, in_dt, M, N, K):
                 assert WS <= v["C"] < WS + need + (1 << 31) and v["ldc"] >= -(-N // 4) * 4 and v["ldc"] % 64 == 0 and not v["c_ragged"]
             else:
                 assert v["ldc"] == c["ldc"]
+
+
+# Under 2^27 operations, everything aligned but the rows of C.
+@pytest.mark.parametrize("M,N,K,ldc", [(1, 129, 128, 129), (16, 1001, 4096, 1001), (64, 71, 14336, 71), (257, 501, 512, 501), (100, 128, 1024, 130),
+                                       (3, 30001, 64, 30001), (1, 4, 16, 5)])
+def test_small_fp8_products_keep_their_fp32_sums(launches, M, N, K, ldc):
+    cases = [case(M, N, K, ac.E4M3, ldc=ldc, room=room, noalloc=noalloc) for room in (0, None, 1 << 26) for noalloc in (False, True)]
+    for st, need, got in launches(cases):
+        assert st == ac.OK and (need == 0 or N % 4 == 0)
+        assert [("gemm_tn_small" if K >= 128 else "gemm_tn_simple") in name for name, _ in got] == [True]
+    for st, need, got in launches([case(M, N, K, ac.BF16, ldc=ldc)]):
+        assert st == ac.OK and all(not matrix_core(name) or v["c_ragged"] for name, v in got) and matrix_core(got[0][0])

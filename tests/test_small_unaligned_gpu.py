@@ -42,3 +42,21 @@ def test_against_float64(dt, ulp, M, N, K):
         B[0, K - 1] = 0.0
         st = ac.gemm_tn(abi, A.cuda(), B.cuda(), C, 1.0, ac.AUTO)
         assert st == ac.OK and bool(torch.isnan(C[0, 0]))
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 33, 128), (16, 33, 1024), (5, 129, 4096), (17, 66, 14336)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16, torch.float8_e4m3fn])
+def test_sums_that_cancel_keep_32_bits(dt, M, N, K):
+    """Only the rows of C are unaligned.  B's second half is the first one negated but for a few elements, so the sums are far
+    smaller than what is added up.  Rounding to fp16 is off by at most 2^-11 of a value: 2^-11 / sqrt(3) in the norm if errors
+    spread evenly up to that; fp32 sums add a few per cent of it."""
+    abi = ac.load()
+    g = torch.Generator().manual_seed(K)
+    a, b = torch.randn(M, K // 2, generator=g).to(dt).float(), torch.randn(N, K // 2, generator=g).to(dt).float()
+    A, B = torch.cat([a, a], 1), torch.cat([b, -b.scatter(1, torch.randint(0, K // 2, (N, 4), generator=g), 0.0)], 1)
+    order = torch.randperm(K, generator=g)
+    A, B = A[:, order].to(dt).contiguous(), B[:, order].to(dt).contiguous()
+    want = A.double() @ B.double().T
+    C = torch.zeros((M, N), dtype=torch.float16, device="cuda")
+    assert ac.gemm_tn(abi, A.cuda(), B.cuda(), C) == ac.OK
+    assert float((C.cpu().double() - want).norm() / want.norm()) <= 2.0 ** -11 / 3 ** 0.5
