@@ -584,7 +584,7 @@ __global__ __launch_bounds__(threads_of(kWavesN), (kTileT == 256 || kAhead > 2) 
 
 // C tiles of a tail split: rne(scale * (partial[0] + ... + partial[S-1])) in that order, for the
 // last g.tail_tiles tiles in tile-map order; one thread per 4 consecutive columns.
-template <class OutT, int kTileT, int kTileNT>
+template <class OutT, bool kRaggedC, int kTileT, int kTileNT>
 __global__ __launch_bounds__(256) void tail_reduce(GemmArgs g) {
   constexpr uint32_t kQuadsPerTile = kTileT * kTileNT / 4;
   const uint32_t q = blockIdx.x * 256u + threadIdx.x;
@@ -603,7 +603,7 @@ __global__ __launch_bounds__(256) void tail_reduce(GemmArgs g) {
   const float scale = output_scale(g);
   const u32x2 out = Pack4<OutT>::run(sum[0] * scale, sum[1] * scale, sum[2] * scale, sum[3] * scale);
   uint16_t* dst = (uint16_t*)g.C + m * g.ldc + n;
-  if (g.c_ragged) store_ragged_quad(dst, out, g.N - n);
+  if constexpr (kRaggedC) store_ragged_quad(dst, out, g.N - n);
   else *(u32x2*)dst = out;   // rows of an aligned C have room for whole quads
 }
 
@@ -625,7 +625,7 @@ int launch_tile(const GemmArgs& g, hipStream_t stream) {
     return launch_splitk_reduce(g.partial, g, std::is_same<OutT, BF16>::value ? 0 : 1, stream);
   if (g.tail_tiles) {
     const int64_t quads = (int64_t)g.tail_tiles * (kTileT * kTileNT / 4);
-    hipLaunchKernelGGL((tail_reduce<OutT, kTileT, kTileNT>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, g);
+    hipLaunchKernelGGL((tail_reduce<OutT, kRaggedC, kTileT, kTileNT>), dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, stream, g);
     if (hipGetLastError() != hipSuccess) return -1;
   }
   return 0;

@@ -149,3 +149,17 @@ def test_small_fp8_products_keep_their_fp32_sums(launches, M, N, K, ldc):
         assert [("gemm_tn_small" if K >= 128 else "gemm_tn_simple") in name for name, _ in got] == [True]
     for st, need, got in launches([case(M, N, K, ac.BF16, ldc=ldc)]):
         assert st == ac.OK and all(not matrix_core(name) or v["c_ragged"] for name, v in got) and matrix_core(got[0][0])
+
+
+@pytest.mark.parametrize("M,N,K,split", [(16, 14336, 4096, False), (16, 14333, 4096, False), (17, 4100, 4096, True), (17, 4099, 4096, True),
+                                         (64, 16896, 2048, False), (64, 16897, 2048, False)])
+def test_streaming_kernel_has_a_form_for_each_kind_of_rows(launches, M, N, K, split):
+    """The form for rows of any alignment is launched for those only, and nothing is decided about C inside a kernel."""
+    (st, _, got), = launches([case(M, N, K)])
+    assert st == ac.OK and len(got) == 1 + split and "gemm_tn_stream" in got[0][0]
+    ragged = N % 4 != 0
+    writes_c = got[-1][0]      # the reduction of a K split, else the product itself
+    assert ("splitk_reduce" in writes_c) == split
+    assert ("Lb1E" in writes_c) == ragged
+    if split:
+        assert "Lb1E" not in got[0][0]
