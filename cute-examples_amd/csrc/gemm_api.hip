@@ -571,21 +571,21 @@ int mi355_gemm_tn_noalloc(const void* A, const void* B, void* C, int64_t M, int6
 
 namespace {
 
+// Rows of C as the kernels are told of them.
+//   kRowsAligned     8-byte aligned, with room for partial_columns(N) columns
+//   kRowsRagged      of any 2-byte alignment (GemmArgs::c_ragged; BASIC and SKINNY only)
+//   kRowsOddSmall    the same, 128 x 128 tiles wherever the plan has tiles of 256 rows (BASIC; see ring_odd_rows)
+enum CRows { kRowsAligned, kRowsRagged, kRowsOddSmall };
+
 // One problem on the variant v (resolved, not AUTO).  from_auto: the caller left the choice to the library, which may then
-// cut the problem in two or leave the streaming kernel for the tile kernel.  c_ragged: C has rows of any 2-byte alignment
-// (GemmArgs::c_ragged; BASIC and SKINNY only); the plan is that of N rounded up to 4.
+// cut the problem in two or leave the streaming kernel for the tile kernel.  The plan is that of N rounded up to 4.
 int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                 int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, int v, bool from_auto,
-                bool c_ragged, void* workspace, size_t workspace_bytes, hipStream_t s, WorkspaceMode mode) {
+                CRows c_rows, void* workspace, size_t workspace_bytes, hipStream_t s, WorkspaceMode mode) {
   const bool strict = mode != kLenient, dry = mode == kStrictDry;
   const int es = elem_bytes(in_dtype);
   const int64_t Np = mi355::partial_columns(N);
-  // Rows of C at odd 2-byte addresses: the tiles of 256 rows store them element by element, about 28 us per round of tiles, the
-  // 128 x 128 tile in wide pieces.  Below 32 k-steps the small tile's longer k loop is the lesser cost: bf16 1000 x 50257 x 768
-  // 182 -> 127 us, 8191 x 8193 x 1024 237 -> 175 us, e4m3 2048 x 8191 x 2048 59 -> 48 us; at 32 and 64 k-steps bf16 2048 x 8191 x
-  // 2048 81 against 82 us, e4m3 4096 x 4097 x 4096 88 against 92 us, 4001 x 6001 x 8192 172 against 191 us.
-  const bool odd_rows = c_ragged && (ldc % 2 != 0 || (uintptr_t)C % 4 != 0) && K * es < 32 * 128;
-  if (from_auto && v == MI355_VARIANT_BASIC && !odd_rows) {
+  if (from_auto && v == MI355_VARIANT_BASIC && c_rows != kRowsOddSmall) {
     // Two launches where the planner finds a cut that spares a partly filled last round (ring_first_piece): each
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
     // the other on the stream and through the same workspace.
@@ -593,13 +593,13 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     const int64_t first = mi355::ring_first_piece(M, Np, K, es, &along_m);
     if (first > 0) {
       const int st = run_variant(A, B, C, along_m ? first : M, along_m ? N : first, K, lda, ldb, ldc, in_dtype, out_dtype, scale,
-                                 scale_a, scale_b, v, false, c_ragged, workspace, workspace_bytes, s, mode);
+                                 scale_a, scale_b, v, false, c_rows, workspace, workspace_bytes, s, mode);
       if (st != MI355_OK) return st;
       const uint8_t* a2 = (const uint8_t*)A + (along_m ? first * lda * es : 0);
       const uint8_t* b2 = (const uint8_t*)B + (along_m ? 0 : first * ldb * es);
       uint8_t* c2 = (uint8_t*)C + (along_m ? first * ldc : first) * 2;   // 16-bit output
       return run_variant(a2, b2, c2, along_m ? M - first : M, along_m ? N : N - first, K, lda, ldb, ldc, in_dtype, out_dtype,
-                         scale, scale_a, scale_b, v, false, c_ragged, workspace, workspace_bytes, s, mode);
+                         scale, scale_a, scale_b, v, false, c_rows, workspace, workspace_bytes, s, mode);
     }
   }
   mi355::GemmArgs g;
@@ -615,7 +615,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
   g.scale_b = scale_b;
   g.mx_a = g.mx_b = nullptr;
   g.c_streams = c_streams(M, N, K, es);
-  g.c_ragged = c_ragged ? 1 : 0;
+  g.c_ragged = c_rows != kRowsAligned ? 1 : 0;
   if (v == MI355_VARIANT_BASIC && rows_want_plain_stores(C, M, N, ldc)) g.c_ragged = 1;
   int rc;
   // The streaming kernel's split count depends on the shape only, never on the leading dimensions,
@@ -648,7 +648,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
         const size_t need = (size_t)splits * (size_t)M * (size_t)Np * sizeof(float);
         if (usable(need)) g.splits = splits;
         else if (strict) return MI355_ERR_SCRATCH;
-      } else if (odd_rows && mi355::ring_tile_rows(tile) == 256) {
+      } else if (c_rows == kRowsOddSmall && mi355::ring_tile_rows(tile) == 256) {
         tile = 128;
       } else {
         int tail_tiles, tail_splits;
@@ -691,28 +691,31 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   if (M <= 0 || N <= 0 || K <= 0 || (uintptr_t)C % 2 != 0) return MI355_OK;
   const bool strict = mode != kLenient;
   const int64_t es = elem_bytes(in_dtype), Np = mi355::partial_columns(N), ldc4 = mi355::partial_columns(ldc);
+  const int64_t Kp = (K + 16 / es - 1) / (16 / es) * (16 / es);
   Repack r;
   const bool large = repack_plan(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, &r);
   if (large && (!workspace || (uintptr_t)workspace % 256 != 0)) return MI355_OK;   // the contract: the generic kernel then
   const bool ab_aligned = (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
+  const bool c_aligned = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 8 == 0, odd = ldc % 2 != 0 || (uintptr_t)C % 4 != 0;
+  const int v = auto_variant(M, Np, Kp, in_dtype);
+  const int v_ragged = v == MI355_VARIANT_ALTERNATE ? MI355_VARIANT_BASIC : v;   // the two kernels that take rows of any alignment
+  const mi355::OddRows how = !c_aligned && odd && v_ragged == MI355_VARIANT_BASIC ? mi355::ring_odd_rows(M, Np, Kp, (int)es) : mi355::OddRows{false, false};
   // The product on operands that the tiled kernels can address, with what is left of the workspace: into the caller's C, or
   // (padded) into a copy of it whose rows are aligned and have room for Np columns.
-  const auto product = [&](const void* a, const void* b, int64_t k, int64_t ld_a, int64_t ld_b, void* c, int64_t ld_c, bool padded,
-                           void* ws, size_t ws_bytes) {
-    const bool c_ragged = !padded && (N % 4 != 0 || ldc % 4 != 0 || (uintptr_t)C % 8 != 0);
-    int v = auto_variant(M, Np, k, in_dtype);
-    if (c_ragged && v == MI355_VARIANT_ALTERNATE) v = MI355_VARIANT_BASIC;   // the two kernels that take such a C
-    return run_variant(a, b, c, M, N, k, ld_a, ld_b, ld_c, in_dtype, out_dtype, scale, scale_a, scale_b, v, true, c_ragged, ws,
-                       ws_bytes, s, mode);
+  const auto product = [&](const void* a, const void* b, int64_t ld_a, int64_t ld_b, void* c, int64_t ld_c, bool padded, void* ws,
+                           size_t ws_bytes) {
+    const CRows rows = padded || c_aligned ? kRowsAligned : how.small_tile ? kRowsOddSmall : kRowsRagged;
+    return run_variant(a, b, c, M, N, Kp, ld_a, ld_b, ld_c, in_dtype, out_dtype, scale, scale_a, scale_b,
+                       rows == kRowsAligned ? v : v_ragged, true, rows, ws, ws_bytes, s, mode);
   };
   // Small e4m3 products stay on fp32 sums (gemm_tn_small, the generic kernel): the matrix cores' fp8 sums are coarser.  Sums that
   // cancel, relative error behind the rounding to fp16: 1.8e-4 with either of the two at every K, 1.8e-4 / 2.4e-4 / 4.0e-4 / 6.9e-4
   // at K = 128 / 1024 / 4096 / 14336 on the matrix cores; bf16 and fp16 products are off by the same on all three.  16-bit
   // products are faster here from the smallest on (M = 1...2048, 1 to 67 million products, us, generic kernel against this: K = 16
   // 4.1...122 / 4.0...8.1, K = 128 13...120 / 4.2...6.0, K = 1024 106...146 / 7...13).
-  if (ab_aligned && (large || in_dtype != MI355_E4M3) && tile256_ok(M, Np, K, lda, ldb, ldc4, in_dtype)) {
+  if (!large && in_dtype != MI355_E4M3 && ab_aligned && tile256_ok(M, Np, K, lda, ldb, ldc4, in_dtype)) {
     *handled = true;
-    return product(A, B, K, lda, ldb, C, ldc, false, workspace, workspace_bytes);
+    return product(A, B, lda, ldb, C, ldc, false, workspace, workspace_bytes);
   }
   if (!large && K >= kSmallMinK && (uintptr_t)A % es == 0 && (uintptr_t)B % es == 0 && 2.0 * (double)M * (double)N * (double)K < kRepackMinFlops) {
     *handled = true;
@@ -731,33 +734,34 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   // they are handed in the end has to pass their check.  So for C, whose padded copy is copied out afterwards.
   const bool copies_b = r.b && (r.Kp != K || (uintptr_t)B % 16 != 0 || !tile256_ok(M, r.Np, r.Kp, r.ld_ab, ldb, r.Np, in_dtype));
   const int64_t ld_a = r.a ? r.ld_ab : lda, ld_b = copies_b ? r.ld_ab : ldb;
-  const bool pads_c = r.c && !tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, ldc4, in_dtype);
-  if (!tile256_ok(M, r.Np, r.Kp, ld_a, ld_b, pads_c ? r.ld_c : ldc4, in_dtype)) return MI355_OK;
-  const size_t bytes_b = copies_b ? r.bytes_b : 0, bytes_c = pads_c ? r.bytes_c : 0, packed = r.bytes_a + bytes_b + bytes_c;
+  const bool in_reach = tile256_ok(M, Np, Kp, ld_a, ld_b, ldc4, in_dtype);
+  const size_t bytes_b = copies_b ? r.bytes_b : 0;
   // What the repacked (aligned) problem wants for its own splits.  The streaming kernel insists
   // on the workspace of its K split, so a lenient call repacks only when the rest covers it.
-  const size_t inner = mi355_gemm_workspace_bytes(M, r.Np, r.Kp, in_dtype, MI355_VARIANT_AUTO);
-  const bool inner_streams = auto_variant(M, r.Np, r.Kp, in_dtype) == MI355_VARIANT_SKINNY;
-  const bool fits = workspace_bytes >= packed && (workspace_bytes - packed >= inner || (!strict && !inner_streams));
-  if (strict && !fits) {
+  const size_t inner = mi355_gemm_workspace_bytes(M, Np, Kp, in_dtype, MI355_VARIANT_AUTO);
+  for (const bool pads_c : {true, false}) {
+    if (pads_c ? in_reach && !how.padded : !in_reach) continue;
+    if (pads_c && !(r.c && tile256_ok(M, Np, Kp, ld_a, ld_b, r.ld_c, in_dtype))) continue;
+    const size_t bytes_c = pads_c ? r.bytes_c : 0, packed = r.bytes_a + bytes_b + bytes_c;
+    const bool fits = !packed || (workspace_bytes >= packed && (workspace_bytes - packed >= inner || (!strict && v != MI355_VARIANT_SKINNY)));
+    *handled = *handled || strict;   // refused unless one of them fits
+    if (!fits) continue;
     *handled = true;
-    return MI355_ERR_SCRATCH;
+    if (packed && mode == kStrictDry) return MI355_OK;
+    uint8_t* wa = (uint8_t*)workspace;
+    uint8_t* wb = wa + r.bytes_a;
+    uint8_t* wc = wb + bytes_b;
+    uint8_t* rest = wc + bytes_c;
+    const size_t rest_bytes = workspace_bytes - packed;
+    const mi355::RepackOperand pack_a = {(const uint8_t*)A, r.a ? M : 0, lda * es, wa, r.ld_ab * es};
+    const mi355::RepackOperand pack_b = {(const uint8_t*)B, copies_b ? N : 0, ldb * es, wb, r.ld_ab * es};
+    if (mi355::launch_repack_rows(pack_a, pack_b, K * es, (int)es, s) != 0) return MI355_ERR_LAUNCH;
+    const int st = product(r.a ? wa : A, copies_b ? wb : B, ld_a, ld_b, pads_c ? (void*)wc : C, pads_c ? r.ld_c : ldc, pads_c,
+                           rest_bytes ? rest : nullptr, rest_bytes);
+    if (st != MI355_OK || !pads_c) return st;
+    return mi355::launch_copy_out(wc, M, N, r.ld_c, C, ldc, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
   }
-  if (!fits) return MI355_OK;
-  *handled = true;
-  if (mode == kStrictDry) return MI355_OK;
-  uint8_t* wa = (uint8_t*)workspace;
-  uint8_t* wb = wa + r.bytes_a;
-  uint8_t* wc = wb + bytes_b;
-  uint8_t* rest = wc + bytes_c;
-  const size_t rest_bytes = workspace_bytes - packed;
-  const mi355::RepackOperand pack_a = {(const uint8_t*)A, r.a ? M : 0, lda * es, wa, r.ld_ab * es};
-  const mi355::RepackOperand pack_b = {(const uint8_t*)B, copies_b ? N : 0, ldb * es, wb, r.ld_ab * es};
-  if (mi355::launch_repack_rows(pack_a, pack_b, K * es, (int)es, s) != 0) return MI355_ERR_LAUNCH;
-  const int st = product(r.a ? wa : A, copies_b ? wb : B, r.Kp, ld_a, ld_b, pads_c ? (void*)wc : C, pads_c ? r.ld_c : ldc, pads_c,
-                         rest_bytes ? rest : nullptr, rest_bytes);
-  if (st != MI355_OK || !pads_c) return st;
-  return mi355::launch_copy_out(wc, M, N, r.ld_c, C, ldc, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
+  return *handled ? MI355_ERR_SCRATCH : MI355_OK;
 }
 
 int run_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,
@@ -784,7 +788,7 @@ int run_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_
                        mode, &handled);
     if (handled) return st;
   }
-  return run_variant(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, out_dtype, scale, scale_a, scale_b, v, from_auto, false, workspace,
+  return run_variant(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, out_dtype, scale, scale_a, scale_b, v, from_auto, kRowsAligned, workspace,
                      workspace_bytes, s, mode);
 }
 

@@ -78,6 +78,12 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
+// How MI355_VARIANT_AUTO stores a C whose rows start at odd 2-byte addresses, where the plan has tiles of 256 rows: into a
+// padded copy that is then copied out (if there is memory for it), and if not, from 128 x 128 tiles or else element by element.
+struct OddRows {
+  bool padded, small_tile;
+};
+OddRows ring_odd_rows(int64_t M, int64_t N, int64_t K, int elem_bytes);
 // C = rne(scale * sum_s partial[s]) for partial laid out [splits][M][partial_columns(N)] in fp32.
 int launch_splitk_reduce(const float* partial, const GemmArgs& g, int out_dtype, hipStream_t stream);
 int launch_tile_ring(const GemmArgs& g, int in_dtype, int out_dtype, int tile, hipStream_t stream);
@@ -125,8 +131,7 @@ struct RepackOperand {
   int64_t dst_ld;
 };
 int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, int64_t row_bytes, int elem_bytes, hipStream_t stream);
-// A (rows x cols) block of 16-bit elements with row stride src_ld elements (a multiple of 4) -> row stride dst_ld elements at any
-// 2-byte alignment.
+// A (rows x cols) block of 16-bit elements with row stride src_ld elements -> row stride dst_ld elements, at any 2-byte alignment.
 int launch_copy_out(const void* src, int64_t rows, int64_t cols, int64_t src_ld, void* dst, int64_t dst_ld, hipStream_t stream);
 
 }  // namespace mi355

@@ -71,14 +71,34 @@ __global__ __launch_bounds__(256) void repack_rows(RepackOperand first, RepackOp
     if (to[i] >= 0) *(u32x4*)(op.dst + to[i]) = v[i];
 }
 
-// One thread per four columns: the source rows are 8-byte aligned, the destination has only element alignment.
-__global__ __launch_bounds__(256) void copy_out(const uint16_t* __restrict__ src, int64_t rows, int64_t cols, int64_t src_ld,
-                                                uint16_t* __restrict__ dst, int64_t dst_ld) {
-  const int64_t quads = (cols + 3) / 4;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= rows * quads) return;
-  const int64_t row = id / quads, col = (id % quads) * 4;
-  store_ragged_quad(dst + row * dst_ld + col, *(const u32x2*)(src + row * src_ld + col), cols - col);
+// Bound by its read and its write: one wave per run of kRunColumns columns of a row, cut where the destination is 16-byte
+// aligned, so that it writes whole lines (a load needs no alignment on this target, and a misaligned one costs less than a
+// misaligned store); four loads in flight per lane.  4096 x 14337 bf16 8 us less than with 8-byte pieces cut at the source's
+// alignment.
+constexpr uint32_t kRunChunks = 4 * 64, kRunColumns = 8 * kRunChunks;
+__global__ __launch_bounds__(256) void copy_out(const uint16_t* __restrict__ src, int64_t waves, int64_t runs_per_row, int64_t cols,
+                                                int64_t src_ld, uint16_t* __restrict__ dst, int64_t dst_ld) {
+  const int64_t wave = (int64_t)blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (wave >= waves) return;
+  const int64_t row = wave / runs_per_row, run = wave % runs_per_row;
+  const uint16_t* from = src + row * src_ld;
+  uint16_t* to = dst + row * dst_ld;
+  const int64_t first = run * kRunColumns - (int64_t)((uintptr_t)to % 16 / 2);   // the first chunk of a row may begin before it
+  u32x4 v[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t col = first + (int64_t)(i * 64 + (threadIdx.x & 63)) * 8;
+    if (col >= 0 && col + 8 <= cols) __builtin_memcpy(&v[i], from + col, 16);
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t col = first + (int64_t)(i * 64 + (threadIdx.x & 63)) * 8;
+    if (col >= 0 && col + 8 <= cols) {
+      *(u32x4*)(to + col) = v[i];
+    } else if (col + 8 > 0 && col < cols) {
+      for (int64_t c = col < 0 ? 0 : col; c < col + 8 && c < cols; ++c) to[c] = from[c];
+    }
+  }
 }
 
 template <class T, class OutT>
@@ -117,11 +137,11 @@ int launch_repack_rows(const RepackOperand& first, const RepackOperand& second, 
 }
 
 int launch_copy_out(const void* src, int64_t rows, int64_t cols, int64_t src_ld, void* dst, int64_t dst_ld, hipStream_t stream) {
-  const int64_t n = rows * ((cols + 3) / 4), blocks = (n + 255) / 256;
-  if (n == 0) return 0;
-  if (blocks >= ((int64_t)1 << 31) || src_ld % 4 != 0 || (uintptr_t)src % 8 != 0) return -1;
-  hipLaunchKernelGGL(copy_out, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)src, rows, cols, src_ld, (uint16_t*)dst,
-                     dst_ld);
+  if (rows == 0 || cols == 0) return 0;
+  const int64_t runs = (cols + 7 + kRunColumns - 1) / kRunColumns, waves = rows * runs, blocks = (waves + 3) / 4;
+  if (blocks >= ((int64_t)1 << 31)) return -1;
+  hipLaunchKernelGGL(copy_out, dim3((unsigned)blocks), dim3(256), 0, stream, (const uint16_t*)src, waves, runs, cols, src_ld,
+                     (uint16_t*)dst, dst_ld);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -141,6 +141,14 @@ double estimate_us(int tile, int64_t M, int64_t N, int64_t K, int elem_bytes, do
   return rounds * (item_steps * step_us + c.fixed) + (partial_mb > 0.0 ? c.reduce_mb * partial_mb + c.reduce : 0.0);
 }
 
+double shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
+  const double a = estimate_us(256, M, N, K, elem_bytes), b = estimate_us(kRingTile256x128, M, N, K, elem_bytes),
+               c = estimate_us(128, M, N, K, elem_bytes);
+  return a < b ? (a < c ? a : c) : (b < c ? b : c);
+}
+
+constexpr double kSecondLaunchUs = 3.0;
+
 }  // namespace
 
 // One row (M <= 128) or one column (N <= 128) of 128 x 128 tiles on the nine-slot ring, K split as
@@ -231,12 +239,8 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
   const int64_t steps = k_steps_of(K, elem_bytes);
   if (tm * tn <= kCuSlots || (tm * tn) % kCuSlots == 0 || steps < kShortSteps) return 0;
   if (10 * tm * tn > 36 * kCuSlots || (10 * tm * tn > 34 * kCuSlots && steps > 64)) return 0;
-  const auto best_of = [&](int64_t m, int64_t n) {
-    const double a = estimate_us(256, m, n, K, elem_bytes), b = estimate_us(kRingTile256x128, m, n, K, elem_bytes),
-                 c = estimate_us(128, m, n, K, elem_bytes);
-    return a < b ? (a < c ? a : c) : (b < c ? b : c);
-  };
-  const double whole = best_of(M, N), second_launch_us = 3.0;
+  const auto best_of = [&](int64_t m, int64_t n) { return shortest_us(m, n, K, elem_bytes); };
+  const double whole = best_of(M, N);
   double best = 0.98 * whole;
   int64_t extent = 0;
   for (int axis = 0; axis < 2; ++axis) {
@@ -247,14 +251,41 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
     int64_t c = (along - 1) / step * step;
     for (int tries = 0; tries < 4 && c >= step; ++tries, c -= step) {
       const double e = axis == 0 ? best_of(M, c * 256) + best_of(M, N - c * 256) : best_of(c * 256, N) + best_of(M - c * 256, N);
-      if (e + second_launch_us < best) {
-        best = e + second_launch_us;
+      if (e + kSecondLaunchUs < best) {
+        best = e + kSecondLaunchUs;
         extent = c * 256;
         *along_m = axis == 1;
       }
     }
   }
   return extent;
+}
+
+// Tiles of 256 rows store rows that start at odd 2-byte addresses element by element, 24...28 us per round of 256 x 256 tiles
+// more than wide stores take; the 128 x 128 tile stores them in wide pieces, but has the longer k loop; a padded copy of C costs
+// a pass that reads and writes it.  The line between the last two: all three timed on 435 problems (22 sizes, M = 512...9335,
+// N = 859...50257, 1...128 k-steps, bf16 and e4m3).  The copy, at 0.1 us per MB moved and 10 us, is taken where the estimate of
+// the plan and it is shorter than that of the small tiles, which take up to 15 % longer than estimated with such rows; the choice
+// costs 1.1 % of the best one's time on average (always small tiles 8.7 %, always the copy 7.0 %, small tiles below 32 k-steps and
+// elements from there on 8.5 %): bf16 4096 x 14337 x 2048 288 us by elements, 282 on small tiles, 235 by the copy, 8192 x 8193 x
+// 4096 524, 499 and 470.  Below 16 k-steps small tiles take 0.58...0.98 of the copy's time but for 4096 x 14337 and 4096 x 9217
+// (1.03...1.14), and below 32 the copy has to come out of the Infinity Cache (9335 x 9969 x 1536, 186 MB of C, 293 us on small
+// tiles, 314 by the copy).
+OddRows ring_odd_rows(int64_t M, int64_t N, int64_t K, int elem_bytes) {
+  bool along_m = false;
+  const int64_t first = ring_first_piece(M, N, K, elem_bytes, &along_m), steps = k_steps_of(K, elem_bytes);
+  const int64_t m1 = along_m ? first : M, n1 = along_m ? N : first, m2 = along_m ? M - first : M, n2 = along_m ? N : N - first;
+  const auto by_elements = [&](int64_t m, int64_t n) {   // sums of a K split are rounded and stored by another kernel
+    return ring_tile_rows(ring_tile_edge(m, n, K, elem_bytes)) == 256 && ring_splits(m, n, K, elem_bytes) == 1;
+  };
+  if (first > 0 ? !by_elements(m1, n1) && !by_elements(m2, n2) : !by_elements(M, N)) return {false, false};
+  const double plan_us = first > 0 ? shortest_us(m1, n1, K, elem_bytes) + shortest_us(m2, n2, K, elem_bytes) + kSecondLaunchUs
+                                   : shortest_us(M, N, K, elem_bytes);
+  const double copy_mb = (double)M * (double)N * 4e-6;
+  const bool few_steps = steps < 2 * kShortSteps;
+  const bool padded = steps >= kShortSteps && (!few_steps || copy_mb <= 2.0 * 134.2) &&
+                      plan_us + 0.1 * copy_mb + 10.0 < 1.15 * estimate_us(128, M, N, K, elem_bytes);
+  return {padded, !padded || few_steps};
 }
 
 // K splits for the single-group kernel on the tile ring_tile_edge picks.

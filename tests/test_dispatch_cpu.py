@@ -163,3 +163,28 @@ def test_streaming_kernel_has_a_form_for_each_kind_of_rows(launches, M, N, K, sp
     assert ("Lb1E" in writes_c) == ragged
     if split:
         assert "Lb1E" not in got[0][0]
+
+
+# What the padded copy of C is for besides: rows at odd 2-byte addresses under a plan with tiles of 256 rows (the planner's choice
+# is held here at sizes where it is clear; everything else is the same product).
+@pytest.mark.parametrize("M,N,K,in_dt,padded", [(4096, 14337, 2048, ac.BF16, True), (8192, 8193, 4096, ac.F16, True), (2048, 4097, 8192, ac.E4M3, True),
+                                                (1000, 50257, 768, ac.BF16, False), (8192, 8193, 512, ac.BF16, False), (9335, 9969, 1536, ac.BF16, False)])
+def test_rows_of_c_at_odd_addresses(launches, M, N, K, in_dt, padded):
+    cases = [case(M, N, K, in_dt), case(M, N, K, in_dt, c=C + 2), case(M, N, K, in_dt, room=256), case(M, N, K, in_dt, noalloc=True),
+             case(M, N + 1 - N % 4, K, in_dt, ldc=N + 4), case(M, N, K + 1, in_dt), case(M, N, K, in_dt, ldc=N + 1)]
+    for c, (st, need, got) in zip(cases, launches(cases)):
+        assert st == ac.OK
+        products = [v for name, v in got if matrix_core(name)]
+        assert products and not any("simple" in name for name, _ in got)
+        room = need if c["room"] is None else c["room"]
+        odd = c["ldc"] % 2 != 0 or c["C"] % 4 != 0
+        fits = room > 2 * M * N and (not c["noalloc"] or 2 * M * -(-N // 64) * 64 <= ac.NOALLOC_SCRATCH_BYTES)
+        assert ("copy_out" in got[-1][0]) == (padded and odd and fits), (c, got)
+        for v in products:
+            assert v["c_ragged"] == 0 or v["C"] >= c["C"] and v["ldc"] == c["ldc"]
+            if "copy_out" in got[-1][0]:      # inside the workspace, behind the copies of the operands if there are any
+                packed = [p for name, p in got if "repack_rows" in name]
+                end = max([o["dst"] + o["rows"] * o["dst_ld"] for p in packed for o in p], default=WS) if not c["noalloc"] else 0
+                assert v["C"] >= end and v["C"] + 2 * ((v["M"] - 1) * v["ldc"] + v["N"]) <= (WS if not c["noalloc"] else 1 << 30) + max(room, 64 << 20)
+        # no row or column is left to nobody
+        assert sum(v["M"] * v["N"] for v in products) == M * c["N"]

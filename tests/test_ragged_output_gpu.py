@@ -76,6 +76,15 @@ def test_aligned_n_in_rows_of_odd_stride_and_address(abi):
         close(C, A, B)
 
 
+def close_everywhere(C, A, B):
+    """close() with the product in float64 on the GPU, for sizes where the CPU takes long; every element against the bound."""
+    want = A.cuda().double() @ B.cuda().double().T
+    tol = 3e-2 if A.dtype == torch.float8_e4m3fn else 1e-2
+    diff = C.cuda() - want
+    assert float(diff.norm() / want.norm()) <= tol
+    assert float(diff.abs().max()) <= 2.0 ** -7 * float(want.abs().max()) + 1e-3
+
+
 @pytest.mark.parametrize("M,N,K,dt", [(4096, 6145, 4096, torch.bfloat16), (4352, 4349, 2048, torch.float16), (2304, 8190, 1024, torch.bfloat16)])
 def test_tail_split_and_two_pieces(abi, M, N, K, dt):
     A, B = operand(M, K, dt, 3).cuda().float().cpu().to(dt), operand(N, K, dt, 4)
@@ -84,6 +93,18 @@ def test_tail_split_and_two_pieces(abi, M, N, K, dt):
     assert kept and need >= 0
     rows = torch.randperm(M, generator=torch.Generator().manual_seed(5))[:48]
     close(C[rows], A[rows], B)
+
+
+# Rows of C at odd 2-byte addresses where the library computes into a padded copy: one launch, a tail split, two launches.
+@pytest.mark.parametrize("M,N,K,dt", [(2049, 2051, 4096, torch.bfloat16), (513, 8195, 4096, torch.float16), (2049, 6145, 4096, torch.float8_e4m3fn),
+                                      (2049, 6145, 2056, torch.bfloat16), (2049, 8195, 4096, torch.bfloat16), (4096, 4111, 4096, torch.bfloat16),
+                                      (1025, 6147, 4090, torch.float16)])
+def test_rows_at_odd_addresses(abi, M, N, K, dt):
+    A, B = operand(M, K, dt, 25), operand(N, K, dt, 26)
+    for offset, pad in ((0, 0), (1, 0), (3, 2), (2, 1)):
+        C, kept = run(abi, A, B, offset, N + pad)
+        assert kept
+        close_everywhere(C, A, B)
 
 
 @pytest.mark.parametrize("workspace", [True, False])
