@@ -4,6 +4,8 @@ matrix-core kernels directly, on every plan that can take them; and operands rep
 The reference product is torch's in float64 on the CPU; tolerances are those of the other GPU tests (1e-2 for 16-bit
 operands, 3e-2 for fp8, relative Frobenius).  Everything around C must keep its bits.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -23,7 +25,7 @@ def abi():
     return ac.load()
 
 
-def run(abi, A, B, offset, ldc, workspace=True, room=True):
+def run(abi, A, B, offset, ldc, workspace=True, room=True, ws_bytes=None):
     """C inside a buffer of a known pattern, `offset` elements in, row stride ldc: (C, whether the rest kept its pattern)."""
     M, N, K = A.shape[0], B.shape[0], A.shape[1]
     out_dt = OUT[A.dtype]
@@ -31,6 +33,8 @@ def run(abi, A, B, offset, ldc, workspace=True, room=True):
     Cv = torch.as_strided(buf, (M, N), (ldc, 1), offset).view(out_dt)
     need = abi.mi355_gemm_workspace_bytes(M, N, K, ac.torch_code(A.dtype), ac.AUTO) if workspace else 0
     need += 4 * M * (N + 4) * 16 if workspace and room else 0   # for every plan, also where the query counts on aligned rows
+    if ws_bytes is not None:
+        need = ws_bytes
     ws = torch.full((max(need, 256),), 0xff, dtype=torch.uint8, device="cuda")
     Ad, Bd = A.cuda(), B.cuda()
     st = abi.mi355_gemm_tn(Ad.data_ptr(), Bd.data_ptr(), Cv.data_ptr(), M, N, K, K, K, ldc, ac.torch_code(A.dtype),
@@ -85,14 +89,23 @@ def close_everywhere(C, A, B):
     assert float(diff.abs().max()) <= 2.0 ** -7 * float(want.abs().max()) + 1e-3
 
 
-@pytest.mark.parametrize("M,N,K,dt", [(4096, 6145, 4096, torch.bfloat16), (4352, 4349, 2048, torch.float16), (2304, 8190, 1024, torch.bfloat16)])
-def test_tail_split_and_two_pieces(abi, M, N, K, dt):
-    A, B = operand(M, K, dt, 3).cuda().float().cpu().to(dt), operand(N, K, dt, 4)
-    need = abi.mi355_gemm_workspace_bytes(M, N, K, ac.torch_code(dt), ac.AUTO)
-    C, kept = run(abi, A, B, 1, N)
-    assert kept and need >= 0
-    rows = torch.randperm(M, generator=torch.Generator().manual_seed(5))[:48]
-    close(C[rows], A[rows], B)
+# N % 4 == 2; the plan is that of N rounded up to 4: a tail split, or two launches with the second one a few columns or rows.
+@pytest.mark.parametrize("M,N,K,dt,pieces", [
+    (5000, 3498, 4096, torch.bfloat16, 1), (4352, 4350, 4096, torch.float16, 1), (6144, 4094, 8192, torch.float8_e4m3fn, 1),
+    (4096, 4110, 4096, torch.bfloat16, 2), (4110, 4094, 4096, torch.float16, 2), (2304, 8190, 2048, torch.bfloat16, 2),
+    (4096, 4110, 8192, torch.float8_e4m3fn, 2)])
+def test_tail_split_and_two_pieces(abi, M, N, K, dt, pieces):
+    code, Np = ac.torch_code(dt), -(-N // 4) * 4
+    cut = [ctypes.c_int64(), ctypes.c_int64()]
+    assert abi.mi355_gemm_pieces(M, Np, K, code, ac.AUTO, *[ctypes.byref(x) for x in cut]) == pieces
+    assert pieces == 2 or ac.plan(abi, M, Np, K, code)[4] > 0
+    A, B = operand(M, K, dt, 3), operand(N, K, dt, 4)
+    inner = max(abi.mi355_gemm_workspace_bytes(M, Np, K, code, ac.AUTO), 256)
+    # rows at even 2-byte addresses; at odd ones with room for the split's planes only (stored directly), and with a padded copy of C
+    for offset, pad, ws_bytes in ((0, 0, inner), (1, 0, inner), (0, 1, inner), (1, 1, None)):
+        C, kept = run(abi, A, B, offset, N + pad, ws_bytes=ws_bytes)
+        assert kept
+        close_everywhere(C, A, B)
 
 
 # Rows of C at odd 2-byte addresses where the library computes into a padded copy: one launch, a tail split, two launches.
