@@ -70,6 +70,9 @@ __global__ __launch_bounds__(kThreads) void gemm_tn_stream(GemmArgs g, float* pa
   static_assert(kVm * (kDepth - 1) < 64, "vmcnt is a 6-bit counter");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[kDepth * kStageBytes];
 
+  // The arguments span three cache lines, and the last one is otherwise asked for only behind the divisions below, with a wait of
+  // its own in front of the first copy (fp8 8 x 1024 x 1024 4.65 -> 4.45 us, bf16 16 x 14336 x 4096 22.1 -> 21.8).
+  asm volatile("" ::"s"(splits));
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
