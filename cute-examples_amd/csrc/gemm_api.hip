@@ -85,7 +85,10 @@ int32_t c_streams(int64_t M, int64_t N, int64_t K, int elem_bytes) {
 // waits for their way to memory.  Rows of C 8 or 16 bytes past a multiple of 128, write-through against plain, bf16 and e4m3,
 // 512...8192 elements of K: outputs of 4 Mi elements and more 3-44 % faster plain (bf16 4096 x 4096 x 1024 41.5 -> 32.1 us,
 // 2048 x 14336 x 4096 197.9 -> 184.9 us, e4m3 8192 x 8192 x 1024 129.3 -> 83.1 us), at 2 Mi elements and below within the
-// noise of a few percent.  Rows of whole 64 bytes: from 7 % faster to 14 % slower, mostly slower.
+// noise of a few percent.  Rows of whole 64 bytes: from 7 % faster to 14 % slower, mostly slower.  A contiguous C with such rows
+// has a partial last tile column, which the tiles of 256 rows then store element by element; bf16 and e4m3 at 32 of these (M =
+// 1024...8192, N = 4100...50260 with N % 4 == 0, K = 768...8192) 3-34 % faster plain all the same (bf16 8192 x 8208 x 8192 826 ->
+// 802 us, 2048 x 14344 x 1024 78 -> 60 us), but for 1024 x 4104 x 8192 (76.1 and 76.5 us).
 bool rows_want_plain_stores(const void* C, int64_t M, int64_t N, int64_t ldc) {
   return ((ldc * 2) % 64 != 0 || (uintptr_t)C % 64 != 0) && M * N >= ((int64_t)4 << 20);
 }

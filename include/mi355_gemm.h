@@ -76,7 +76,9 @@ enum mi355_status {
  *             problem the tiled kernels cannot address (K*elem_bytes % 16, strides, pointers);
  *             without it such a problem, or a large one with N or ldc % 4 != 0, runs on the slow
  *             generic kernel.  With it, an output whose rows only its element type aligns is stored
- *             by the tiled kernels directly (mi355_gemm_select_variant still reports SIMPLE)
+ *             by the tiled kernels directly, or computed in a padded copy of it that the workspace
+ *             holds and copied out, whichever is shorter (mi355_gemm_select_variant still reports
+ *             SIMPLE)
  *   stream    hipStream_t on which the kernels are enqueued (NULL = the null stream)
  *
  * Replaces test::gemm_tn_test (kernels/gemm_kernels/sm90a/gemm_test.cu:12-92): same operand
@@ -124,8 +126,9 @@ int mi355_gemm_tn_scaled(const void *A, const void *B, void *C,
  *     is never silently run on a slower path.  K-split partial planes and tail-split partial tiles
  *     always fit (a plan has at most 256 split items of at most 256 x 256 floats = 64 MiB), and
  *     problems that want no workspace have no size limit, so in practice the limit applies to the
- *     repacked operands of a large misaligned problem (K*elem_bytes % 16, N % 4, strides, pointers;
- *     mi355_gemm_workspace_bytes reports the figure for contiguous operands).
+ *     repacked operands of a large misaligned problem (K*elem_bytes % 16, strides, pointers;
+ *     mi355_gemm_workspace_bytes reports the most that contiguous operands can take, copies that are
+ *     only made of rows out of reach among it).
  *   - All calls on one GPU share that GPU's buffer, which keeps the last call's contents (nothing
  *     in it needs to start at zero).  Calls that may overlap on one GPU (different streams, or
  *     several host threads) race on it: serialise them, or use mi355_gemm_tn with a workspace each.

@@ -72,6 +72,16 @@ def test_ragged_rows(abi, dt, M, N, K, offset, pad):
     close(C, A, B)
 
 
+# Small e4m3 products do not get to the kernels that the smaller sizes above are there for; these do.
+@pytest.mark.parametrize("M,N,K", [(16, 14333, 592), (30, 14333, 4096), (700, 1303, 192)])   # streaming, unsplit; a ragged last k-step
+@pytest.mark.parametrize("offset,pad", [(0, 0), (1, 0), (2, 3), (4, 2)])
+def test_ragged_rows_of_large_fp8_products(abi, M, N, K, offset, pad):
+    A, B = operand(M, K, torch.float8_e4m3fn, M), operand(N, K, torch.float8_e4m3fn, N)
+    C, kept = run(abi, A, B, offset, N + pad)
+    assert kept
+    close(C, A, B)
+
+
 def test_aligned_n_in_rows_of_odd_stride_and_address(abi):
     for M, N, K, offset, pad in [(300, 512, 256, 1, 1), (300, 512, 256, 2, 0), (40, 512, 512, 0, 2), (4096, 4096, 128, 1, 0)]:
         A, B = operand(M, K, torch.bfloat16, 1), operand(N, K, torch.bfloat16, 2)

@@ -1,4 +1,4 @@
-"""Small products with rows of any alignment (gemm_tn_small.hip through MI355_VARIANT_AUTO).
+"""Small products with rows of any alignment (gemm_tn_small.hip through MI355_VARIANT_AUTO; the generic kernel below K = 128).
 
 Reference: the product in float64 on the CPU.  fp32 sums of exact products in any order are off by at most about
 K * 2^-24 of the sum of magnitudes; the output's rounding (2^-8 bf16, 2^-11 fp16 of the value) comes on top.
