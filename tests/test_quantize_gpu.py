@@ -32,6 +32,19 @@ def test_sizes_around_the_launch_rules(dtype, n):
         assert torch.equal(q.cpu().view(torch.uint8), want_q)
 
 
+# Around 32 MiB of input (1024 workgroups up to there) with more than one turn of four pieces each, and with pieces left over.
+@pytest.mark.parametrize("dtype,n", [
+    (torch.bfloat16, 16 << 20), (torch.bfloat16, (16 << 20) + 5), (torch.float16, 4099 * 2048 + 9), (torch.float32, 8 << 20),
+    (torch.float32, (8 << 20) + 2055), (torch.bfloat16, 1023 * 2048 + 8), (torch.bfloat16, 4096 * 2048 - 8)])
+def test_pieces_of_a_workgroup(dtype, n):
+    import gemm_kernels
+    x = torch.randn(n, generator=torch.Generator().manual_seed(n)).to(dtype)
+    want_q, want_s = expected(x)
+    q, s = gemm_kernels.quantize_e4m3(x.cuda())
+    assert float(s) == want_s
+    assert torch.equal(q.cpu().view(torch.uint8), want_q)
+
+
 # amax from the subnormals to the largest finite number: the corrected reciprocal up to and beyond its range, the division outside.
 # The smallest is above 448 * 2^-150: below, the scale itself is 0 and the quotients are infinities and NaNs of either sign.
 @pytest.mark.parametrize("amax", [1e-42, 3e-39, 448 * 2.0 ** -61, 448 * 2.0 ** -60, 448 * 2.0 ** -59, 7e-6, 0.7, 300.0, 448 * 1.99999988,
