@@ -86,9 +86,10 @@ int32_t c_streams(int64_t M, int64_t N, int64_t K, int elem_bytes) {
 // 512...8192 elements of K: outputs of 4 Mi elements and more 3-44 % faster plain (bf16 4096 x 4096 x 1024 41.5 -> 32.1 us,
 // 2048 x 14336 x 4096 197.9 -> 184.9 us, e4m3 8192 x 8192 x 1024 129.3 -> 83.1 us), at 2 Mi elements and below within the
 // noise of a few percent.  Rows of whole 64 bytes: from 7 % faster to 14 % slower, mostly slower.  A contiguous C with such rows
-// has a partial last tile column, which the tiles of 256 rows then store element by element; bf16 and e4m3 at 32 of these (M =
-// 1024...8192, N = 4100...50260 with N % 4 == 0, K = 768...8192) 3-34 % faster plain all the same (bf16 8192 x 8208 x 8192 826 ->
-// 802 us, 2048 x 14344 x 1024 78 -> 60 us), but for 1024 x 4104 x 8192 (76.1 and 76.5 us).
+// has a partial last tile column (stored in quads, tile_store.h): 220 of them and of padded ones drawn from M = 181...8192, N =
+// 256...32768, K = 45...11585, all three input types, 11 % faster plain on average (e4m3 5484 x 5608 x 224 41.1 -> 24.7 us, 4476 x
+// 6064 x 864 51.1 -> 35.8, fp16 304 x 14448 x 1648 34.0 -> 31.1), nine of them 2-7 % slower, by 0.8 us at most (less than a round
+// of tiles: e4m3 232 x 26160 x 448 9.6 -> 10.2 us, fp16 2206 x 4080 x 1472 31.5 -> 32.3).
 bool rows_want_plain_stores(const void* C, int64_t M, int64_t N, int64_t ldc) {
   return ((ldc * 2) % 64 != 0 || (uintptr_t)C % 64 != 0) && M * N >= ((int64_t)4 << 20);
 }

@@ -188,3 +188,14 @@ def test_rows_of_c_at_odd_addresses(launches, M, N, K, in_dt, padded):
                 assert v["C"] >= end and v["C"] + 2 * ((v["M"] - 1) * v["ldc"] + v["N"]) <= (WS if not c["noalloc"] else 1 << 30) + max(room, 64 << 20)
         # no row or column is left to nobody
         assert sum(v["M"] * v["N"] for v in products) == M * c["N"]
+
+
+@pytest.mark.parametrize("M,N,K,in_dt", [(908, 10640, 832, ac.F16), (3612, 1516, 4016, ac.E4M3), (8192, 8192, 512, ac.BF16), (1024, 1032, 512, ac.BF16)])
+def test_rows_of_less_than_64_bytes_are_stored_plainly(launches, M, N, K, in_dt):
+    cases = [case(M, N, K, in_dt, ldc=N + pad, c=C + off) for pad in (0, 4, 32) for off in (0, 8, 64)]
+    for c, (st, _, got) in zip(cases, launches(cases)):
+        assert st == ac.OK
+        plain = M * N >= 4 << 20 and (c["ldc"] * 2 % 64 != 0 or c["C"] % 64 != 0)
+        for name, v in got:
+            if "gemm_tn_tile_ring" in name:
+                assert bool(v["c_ragged"]) == plain

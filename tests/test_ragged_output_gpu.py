@@ -118,6 +118,17 @@ def test_tail_split_and_two_pieces(abi, M, N, K, dt, pieces):
         close_everywhere(C, A, B)
 
 
+# Rows of C that are aligned, but not by 64 bytes, and a partial last tile column of tiles of 256 rows (4 Mi outputs and more).
+@pytest.mark.parametrize("M,N,K,dt", [(908, 10640, 832, torch.float16), (2206, 4076, 1472, torch.bfloat16), (3612, 1516, 4016, torch.float8_e4m3fn),
+                                      (5484, 5608, 224, torch.float8_e4m3fn), (2049, 8196, 2048, torch.bfloat16)])
+def test_aligned_rows_with_a_partial_last_column(abi, M, N, K, dt):
+    A, B = operand(M, K, dt, 27), operand(N, K, dt, 28)
+    for offset, pad in ((0, 0), (4, 0), (0, 4), (8, 12)):
+        C, kept = run(abi, A, B, offset, N + pad)
+        assert kept
+        close_everywhere(C, A, B)
+
+
 # Rows of C at odd 2-byte addresses where the library computes into a padded copy: one launch, a tail split, two launches.
 @pytest.mark.parametrize("M,N,K,dt", [(2049, 2051, 4096, torch.bfloat16), (513, 8195, 4096, torch.float16), (2049, 6145, 4096, torch.float8_e4m3fn),
                                       (2049, 6145, 2056, torch.bfloat16), (2049, 8195, 4096, torch.bfloat16), (4096, 4111, 4096, torch.bfloat16),
