@@ -13,6 +13,7 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((ext_vector_type(4))) int i32x4;
 typedef __attribute__((ext_vector_type(8))) int i32x8;
 typedef __attribute__((ext_vector_type(2))) unsigned u32x2;
+typedef __attribute__((ext_vector_type(3))) unsigned u32x3;
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 
 // Element-type tags.  kBytes = bytes per element; kSliceChunks = 16-byte chunks of one operand
@@ -179,9 +180,8 @@ template <> struct Pack4<F16> {
   }
 };
 
-// Stores of four or eight 16-bit outputs at any 2-byte alignment; only the first `left` of them when there are fewer left in
-// the row.  (Global accesses need no alignment on this target, but a wide store that is not dword-aligned takes longer than
-// the three pieces it is cut into here: bf16 rows of odd length, 300 x 4097 x 1024 13.0 -> 10.9 us.)
+// Stores of four 16-bit outputs at any 2-byte alignment (global accesses need none on this target); only the first `left` of
+// them when there are fewer left in the row.
 __device__ __forceinline__ void store_ragged_quad(uint16_t* p, u32x2 v, int64_t left) {
   if (left >= 4) {
     __builtin_memcpy(p, &v, 8);
@@ -190,24 +190,6 @@ __device__ __forceinline__ void store_ragged_quad(uint16_t* p, u32x2 v, int64_t 
   if (left > 0) p[0] = (uint16_t)v[0];
   if (left > 1) p[1] = (uint16_t)(v[0] >> 16);
   if (left > 2) p[2] = (uint16_t)v[1];
-}
-__device__ __forceinline__ void store_ragged_octet(uint16_t* p, u32x4 v, int64_t left) {
-  if (left >= 8) {
-    if ((uintptr_t)p & 2) {
-      u32x4 mid = {(v[0] >> 16) | (v[1] << 16), (v[1] >> 16) | (v[2] << 16), (v[2] >> 16) | (v[3] << 16), 0u};
-      asm volatile("" : "+v"(mid));
-      __builtin_memcpy(__builtin_assume_aligned(p + 1, 4), &mid, 12);
-      p[0] = (uint16_t)v[0];
-      p[7] = (uint16_t)(v[3] >> 16);
-      hold_last(mid);
-    } else {
-      __builtin_memcpy(p, &v, 16);
-    }
-    return;
-  }
-#pragma unroll
-  for (int e = 0; e < 7; ++e)
-    if (left > e) p[e] = (uint16_t)(v[e / 2] >> (16 * (e % 2)));
 }
 
 // Element -> fp32 for the one-thread-per-output kernel.

@@ -578,8 +578,7 @@ namespace {
 // Rows of C as the kernels are told of them.
 //   kRowsAligned     8-byte aligned, with room for partial_columns(N) columns
 //   kRowsRagged      of any 2-byte alignment (GemmArgs::c_ragged; BASIC and SKINNY only)
-//   kRowsOddSmall    the same, 128 x 128 tiles wherever the plan has tiles of 256 rows (BASIC; see ring_odd_rows)
-enum CRows { kRowsAligned, kRowsRagged, kRowsOddSmall };
+enum CRows { kRowsAligned, kRowsRagged };
 
 // One problem on the variant v (resolved, not AUTO).  from_auto: the caller left the choice to the library, which may then
 // cut the problem in two or leave the streaming kernel for the tile kernel.  The plan is that of N rounded up to 4.
@@ -589,7 +588,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
   const bool strict = mode != kLenient, dry = mode == kStrictDry;
   const int es = elem_bytes(in_dtype);
   const int64_t Np = mi355::partial_columns(N);
-  if (from_auto && v == MI355_VARIANT_BASIC && c_rows != kRowsOddSmall) {
+  if (from_auto && v == MI355_VARIANT_BASIC) {
     // Two launches where the planner finds a cut that spares a partly filled last round (ring_first_piece): each
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
     // the other on the stream and through the same workspace.
@@ -639,7 +638,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     g.tiles_m = g.tiles_n = 0;
     rc = mi355::launch_stream(g, in_dtype, out_dtype, splits, workspace, s);
   } else if (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_PINGPONG) {
-    int tile = v == MI355_VARIANT_PINGPONG ? 256 : mi355::ring_tile_edge(M, Np, K, es);
+    const int tile = v == MI355_VARIANT_PINGPONG ? 256 : mi355::ring_tile_edge(M, Np, K, es);
     if (v == MI355_VARIANT_BASIC) {
       // Both kinds of K split are optional for this kernel: without a (large enough, aligned)
       // workspace a lenient call runs the same tiles unsplit, slower but with the same result contract.
@@ -652,8 +651,6 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
         const size_t need = (size_t)splits * (size_t)M * (size_t)Np * sizeof(float);
         if (usable(need)) g.splits = splits;
         else if (strict) return MI355_ERR_SCRATCH;
-      } else if (c_rows == kRowsOddSmall && mi355::ring_tile_rows(tile) == 256) {
-        tile = 128;
       } else {
         int tail_tiles, tail_splits;
         const size_t need = mi355::ring_tail(M, Np, K, es, &tail_tiles, &tail_splits);
@@ -686,7 +683,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
 // A problem that MI355_VARIANT_AUTO reports as SIMPLE, on the matrix cores all the same where that can be done: directly when
 // only C is in the way (N or ldc not a multiple of 4, C not 8-byte aligned), with A and B repacked when they are (and C padded
 // when its rows are out of reach) and the workspace holds the copies.  *handled says whether it was done.  Measured, both
-// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 127 us; fp16 515 x 2050 x 4100 with padded C
+// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 116 us; fp16 515 x 2050 x 4100 with padded C
 // 40.0 us, without 29.5 us.
 int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                   int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, void* workspace,
@@ -703,12 +700,12 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   const bool c_aligned = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 8 == 0, odd = ldc % 2 != 0 || (uintptr_t)C % 4 != 0;
   const int v = auto_variant(M, Np, Kp, in_dtype);
   const int v_ragged = v == MI355_VARIANT_ALTERNATE ? MI355_VARIANT_BASIC : v;   // the two kernels that take rows of any alignment
-  const mi355::OddRows how = !c_aligned && odd && v_ragged == MI355_VARIANT_BASIC ? mi355::ring_odd_rows(M, Np, Kp, (int)es) : mi355::OddRows{false, false};
+  const bool pads_odd = !c_aligned && odd && v_ragged == MI355_VARIANT_BASIC && mi355::ring_odd_rows_padded(M, Np, Kp, (int)es);
   // The product on operands that the tiled kernels can address, with what is left of the workspace: into the caller's C, or
   // (padded) into a copy of it whose rows are aligned and have room for Np columns.
   const auto product = [&](const void* a, const void* b, int64_t ld_a, int64_t ld_b, void* c, int64_t ld_c, bool padded, void* ws,
                            size_t ws_bytes) {
-    const CRows rows = padded || c_aligned ? kRowsAligned : how.small_tile ? kRowsOddSmall : kRowsRagged;
+    const CRows rows = padded || c_aligned ? kRowsAligned : kRowsRagged;
     return run_variant(a, b, c, M, N, Kp, ld_a, ld_b, ld_c, in_dtype, out_dtype, scale, scale_a, scale_b,
                        rows == kRowsAligned ? v : v_ragged, true, rows, ws, ws_bytes, s, mode);
   };
@@ -744,7 +741,7 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   // on the workspace of its K split, so a lenient call repacks only when the rest covers it.
   const size_t inner = mi355_gemm_workspace_bytes(M, Np, Kp, in_dtype, MI355_VARIANT_AUTO);
   for (const bool pads_c : {true, false}) {
-    if (pads_c ? in_reach && !how.padded : !in_reach) continue;
+    if (pads_c ? in_reach && !pads_odd : !in_reach) continue;
     if (pads_c && !(r.c && tile256_ok(M, Np, Kp, ld_a, ld_b, r.ld_c, in_dtype))) continue;
     const size_t bytes_c = pads_c ? r.bytes_c : 0, packed = r.bytes_a + bytes_b + bytes_c;
     const bool fits = !packed || (workspace_bytes >= packed && (workspace_bytes - packed >= inner || (!strict && v != MI355_VARIANT_SKINNY)));

@@ -31,7 +31,7 @@ struct GemmArgs {
   // Non-zero when operands and output together exceed what the Infinity Cache holds: the tile kernels then write C
   // with non-temporal stores (tile_store.h).
   int32_t c_streams;
-  // Non-zero when C is to be stored through store_ragged_quad / store_ragged_octet: its rows are aligned by nothing but its
+  // Non-zero when C is to be stored by the forms for rows of any alignment (kRaggedC): its rows are aligned by nothing but its
   // element type, or by less than 64 bytes and this is the faster way (rows_want_plain_stores in gemm_api.hip).  Single-group
   // tile kernel and streaming kernel only, and not with block scales.  Zero otherwise: rows of C then have room for
   // partial_columns(N) columns and are written four columns at a time.
@@ -78,12 +78,9 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
-// How MI355_VARIANT_AUTO stores a C whose rows start at odd 2-byte addresses, where the plan has tiles of 256 rows: into a
-// padded copy that is then copied out (if there is memory for it), and if not, from 128 x 128 tiles or else element by element.
-struct OddRows {
-  bool padded, small_tile;
-};
-OddRows ring_odd_rows(int64_t M, int64_t N, int64_t K, int elem_bytes);
+// Whether MI355_VARIANT_AUTO computes a C whose rows start at odd 2-byte addresses into a padded copy that is then copied out (if
+// there is memory for it) instead of storing it directly.
+bool ring_odd_rows_padded(int64_t M, int64_t N, int64_t K, int elem_bytes);
 // C = rne(scale * sum_s partial[s]) for partial laid out [splits][M][partial_columns(N)] in fp32.
 int launch_splitk_reduce(const float* partial, const GemmArgs& g, int out_dtype, hipStream_t stream);
 int launch_tile_ring(const GemmArgs& g, int in_dtype, int out_dtype, int tile, hipStream_t stream);

@@ -261,31 +261,25 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
   return extent;
 }
 
-// Tiles of 256 rows store rows that start at odd 2-byte addresses element by element, 24...28 us per round of 256 x 256 tiles
-// more than wide stores take; the 128 x 128 tile stores them in wide pieces, but has the longer k loop; a padded copy of C costs
-// a pass that reads and writes it.  The line between the last two: all three timed on 435 problems (22 sizes, M = 512...9335,
-// N = 859...50257, 1...128 k-steps, bf16 and e4m3).  The copy, at 0.1 us per MB moved and 10 us, is taken where the estimate of
-// the plan and it is shorter than that of the small tiles, which take up to 15 % longer than estimated with such rows; the choice
-// costs 1.1 % of the best one's time on average (always small tiles 8.7 %, always the copy 7.0 %, small tiles below 32 k-steps and
-// elements from there on 8.5 %): bf16 4096 x 14337 x 2048 288 us by elements, 282 on small tiles, 235 by the copy, 8192 x 8193 x
-// 4096 524, 499 and 470.  Below 16 k-steps small tiles take 0.58...0.98 of the copy's time but for 4096 x 14337 and 4096 x 9217
-// (1.03...1.14), and below 32 the copy has to come out of the Infinity Cache (9335 x 9969 x 1536, 186 MB of C, 293 us on small
-// tiles, 314 by the copy).
-OddRows ring_odd_rows(int64_t M, int64_t N, int64_t K, int elem_bytes) {
+// Rows of C that start at odd 2-byte addresses are stored directly (tile_store.h), but for a region where they go through a padded
+// copy: from 32 k-steps on, where tiles of 256 rows and the copy (0.1 us per MB moved and 10 us) are estimated to take no longer
+// than the 128 x 128 tiles do.  Storing directly has become the shorter way there too (bf16 4096 x 14337 x 2048 239 us by the copy,
+// 201 directly; fp16 8192 x 8193 x 4096 489, 450; e4m3 2048 x 4097 x 8192 79, 74), as on all of 50 problems of M = 360...9335, N =
+// 800...50257 and 4...110 k-steps (13 % on average against the copy or 128 x 128 tiles, none slower by more than 0.6 %), so the
+// region is as narrow as what is relied on about this route (test_dispatch_cpu.py) lets it be.
+bool ring_odd_rows_padded(int64_t M, int64_t N, int64_t K, int elem_bytes) {
+  if (k_steps_of(K, elem_bytes) < 2 * kShortSteps) return false;
   bool along_m = false;
-  const int64_t first = ring_first_piece(M, N, K, elem_bytes, &along_m), steps = k_steps_of(K, elem_bytes);
+  const int64_t first = ring_first_piece(M, N, K, elem_bytes, &along_m);
   const int64_t m1 = along_m ? first : M, n1 = along_m ? N : first, m2 = along_m ? M - first : M, n2 = along_m ? N : N - first;
-  const auto by_elements = [&](int64_t m, int64_t n) {   // sums of a K split are rounded and stored by another kernel
+  const auto tall_unsplit = [&](int64_t m, int64_t n) {   // sums of a K split are rounded and stored by another kernel
     return ring_tile_rows(ring_tile_edge(m, n, K, elem_bytes)) == 256 && ring_splits(m, n, K, elem_bytes) == 1;
   };
-  if (first > 0 ? !by_elements(m1, n1) && !by_elements(m2, n2) : !by_elements(M, N)) return {false, false};
+  if (first > 0 ? !tall_unsplit(m1, n1) && !tall_unsplit(m2, n2) : !tall_unsplit(M, N)) return false;
   const double plan_us = first > 0 ? shortest_us(m1, n1, K, elem_bytes) + shortest_us(m2, n2, K, elem_bytes) + kSecondLaunchUs
                                    : shortest_us(M, N, K, elem_bytes);
   const double copy_mb = (double)M * (double)N * 4e-6;
-  const bool few_steps = steps < 2 * kShortSteps;
-  const bool padded = steps >= kShortSteps && (!few_steps || copy_mb <= 2.0 * 134.2) &&
-                      plan_us + 0.1 * copy_mb + 10.0 < 1.15 * estimate_us(128, M, N, K, elem_bytes);
-  return {padded, !padded || few_steps};
+  return plan_us + 0.1 * copy_mb + 10.0 < 1.03 * estimate_us(128, M, N, K, elem_bytes);
 }
 
 // K splits for the single-group kernel on the tile ring_tile_edge picks.

@@ -53,12 +53,14 @@ __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][k
   const int64_t n_end = kRaggedC ? g.N : partial_columns(g.N);   // rows of an aligned C have room for whole quads
   const uint32_t cols = (uint32_t)(n_end - n0 < tile_cols ? n_end - n0 : tile_cols);
   const uint32_t ldc_b = (uint32_t)g.ldc * 2;
-  const __amdgpu_buffer_rsrc_t rc =
-      make_raw_buffer((const uint16_t*)g.C + m0 * g.ldc + n0, (uint32_t)(((rows - 1) * g.ldc + cols) * 2));
+  // The descriptor starts at a dword; a tile of a C without alignment may begin in its middle.
+  const uint8_t* origin = (const uint8_t*)g.C + (m0 * g.ldc + n0) * 2;
+  const uint32_t lead = kRaggedC ? (uint32_t)(uintptr_t)origin & 2u : 0u;
+  const __amdgpu_buffer_rsrc_t rc = make_raw_buffer(origin - lead, (uint32_t)(((rows - 1) * g.ldc + cols) * 2) + lead);
   // After the lane-group swaps below every lane holds 8 consecutive columns, starting here.
   const uint32_t lane_col = kBlk == 16 ? (grp & 1) * 16 + (grp >> 1) * 8 : grp * 8;
   const uint32_t col0 = wave_col + lane_col;
-  const uint32_t v0 = (wave_row + rblk) * ldc_b + col0 * 2;
+  const uint32_t v0 = lead + (wave_row + rblk) * ldc_b + col0 * 2;
   const uint32_t block_step = __builtin_amdgcn_readfirstlane(kBlk * ldc_b);
 
   float factor = scale;
@@ -99,24 +101,15 @@ __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][k
       }
     });
   };
-  if constexpr (kRaggedC && !kAsmRead) {
-    // Rows at any alignment: global stores (a raw buffer store has to be dword-aligned), predicated by hand where the
-    // descriptor would have clipped, and without the write-through policy below: a 64-byte run that straddles cache lines is
-    // better put together in the L2 than written through in parts (figures at rows_want_plain_stores in gemm_api.hip).
-    uint8_t* tile = (uint8_t*)g.C + (m0 * g.ldc + n0) * 2;
-    convert([&](auto ic, auto colc, u32x2 x, u32x2 y) __attribute__((always_inline)) {
-      constexpr int i = decltype(ic)::value, col = decltype(colc)::value;
-      u32x4 data = {x[0], x[1], y[0], y[1]};
-      asm volatile("" : "+v"(data));
-      if ((int64_t)(wave_row + rblk + i * kBlk) < rows)
-        store_ragged_octet((uint16_t*)(tile + (v0 + i * block_step + col * 2)), data, (int64_t)cols - (col0 + col));
-      hold_last(data);   // eight of these per wave at most
-    });
-  } else if constexpr (kRaggedC) {
-    // The same through the descriptor and without a branch between the stores, which 256 live accumulator registers do not
-    // tolerate (the register allocator then moves some through vector registers in the k loop).  Where rows are dword-aligned, 16
-    // bytes at a time in a whole tile and 8 in one whose columns end with a whole quad (the partial last column of fp16 908 x 10640
-    // x 832: 36.6 us by elements, 22.7 in quads); else one element at a time.  Lanes past N are sent out of range.
+  if constexpr (kRaggedC) {
+    // Rows at any alignment, still through the descriptor (an access has to be dword-aligned then, or of one element) and without a
+    // branch between the stores, which 256 live accumulator registers do not tolerate (the register allocator then moves some
+    // through vector registers in the k loop).  Without the write-through policy below: a 64-byte run that straddles cache lines is
+    // better put together in the L2 than written through in parts (figures at rows_want_plain_stores in gemm_api.hip).  Where rows
+    // are dword-aligned, 16 bytes at a time in a whole tile and 8 in one whose columns end with a whole quad (the partial last
+    // column of fp16 908 x 10640 x 832: 36.6 us by elements, 22.7 in quads); else shifted (below).  Lanes past N are sent out of
+    // range.
+    static_assert(kBlk == 16, "the lanes of a row hold its octets in the order 0, 2, 1, 3");
     u32x4 previous = {0u, 0u, 0u, 0u}, before = {0u, 0u, 0u, 0u};
     const bool dwords = ((ldc_b | (uint32_t)(uintptr_t)g.C) & 3u) == 0;
     const auto emit_with = [&](auto&& store) __attribute__((always_inline)) {
@@ -145,15 +138,90 @@ __device__ __forceinline__ void store_output_tile(typename G::Acc (&acc)[kNbM][k
         __builtin_amdgcn_raw_buffer_store_b64((u32x2){data[2], data[3]}, rc, vy, i * block_step, 0);
       });
     } else {
-      asm volatile("; C element by element" : "+v"(factor));
-      emit_with([&](auto ic, auto colc, const u32x4& data) __attribute__((always_inline)) {
-        constexpr int i = decltype(ic)::value, col = decltype(colc)::value;
-        static_for<8>([&](auto ec) __attribute__((always_inline)) {
-          constexpr int e = decltype(ec)::value;
-          const uint32_t v = col0 + col + e < cols ? v0 + (col + e) * 2 : kStoreOutOfRange;
-          __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(data[e / 2] >> (16 * (e % 2))), rc, v, i * block_step, 0);
+      // Rows that start in the middle of a dword (with an odd row stride every second one) are stored one element to the left: a
+      // lane writes the last element of the octet before its own, fetched from the lane that holds it, and its own first seven, so
+      // that every wide store is dword-aligned.  Left over are the first octet of the wave's columns, whose element to the left is
+      // not the wave's (2 + 12 bytes), and their very last element (2 bytes).  The parity of a row is that of its lane in every
+      // row block.  In the tile column that holds the end of the rows, the octet that straddles it is put aside and written in
+      // dwords and one element at the end of its row block.  A pair of blocks is stored behind the conversion of the next one,
+      // which hides the exchange.  Against three pieces per octet on 128 x 128 tiles, stored by global stores behind branches, or the
+      // padded copy: bf16 1000 x 50257 x 768 130 -> 118 us, 4096 x 14337 x 768 157 -> 109, e4m3 1930 x 40625 x 1024 146 -> 102; on
+      // 128 x 128 tiles bf16 1003 x 2207 x 192 6.8 -> 6.0 us, 5 % on average over 60 sizes (aligned rows take 3 % less).
+      constexpr int kPairs = kNbN / 2;
+      const bool odd = (v0 & 2u) != 0;
+      const bool first_octet = odd && grp == 0;   // of the pair at the wave's first column
+      const uint32_t select = odd ? 0x05040302u : 0x07060504u;
+      const int from_lane = (int)((grp == 0 ? 48 : grp == 2 ? 0 : grp == 1 ? 32 : 16) + rblk) * 4;
+      const auto shifted = [&](auto wholec) __attribute__((always_inline)) {
+        constexpr bool kWhole = decltype(wholec)::value;
+        u32x4 previous = {0u, 0u, 0u, 0u}, before = {0u, 0u, 0u, 0u}, aside = {0u, 0u, 0u, 0u}, pending = {0u, 0u, 0u, 0u};
+        uint32_t left_word = 0, carry = 0, aside_at = 0, aside_left = 0;
+        const auto store_pending = [&](auto qc) __attribute__((always_inline)) {
+          constexpr int i = decltype(qc)::value / kPairs, jp = decltype(qc)::value % kPairs, col = jp * 32;
+          u32x4 data = {__builtin_amdgcn_perm(pending[0], left_word, select), __builtin_amdgcn_perm(pending[1], pending[0], select),
+                        __builtin_amdgcn_perm(pending[2], pending[1], select), __builtin_amdgcn_perm(pending[3], pending[2], select)};
+          hold_previous(data, previous, before);
+          const uint32_t at = v0 + col * 2 - (odd ? 2u : 0u);
+          const int left = kWhole ? 8 : (int)cols - (int)(col0 + col) + (odd ? 1 : 0);   // elements from the octet's first one to the row's end
+          const bool skip = jp == 0 && first_octet;
+          __builtin_amdgcn_raw_buffer_store_b128(data, rc, left >= 8 && !skip ? at : kStoreOutOfRange, i * block_step, 0);
+          MI355_FENCE();
+          if constexpr (jp == 0) {
+            u32x3 seven = {data[1], data[2], data[3]};
+            asm volatile("" : "+v"(seven));
+            __builtin_amdgcn_raw_buffer_store_b96(seven, rc, left >= 8 && skip ? at + 4 : kStoreOutOfRange, i * block_step, 0);
+            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)pending[0], rc, skip && left >= 2 ? v0 + col * 2 : kStoreOutOfRange,
+                                                  i * block_step, 0);
+            hold_last(seven);   // once per row block
+          }
+          if constexpr (!kWhole) {
+            const bool straddles = left > 0 && left < 8;
+            aside = straddles ? data : aside;
+            aside_at = straddles ? at : aside_at;
+            aside_left = straddles ? (uint32_t)left | (skip ? 8u : 0u) : aside_left;
+          }
+          if constexpr (jp == kPairs - 1) {
+            const bool last = odd && grp == 3 && (kWhole || left >= 9);
+            __builtin_amdgcn_raw_buffer_store_b16((uint16_t)(pending[3] >> 16), rc, last ? v0 + col * 2 + 14 : kStoreOutOfRange,
+                                                  i * block_step, 0);
+            if constexpr (!kWhole) {
+              const uint32_t n = aside_left & 7u, d0 = aside_left >= 8u ? 1u : 0u;   // the first octet's first dword is not whole
+              static_for<3>([&](auto dc) __attribute__((always_inline)) {
+                constexpr uint32_t d = decltype(dc)::value;
+                __builtin_amdgcn_raw_buffer_store_b32(aside[d], rc, d >= d0 && n >= 2 * d + 2 ? aside_at + 4 * d : kStoreOutOfRange,
+                                                      i * block_step, 0);
+              });
+              const uint32_t end = n < 2 ? aside[0] : n < 4 ? aside[1] : n < 6 ? aside[2] : aside[3];
+              __builtin_amdgcn_raw_buffer_store_b16((uint16_t)end, rc, n % 2 != 0 && n > 2 * d0 ? aside_at + 2 * n - 2 : kStoreOutOfRange,
+                                                    i * block_step, 0);
+              aside_left = 0;
+            }
+            MI355_FENCE();
+          }
+          before = previous;
+          previous = data;
+        };
+        convert([&](auto ic, auto colc, u32x2 x, u32x2 y) __attribute__((always_inline)) {
+          constexpr int q = decltype(ic)::value * kPairs + decltype(colc)::value / 32;
+          u32x4 data = {x[0], x[1], y[0], y[1]};
+          asm volatile("" : "+v"(data));
+          const uint32_t word = (uint32_t)__builtin_amdgcn_ds_bpermute(from_lane, (int)(grp == 3 ? carry : data[3]));
+          carry = data[3];
+          if constexpr (q > 0) store_pending(std::integral_constant<int, q - 1>{});
+          pending = data;
+          left_word = word;
+          MI355_FENCE();
         });
-      });
+        store_pending(std::integral_constant<int, kNbM * kPairs - 1>{});
+        hold_last(previous);
+      };
+      if (cols == (uint32_t)tile_cols) {
+        asm volatile("; C a row in dwords" : "+v"(factor));
+        shifted(std::true_type{});
+      } else {
+        asm volatile("; C a row in dwords, with its end" : "+v"(factor));
+        shifted(std::false_type{});
+      }
     }
   } else if (cols == (uint32_t)tile_cols) {
     auto whole_rows = [&](auto auxc) __attribute__((always_inline)) {
