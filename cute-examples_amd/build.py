@@ -20,7 +20,7 @@ OUT = os.path.join(HERE, "gemm_kernels")
 LIB = os.path.join(OUT, "libmi355gemm.so")
 LIB_SYNC_SCALES = os.path.join(OUT, "libmi355gemm_syncscales.so")
 
-HIP_SOURCES = ["gemm_api.hip", "gemm_tn_simple.hip", "gemm_tn_small.hip", "gemm_tn_ring_bf16.hip", "gemm_tn_ring_f16.hip", "gemm_tn_ring_e4m3.hip", "gemm_tn_ring_mx.hip",
+HIP_SOURCES = ["gemm_api.hip", "gemm_tn_simple.hip", "gemm_tn_small.hip", "gemm_tn_slices.hip", "gemm_tn_ring_bf16.hip", "gemm_tn_ring_f16.hip", "gemm_tn_ring_e4m3.hip", "gemm_tn_ring_mx.hip",
                "gemm_tn_ring_bf16_ragged.hip", "gemm_tn_ring_f16_ragged.hip", "gemm_tn_ring_e4m3_ragged.hip", "ring_plan.hip", "gemm_tn_pingpong.hip", "gemm_tn_alternate.hip", "gemm_tn_stream.hip", "quantize_e4m3.hip", "mx_scales.hip", "calibrate.hip"]
 
 # Sources whose device assembly is verified after compilation (check_async_loads.py): the copies'
@@ -30,7 +30,7 @@ CHECKED_SOURCES = ["gemm_tn_ring_bf16.hip", "gemm_tn_ring_f16.hip", "gemm_tn_rin
 CHECKED_SOURCE = "gemm_tn_ring_mx.hip"
 # Sources whose kernels must keep the hardware's distances the compiler does not enforce (wide
 # stores and their data registers, inline-assembly MFMAs and their results): every GEMM kernel.
-HAZARD_SOURCES = CHECKED_SOURCES + ["gemm_tn_pingpong.hip", "gemm_tn_alternate.hip", "gemm_tn_stream.hip", "calibrate.hip"]
+HAZARD_SOURCES = CHECKED_SOURCES + ["gemm_tn_pingpong.hip", "gemm_tn_alternate.hip", "gemm_tn_stream.hip", "gemm_tn_slices.hip", "calibrate.hip"]
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",

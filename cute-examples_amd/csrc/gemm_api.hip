@@ -93,6 +93,25 @@ int32_t c_streams(int64_t M, int64_t N, int64_t K, int elem_bytes) {
 bool rows_want_plain_stores(const void* C, int64_t M, int64_t N, int64_t ldc) {
   return ((ldc * 2) % 64 != 0 || (uintptr_t)C % 64 != 0) && M * N >= ((int64_t)4 << 20);
 }
+// The form of the kernel for products of few outputs that MI355_VARIANT_AUTO takes instead of the streaming kernel (streams) or the
+// tile kernel, -1 for none (slices_config).  N: rounded up to 4.
+int few_outputs(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, bool streams) {
+  if ((double)M * (double)N * (double)K > mi355::kSlicesMaxProducts) return -1;
+  mi355::SlicesAlternative other;
+  other.streams = streams;
+  if (streams) {
+    other.tile_cols = mi355::stream_tile_cols(M, N, K, elem_bytes, mx);
+    other.tile_rows = M <= 16 ? 16 : M <= 32 ? 32 : M <= 64 ? 64 : M <= 128 ? 128 : 256;
+    if (other.tile_cols == 128) other.tile_rows = 64;
+    other.splits = mi355::stream_splits(M, N, K, elem_bytes, mx);
+  } else {
+    const int tile = mi355::ring_tile_edge(M, N, K, elem_bytes, mx);
+    other.tile_rows = mi355::ring_tile_rows(tile);
+    other.tile_cols = mi355::ring_tile_cols(tile);
+    other.splits = mi355::ring_splits(M, N, K, elem_bytes, mx);
+  }
+  return mi355::slices_config(M, N, K, elem_bytes, mx, other);
+}
 bool skinny_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int in_dtype) {
   if (M > 256) return false;
   return tile256_ok(M, N, K, lda, ldb, ldc, in_dtype);
@@ -496,6 +515,12 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
     g.mx_b = wb;
     used = bytes_a + bytes_b;
   }
+  // A product of few outputs, as for plain operands.
+  const int config = few_outputs(M, N, K, 1, true, M <= kSkinnyAutoMaxM);
+  if (config >= 0) {
+    g.tiles_m = g.tiles_n = 0;
+    return mi355::launch_slices(g, MI355_E4M3, out_dtype, config, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
+  }
   // A few rows of activations: stream the weights, as for plain fp8 (when the workspace holds the
   // partial results of its K split, if it has one; otherwise the tile kernel below takes it).
   if (const int ss = mx_stream_splits(M, N, K, lda, ldb, ldc)) {
@@ -588,7 +613,8 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
   const bool strict = mode != kLenient, dry = mode == kStrictDry;
   const int es = elem_bytes(in_dtype);
   const int64_t Np = mi355::partial_columns(N);
-  if (from_auto && v == MI355_VARIANT_BASIC) {
+  const int config = from_auto && (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_SKINNY) ? few_outputs(M, Np, K, es, false, v == MI355_VARIANT_SKINNY) : -1;
+  if (config < 0 && from_auto && v == MI355_VARIANT_BASIC) {
     // Two launches where the planner finds a cut that spares a partly filled last round (ring_first_piece): each
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
     // the other on the stream and through the same workspace.
@@ -625,6 +651,11 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
   // so it matches what mi355_gemm_workspace_bytes reported.  Its K split needs the workspace: an
   // explicit MI355_VARIANT_SKINNY without it is an error, MI355_VARIANT_AUTO goes to the tile
   // kernel instead, whose split is optional.
+  if (config >= 0) {   // no workspace needed
+    if (dry) return MI355_OK;
+    g.tiles_m = g.tiles_n = 0;
+    return mi355::launch_slices(g, in_dtype, out_dtype, config, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
+  }
   const int stream_s = v == MI355_VARIANT_SKINNY ? mi355::stream_splits(M, Np, K, es) : 1;
   const size_t stream_need = stream_s > 1 ? (size_t)stream_s * (size_t)M * (size_t)Np * sizeof(float) : 0;
   if (stream_need && (!workspace || workspace_bytes < stream_need || (uintptr_t)workspace % 16 != 0)) {

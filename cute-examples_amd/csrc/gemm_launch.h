@@ -110,6 +110,15 @@ int stream_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx = fal
 int stream_tile_cols(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx = false);  // rows of W per workgroup: 64 or 128
 int launch_stream_mx(const GemmArgs& g, int out_dtype, int splits, void* workspace, hipStream_t stream);
 int launch_stream(const GemmArgs& g, int in_dtype, int out_dtype, int splits, void* workspace, hipStream_t stream);
+// Products of few outputs (gemm_tn_slices.hip).  slices_config: the form of that kernel MI355_VARIANT_AUTO takes instead of the
+// route described by `other`, or -1 to stay on that; a pure host heuristic.  Needs no workspace.
+struct SlicesAlternative {
+  bool streams;   // the streaming kernel, else the single-group tile kernel
+  int64_t tile_rows, tile_cols, splits;
+};
+constexpr double kSlicesMaxProducts = 1.5e10;   // M * N * K; the rule was fitted below
+int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other);
+int launch_slices(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);
 // Per-tensor e4m3 quantisation (amax -> scale -> cast); scale_amax points to two floats.  partial: scratch memory of
 // `partials` floats, or null; quantize_e4m3_partials(n) is how many the quantiser would like.
 int64_t quantize_e4m3_partials(int64_t n);

@@ -79,6 +79,10 @@ enum mi355_status {
  *             by the tiled kernels directly, or computed in a padded copy of it that the workspace
  *             holds and copied out, whichever is shorter (mi355_gemm_select_variant still reports
  *             SIMPLE)
+ *             A product of few outputs that MI355_VARIANT_AUTO would stream or tile runs on a kernel
+ *             for those instead where that is estimated to be faster, without a workspace
+ *             (mi355_gemm_select_variant, mi355_gemm_plan and the workspace query still report the
+ *             variant whose place it takes)
  *   stream    hipStream_t on which the kernels are enqueued (NULL = the null stream)
  *
  * Replaces test::gemm_tn_test (kernels/gemm_kernels/sm90a/gemm_test.cu:12-92): same operand
@@ -184,6 +188,7 @@ int mi355_quantize_e4m3_scratch(const void *x, int x_dtype, int64_t n, void *x_q
  *                      tiled kernel instead of the weight-streaming one).
  * Constraints: K % 128 == 0; A, B 16-byte aligned with row strides that are multiples of 16;
  * N % 4 == 0, ldc % 4 == 0, C 8-byte aligned; the size limits of the tiled variants.  Runs the
+ * kernel for products of few outputs where mi355_gemm_tn would (MI355_VARIANT_AUTO), else the
  * weight-streaming kernel (MI355_VARIANT_SKINNY) for M <= 64 and otherwise the tiled kernel
  * (MI355_VARIANT_BASIC) with the planner's choice of tile and splits among the tiles this kernel
  * has: what mi355_gemm_plan reports for MI355_E4M3 operands of this shape and that variant,

@@ -1,0 +1,46 @@
+"""Which problems go to the kernel for products of few outputs, and with which form of it: what a call launches, on the CPU."""
+import re
+
+import pytest
+
+from tests import abi_ctypes as ac
+from tests.few_outputs_cases import PLAIN
+from tests.test_dispatch_cpu import C, case, launches  # noqa: F401  (fixture)
+
+
+def form(name):
+    m = re.search(r"gemm_tn_slices\w*?Li(\d)ELi(\d)ELi(\d)ELb(\d)E", name)
+    return m and tuple(int(x) for x in m.groups())
+
+
+def test_every_form_is_among_the_cases(launches):  # noqa: F811
+    got = [form(got[0][0]) for _, _, got in launches([case(*c) for c in PLAIN])]
+    assert {f[:3] for f in got if f} == {(1, 1, 4), (1, 1, 8), (1, 2, 4), (2, 2, 2), (2, 2, 4), (2, 4, 4), (4, 4, 4)}
+    assert sum(f is not None for f in got) >= 0.9 * len(PLAIN)
+
+
+def test_one_launch_without_a_workspace_and_with_it(launches):  # noqa: F811
+    for room in (0, None):
+        for noalloc in (False, True):
+            for c, (st, _, got) in zip(PLAIN, launches([case(*c, room=room, noalloc=noalloc) for c in PLAIN])):
+                if form(got[0][0]):
+                    assert st == ac.OK and len(got) == 1 and not form(got[0][0])[3], c
+
+
+@pytest.mark.parametrize("in_dt", [ac.BF16, ac.E4M3])
+def test_rows_of_c_of_any_alignment_have_a_form_of_their_own(launches, in_dt):  # noqa: F811
+    for c, (st, _, got) in zip(PLAIN, launches([case(*c[:3], in_dt, ldc=c[1] + 1, c=C + 2, room=1 << 26) for c in PLAIN])):
+        assert st == ac.OK
+        f = form(got[0][0])
+        assert f is None or f[3] == 1, c
+
+
+@pytest.mark.parametrize("variant", [ac.BASIC, ac.SKINNY, ac.PINGPONG, ac.SIMPLE])
+def test_explicit_variants_stay_on_their_kernels(launches, variant):  # noqa: F811
+    cases = [case(*c, variant=variant) for c in PLAIN if variant != ac.SKINNY or c[0] <= 256]
+    assert all(form(name) is None for _, _, got in launches(cases) for name, _ in got)
+
+
+def test_large_products_stay_where_they_were(launches):  # noqa: F811
+    large = [(16, 14336, 4096), (64, 4096, 14336), (256, 4096, 4096), (2048, 2048, 2048), (17, 4100, 4096), (512, 6144, 4096), (8192, 128, 4096)]
+    assert all(form(name) is None for _, _, got in launches([case(*c) for c in large]) for name, _ in got)
