@@ -93,10 +93,8 @@ int32_t c_streams(int64_t M, int64_t N, int64_t K, int elem_bytes) {
 bool rows_want_plain_stores(const void* C, int64_t M, int64_t N, int64_t ldc) {
   return ((ldc * 2) % 64 != 0 || (uintptr_t)C % 64 != 0) && M * N >= ((int64_t)4 << 20);
 }
-// The form of the kernel for products of few outputs that MI355_VARIANT_AUTO takes instead of the streaming kernel (streams) or the
-// tile kernel, -1 for none (slices_config).  N: rounded up to 4.
-int few_outputs(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, bool streams) {
-  if ((double)M * (double)N * (double)K > mi355::kSlicesMaxProducts) return -1;
+// Where the kernel for products of few outputs stands aside: the streaming kernel (streams) or the tile kernel.
+mi355::SlicesAlternative alternative_to_slices(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, bool streams) {
   mi355::SlicesAlternative other;
   other.streams = streams;
   if (streams) {
@@ -110,7 +108,12 @@ int few_outputs(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, bool s
     other.tile_cols = mi355::ring_tile_cols(tile);
     other.splits = mi355::ring_splits(M, N, K, elem_bytes, mx);
   }
-  return mi355::slices_config(M, N, K, elem_bytes, mx, other);
+  return other;
+}
+// The form of that kernel that MI355_VARIANT_AUTO takes, -1 for none.  N: rounded up to 4.
+int few_outputs(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, bool streams) {
+  if ((double)M * (double)N * (double)K > mi355::kSlicesMaxProducts) return -1;
+  return mi355::slices_config(M, N, K, elem_bytes, mx, alternative_to_slices(M, N, K, elem_bytes, mx, streams));
 }
 bool skinny_ok(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int in_dtype) {
   if (M > 256) return false;
@@ -170,8 +173,8 @@ struct Repack {
 size_t round_up(size_t x, size_t to) { return (x + to - 1) / to * to; }
 
 constexpr double kRepackMinFlops = 134217728.0;   // below, repacking is not worth its launches
-// From here on a small problem with unaligned operands, or an e4m3 one with any unaligned rows, runs on gemm_tn_small instead of
-// the generic kernel.  Both timed at M = 1...2048 and 1 to 67 million products: K = 65 small 0.5-1.0 of the generic kernel's
+// From here on a small e4m3 problem with any unaligned rows (or a 16-bit one whose rows are out of the reach of gemm_tn_slices) runs
+// on gemm_tn_small instead of the generic kernel.  Both timed at M = 1...2048 and 1 to 67 million products: K = 65 small 0.5-1.0 of the generic kernel's
 // speed, K = 129 1.0-1.7, 257 2.0-3.5, 513 3.9-7.7, 1025 7-16 times (bf16 16 x 4025 x 1025 128 -> 13 us), 14335 51-157 times
 // (bf16 16 x 287 x 14335 1808 -> 33 us).
 constexpr int64_t kSmallMinK = 128;
@@ -713,9 +716,10 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
 
 // A problem that MI355_VARIANT_AUTO reports as SIMPLE, on the matrix cores all the same where that can be done: directly when
 // only C is in the way (N or ldc not a multiple of 4, C not 8-byte aligned), with A and B repacked when they are (and C padded
-// when its rows are out of reach) and the workspace holds the copies.  *handled says whether it was done.  Measured, both
-// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 116 us; fp16 515 x 2050 x 4100 with padded C
-// 40.0 us, without 29.5 us.
+// when its rows are out of reach) and the workspace holds the copies; few outputs on gemm_tn_slices as they are, where the workspace
+// would hold the copies or none are made.  *handled says whether it was done.  Measured, both
+// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 116 us; fp16 515 x 2050 x 4100 repacked
+// 30 us (37 on another box), as it is 26.
 int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                   int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, void* workspace,
                   size_t workspace_bytes, hipStream_t s, WorkspaceMode mode, bool* handled) {
@@ -749,17 +753,38 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
     *handled = true;
     return product(A, B, lda, ldb, C, ldc, false, workspace, workspace_bytes);
   }
-  if (!large && K >= kSmallMinK && (uintptr_t)A % es == 0 && (uintptr_t)B % es == 0 && 2.0 * (double)M * (double)N * (double)K < kRepackMinFlops) {
+  // Products of few outputs on rows of any alignment, as they are: small 16-bit ones (bf16 112 x 154 x 3092 13.5 us on gemm_tn_small,
+  // 5.9 here; 9 x 234 x 2291 12.0, 4.7), and larger ones of either size of element that would be copied (below).
+  const bool elements_aligned = (uintptr_t)A % es == 0 && (uintptr_t)B % es == 0;
+  mi355::GemmArgs as_is = {};
+  as_is.A = A; as_is.B = B; as_is.C = C;
+  as_is.M = M; as_is.N = N; as_is.K = K;
+  as_is.lda = lda; as_is.ldb = ldb; as_is.ldc = ldc;
+  as_is.scale = scale;
+  as_is.scale_a = scale_a;
+  as_is.scale_b = scale_b;
+  const auto on_slices = [&](int form) {
+    if (mode == kStrictDry) return (int)MI355_OK;
+    return mi355::launch_slices_any_rows(as_is, in_dtype, out_dtype, form, s) == 0 ? (int)MI355_OK : (int)MI355_ERR_LAUNCH;
+  };
+  const auto slices_form = [&](int64_t copied) {
+    if (!elements_aligned || (double)M * (double)N * (double)K > mi355::kSlicesMaxProductsAnyRows) return -1;
+    if (256 * lda * es >= (int64_t)1 << 31 || 256 * ldb * es >= (int64_t)1 << 31) return -1;   // as tile256_ok
+    const uintptr_t bits = (uintptr_t)A | (uintptr_t)B | (uintptr_t)(lda * es) | (uintptr_t)(ldb * es);
+    return mi355::slices_any_rows_config(M, N, K, (int)es, (int)(bits & (~bits + 1) & 255), copied,
+                                         copied ? alternative_to_slices(M, Np, Kp, (int)es, false, v == MI355_VARIANT_SKINNY) : mi355::SlicesAlternative{});
+  };
+  if (!large && in_dtype != MI355_E4M3) {
+    const int form = slices_form(0);
+    if (form >= 0) {
+      *handled = true;
+      return on_slices(form);
+    }
+  }
+  if (!large && K >= kSmallMinK && elements_aligned && 2.0 * (double)M * (double)N * (double)K < kRepackMinFlops) {
     *handled = true;
     if (mode == kStrictDry) return MI355_OK;
-    mi355::GemmArgs g = {};
-    g.A = A; g.B = B; g.C = C;
-    g.M = M; g.N = N; g.K = K;
-    g.lda = lda; g.ldb = ldb; g.ldc = ldc;
-    g.scale = scale;
-    g.scale_a = scale_a;
-    g.scale_b = scale_b;
-    return mi355::launch_small(g, in_dtype, out_dtype, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
+    return mi355::launch_small(as_is, in_dtype, out_dtype, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
   }
   if (!large) return MI355_OK;
   // N alone is no reason to copy B (rows past N read as zeros), a row stride beyond the tiled kernels' 32-bit offsets is; what
@@ -779,6 +804,10 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
     *handled = *handled || strict;   // refused unless one of them fits
     if (!fits) continue;
     *handled = true;
+    if (r.a || copies_b) {
+      const int form = slices_form((r.a ? M * K * es : 0) + (copies_b ? N * K * es : 0));
+      if (form >= 0) return on_slices(form);
+    }
     if (packed && mode == kStrictDry) return MI355_OK;
     uint8_t* wa = (uint8_t*)workspace;
     uint8_t* wb = wa + r.bytes_a;

@@ -78,6 +78,7 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
+double ring_shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // estimate of the single-group kernel's plan
 // Whether MI355_VARIANT_AUTO computes a C whose rows start at odd 2-byte addresses into a padded copy that is then copied out (if
 // there is memory for it) instead of storing it directly.
 bool ring_odd_rows_padded(int64_t M, int64_t N, int64_t K, int elem_bytes);
@@ -111,14 +112,18 @@ int stream_tile_cols(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx = 
 int launch_stream_mx(const GemmArgs& g, int out_dtype, int splits, void* workspace, hipStream_t stream);
 int launch_stream(const GemmArgs& g, int in_dtype, int out_dtype, int splits, void* workspace, hipStream_t stream);
 // Products of few outputs (gemm_tn_slices.hip).  slices_config: the form of that kernel MI355_VARIANT_AUTO takes instead of the
-// route described by `other`, or -1 to stay on that; a pure host heuristic.  Needs no workspace.
+// route described by `other`, or -1 to stay on that, and the estimate of the choice (route_us, may be null); a pure host heuristic.
+// Needs no workspace.  The any_rows pair is for rows of A and B that are aligned by `alignment` bytes only, where the other route
+// copies `copied` bytes to aligned rows first (0: a small 16-bit product, which is not copied).
 struct SlicesAlternative {
   bool streams;   // the streaming kernel, else the single-group tile kernel
   int64_t tile_rows, tile_cols, splits;
 };
-constexpr double kSlicesMaxProducts = 1.5e10;   // M * N * K; the rule was fitted below
-int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other);
+constexpr double kSlicesMaxProducts = 1.5e10, kSlicesMaxProductsAnyRows = 3e10;   // M * N * K; the rules were fitted below
+int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other, double* route_us = nullptr);
 int launch_slices(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);
+int slices_any_rows_config(int64_t M, int64_t N, int64_t K, int elem_bytes, int alignment, int64_t copied, const SlicesAlternative& other);
+int launch_slices_any_rows(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);
 // Per-tensor e4m3 quantisation (amax -> scale -> cast); scale_amax points to two floats.  partial: scratch memory of
 // `partials` floats, or null; quantize_e4m3_partials(n) is how many the quantiser would like.
 int64_t quantize_e4m3_partials(int64_t n);

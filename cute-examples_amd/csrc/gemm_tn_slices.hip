@@ -14,7 +14,9 @@
 // 2048 7.0 -> 4.3 us, 66 x 2064 x 768 9.8 -> 4.2, 579 x 208 x 2304 14.4 -> 6.2, e4m3 55 x 2144 x 6144 10.3 -> 7.2, MXFP8 368 x 224 x 2816
 // 13.8 -> 5.1, bf16 53 x 1120 x 8448 11.6 -> 13.4 (not taken); calls back to back, fp16 512^3 6.1 -> 4.3, an fp8 layer of 16 x 6144 x
 // 4096 with its quantiser 13.6 -> 11.0.  Over 800 problems of M = 1...5800, N = 128...46000, K = 128...14000 the rule of slices_config leaves
-// 0.70 of the time before on average, as the better choice on each of them would.
+// 0.70 of the time before on average, as the better choice on each of them would.  Rows of any alignment (kAnyRows) spare such products
+// the repacking, or the kernel that computes 4 x 4 outputs per wave: bf16 10 x 10028 x 12846 146 -> 70 us, 112 x 154 x 3092 13.5 -> 5.9,
+// fp16 515 x 2050 x 4100 30 -> 26; what bounds them is the same intake, at 50-80 KB per us since most pieces of rows straddle lines.
 //
 // Counterpart in the reference: none (its launcher rejects shapes that are not multiples of its tile,
 // kernels/gemm_kernels/sm90a/gemm_test.cu:33-41); the arithmetic is gemm.cuh:352-377: fp32 accumulation, one rounding.
@@ -36,7 +38,10 @@ constexpr int kDepth = 2;           // stages of a wave's ring
 constexpr uint32_t kMxUnit = 512;   // block scales: bytes of one (128 rows, k-step) unit, see gemm_tn_stream.hip
 
 // kMB x kNB blocks of 16 x 16 outputs per workgroup.  kRaggedC: rows of C at any 2-byte alignment (g.c_ragged).
-template <class T, class OutT, int kMB, int kNB, int kWaves, bool kRaggedC>
+// kAnyRows: rows of A and B at any alignment of their elements.  They cannot be copied straight into LDS then, and go through
+// registers instead: global loads of 16 bytes need no alignment on this target, and a wave's accesses to LDS keep their order, so
+// that one stage does.  A row has at least 16 bytes (host check).
+template <class T, class OutT, int kMB, int kNB, int kWaves, bool kRaggedC, bool kAnyRows>
 __global__ __launch_bounds__(64 * kWaves) void gemm_tn_slices(GemmArgs g) {
   typedef typename SliceGeo<T>::type G;
   typedef typename G::Frag Frag;
@@ -49,7 +54,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_tn_slices(GemmArgs g) {
   constexpr int kStageBytes = kDataBytes + (kMx ? 512 : 0);
   constexpr int kCopies = (kTm + kTn) / 8;
   constexpr int kVm = kCopies + (kMx ? 2 : 0);
-  constexpr int kRingBytes = kWaves * kDepth * kStageBytes, kSumBytes = kWaves * kMB * kNB * 1024;
+  constexpr int kStages = kAnyRows ? 1 : kDepth;
+  constexpr int kRingBytes = kWaves * kStages * kStageBytes, kSumBytes = kWaves * kMB * kNB * 1024;
   static_assert(kVm * (kDepth - 1) < 64, "vmcnt is a 6-bit counter");
   static_assert(kRingBytes <= 160 * 1024 && kSumBytes <= 160 * 1024, "LDS of a CU");
   __shared__ __attribute__((aligned(1024))) uint8_t ring[kRingBytes > kSumBytes ? kRingBytes : kSumBytes];
@@ -78,7 +84,7 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_tn_slices(GemmArgs g) {
   const uint32_t voff_sw = (uint32_t)(n0 / 128) * steps * kMxUnit + lane * 8 + (uint32_t)(n0 % 128) / 64 * 4;
 
   const uint32_t r8 = lane >> 3, c8 = lane & 7u;
-  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_address(ring) + wave * (kDepth * kStageBytes));
+  const uint32_t ring0 = __builtin_amdgcn_readfirstlane(lds_address(ring) + wave * (kStages * kStageBytes));
   uint32_t voff_x[2], voff_w[2], chunk16[2];
 #pragma unroll
   for (int p = 0; p < 2; ++p) {
@@ -132,13 +138,8 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_tn_slices(GemmArgs g) {
 #pragma unroll
     for (int j = 0; j < kNB; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
-  const uint8_t* const mine = ring + wave * (kDepth * kStageBytes);
-  issue_step(0, wave);
-  uint32_t stage = 0;
-  for (uint32_t at = wave; at < steps; at += kWaves) {
-    issue_step(stage ^ 1u, at + (kDepth - 1) * kWaves);
-    wait_vmcnt<kVm * (kDepth - 1)>();
-    const uint8_t* base = mine + stage * kStageBytes;
+  uint8_t* const mine = ring + wave * (kStages * kStageBytes);
+  const auto multiply = [&](const uint8_t* base) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < kSlices; ++s) {
       Frag fx[kMB], fw[kNB];
@@ -162,10 +163,65 @@ __global__ __launch_bounds__(64 * kWaves) void gemm_tn_slices(GemmArgs g) {
           for (int j = 0; j < kNB; ++j) acc[i][j] = G::mfma(fw[j], fx[i], acc[i][j]);
       }
     }
-    wait_lgkmcnt0();   // the reads are back before the next turn refills a stage
-    stage ^= 1u;
+  };
+  if constexpr (kAnyRows) {
+    typedef typename std::conditional<T::kBytes == 2, uint16_t, uint8_t>::type E;
+    const uint8_t* const base_x = (const uint8_t*)g.A + m0 * (int64_t)lda_b;
+    const uint8_t* const base_w = (const uint8_t*)g.B + n0 * (int64_t)ldb_b;
+    uint32_t off[kCopies];   // rows past the end repeat the last one: nothing of them is stored
+#pragma unroll
+    for (int c = 0; c < kCopies; ++c) {
+      const uint32_t row = c * 8 + r8, last_x = (uint32_t)rows_x - 1, last_w = (uint32_t)rows_w - 1;
+      off[c] = (c < kTm / 8 ? (row < last_x ? row : last_x) * lda_b : (row - kTm < last_w ? row - kTm : last_w) * ldb_b) + chunk16[c & 1];
+    }
+    u32x4 next[kCopies];
+    const auto load = [&](uint32_t at) __attribute__((always_inline)) {
+      uint32_t kk = at + rot;
+      kk = kk >= steps ? kk - steps : kk;
+      const uint32_t soff = __builtin_amdgcn_readfirstlane(kk * kRowBytes);
+      if (tail_bytes == 0 || kk != steps - 1) {
+#pragma unroll
+        for (int c = 0; c < kCopies; ++c)
+          __builtin_memcpy(&next[c], (const E*)((c < kTm / 8 ? base_x : base_w) + soff + (uint64_t)off[c]), 16);
+      } else {
+        // Chunks up to the row's end as they are; the one that straddles it from the row's last 16 bytes, moved down; zeros behind.
+        const uint32_t drop = 16u - tail_bytes % 16u;   // bytes of a chunk past the row's end; 16: none straddles it
+#pragma unroll
+        for (int c = 0; c < kCopies; ++c) {
+          const uint32_t chunk = chunk16[c & 1];
+          const bool whole = chunk + 16 <= tail_bytes, straddles = !whole && chunk < tail_bytes;
+          const int64_t to_end = whole ? 0 : (int64_t)tail_bytes - 16 - (int64_t)chunk;
+          u32x4 v;
+          __builtin_memcpy(&v, (const E*)((c < kTm / 8 ? base_x : base_w) + soff + (uint64_t)off[c] + to_end), 16);
+          u32x4 d = v;
+          if (drop & 8u) d = (u32x4){d[2], d[3], 0u, 0u};
+          if (drop & 4u) d = (u32x4){d[1], d[2], d[3], 0u};
+          d = (u32x4){__builtin_amdgcn_alignbyte(d[1], d[0], drop), __builtin_amdgcn_alignbyte(d[2], d[1], drop),
+                      __builtin_amdgcn_alignbyte(d[3], d[2], drop), __builtin_amdgcn_alignbyte(0u, d[3], drop)};
+#pragma unroll
+          for (int i = 0; i < 4; ++i) next[c][i] = whole ? v[i] : straddles ? d[i] : 0u;
+        }
+      }
+    };
+    if (wave < steps) load(wave);
+    for (uint32_t at = wave; at < steps; at += kWaves) {
+#pragma unroll
+      for (int c = 0; c < kCopies; ++c) *(u32x4*)(mine + c * 1024 + lane * 16) = next[c];
+      if (at + kWaves < steps) load(at + kWaves);
+      multiply(mine);
+    }
+  } else {
+    issue_step(0, wave);
+    uint32_t stage = 0;
+    for (uint32_t at = wave; at < steps; at += kWaves) {
+      issue_step(stage ^ 1u, at + kWaves);
+      wait_vmcnt<kVm>();
+      multiply(mine + stage * kStageBytes);
+      wait_lgkmcnt0();   // the reads are back before the next turn refills a stage
+      stage ^= 1u;
+    }
+    wait_vmcnt<0>();
   }
-  wait_vmcnt<0>();
   // the scaled MFMAs are inline assembly: the compiler does not know how long their results take
   if constexpr (kMx) asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
   __syncthreads();
@@ -210,18 +266,40 @@ constexpr Form kForms[] = {
     {2, 2, 4, 2.79, 0.085, 5.76, 4.26, 0.087, 1.63}, {2, 4, 4, 3.08, 0.178, 4.55, 5.30, 0.088, 2.00},
     {4, 4, 4, 3.74, 0.281, 5.08, 6.84, 0.036, 2.68}};
 
+// With rows of any alignment (420 problems, 9-12 % rms): a CU takes in less, as most pieces of rows straddle cache lines (rows at
+// multiples of 4 bytes and more as below, of 2 bytes 1.25 times the MB, of 1 byte 1.6 times).
+constexpr Form kAnyRowsForms[] = {
+    {1, 1, 4, 2.41, 0.158, 10.1, 3.56, 0.080, 0.65}, {1, 1, 8, 2.74, 0.010, 11.7, 1.83, 0.089, 0.88},
+    {1, 2, 4, 2.61, 0.089, 11.4, 3.21, 0.105, 0.56}, {2, 2, 2, 2.65, 0.239, 9.87, 4.95, 0.068, 1.50},
+    {2, 2, 4, 2.97, 0.069, 11.1, 3.70, 0.087, 1.09}, {4, 4, 4, 4.32, 0.158, 10.8, 5.78, 0.071, 2.95},
+    {5, 4, 4, 4.67, 0.224, 10.5, 7.01, 0.043, 3.19}};
+
 constexpr int64_t kCuSlots = 256;
 int64_t ceil_div(int64_t a, int64_t b) { return (a + b - 1) / b; }
 
-double form_us(const Form& f, int64_t M, int64_t N, int64_t steps, bool mx) {
+double form_us(const Form& f, int stages, int64_t M, int64_t N, int64_t steps, bool mx, double intake = 1.0) {
   const int64_t tiles = ceil_div(M, 16 * f.mb) * ceil_div(N, 16 * f.nb);
-  const int64_t lds = (int64_t)f.waves * kDepth * (16 * (f.mb + f.nb) * kRowBytes + (mx ? 512 : 0));
+  const int64_t lds = (int64_t)f.waves * stages * (16 * (f.mb + f.nb) * kRowBytes + (mx ? 512 : 0));
   const int64_t by_lds = 163840 / lds, by_waves = 32 / f.waves, resident = by_lds < by_waves ? by_lds : by_waves;
-  const double tile_mb = 16e-6 * (f.mb + f.nb) * kRowBytes * (double)steps;
+  const double tile_mb = intake * 16e-6 * (f.mb + f.nb) * kRowBytes * (double)steps;
   return f.launch + f.per_step * (double)ceil_div(steps, f.waves) + f.round_mb * (double)ceil_div(tiles, kCuSlots) * tile_mb +
          f.mean_mb * (double)tiles / kCuSlots * tile_mb + f.unique_mb * 1e-6 * kRowBytes * (double)((M + N) * steps) +
          f.round * (double)(ceil_div(tiles, kCuSlots * resident) - 1);
 }
+
+// The shortest of `n` forms and its estimate.
+int shortest_form(const Form* forms, int n, int stages, int64_t M, int64_t N, int64_t steps, bool mx, double intake, double* us) {
+  int best = 0;
+  for (int f = 0; f < n; ++f) {
+    const double e = form_us(forms[f], stages, M, N, steps, mx, intake);
+    if (f == 0 || e < *us) {
+      *us = e;
+      best = f;
+    }
+  }
+  return best;
+}
+constexpr int kFormCount = sizeof(kForms) / sizeof(kForms[0]), kAnyRowsFormCount = sizeof(kAnyRowsForms) / sizeof(kAnyRowsForms[0]);
 
 // The same for the route the problem takes otherwise, fitted on the same problems (5-9 % rms): the streaming kernel or 128 x 128
 // tiles, with or without a K split.
@@ -238,40 +316,43 @@ double other_us(const SlicesAlternative& o, int64_t M, int64_t N, int64_t steps)
   return 4.98 + 0.479 * round_steps + 0.108 * unique_mb + 0.323 * planes_mb;
 }
 
-template <class T, class OutT, int kForm>
+template <class T, class OutT, bool kAnyRows, int kForm>
 int launch_form(GemmArgs g, hipStream_t stream) {
-  constexpr Form f = kForms[kForm];
+  constexpr Form f = kAnyRows ? kAnyRowsForms[kForm] : kForms[kForm];
   g.tiles_m = (g.M + 16 * f.mb - 1) / (16 * f.mb);
   g.tiles_n = (g.N + 16 * f.nb - 1) / (16 * f.nb);
-  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n));
+  const dim3 grid((unsigned)(g.tiles_m * g.tiles_n)), threads(64 * f.waves);
   if constexpr (!std::is_same<T, MxE4M3>::value) {
-    if (g.c_ragged) {
-      hipLaunchKernelGGL((gemm_tn_slices<T, OutT, f.mb, f.nb, f.waves, true>), grid, dim3(64 * f.waves), 0, stream, g);
+    if (kAnyRows || g.c_ragged) {   // one form for every C beside rows of A and B of any alignment
+      hipLaunchKernelGGL((gemm_tn_slices<T, OutT, f.mb, f.nb, f.waves, true, kAnyRows>), grid, threads, 0, stream, g);
       return hipGetLastError() == hipSuccess ? 0 : -1;
     }
   }
-  hipLaunchKernelGGL((gemm_tn_slices<T, OutT, f.mb, f.nb, f.waves, false>), grid, dim3(64 * f.waves), 0, stream, g);
+  if constexpr (!kAnyRows) hipLaunchKernelGGL((gemm_tn_slices<T, OutT, f.mb, f.nb, f.waves, false, false>), grid, threads, 0, stream, g);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-template <class T, class OutT>
+template <class T, class OutT, bool kAnyRows>
 int launch_any(const GemmArgs& g, int form, hipStream_t s) {
+  static_assert(kFormCount == 7 && kAnyRowsFormCount == 7, "one case per form");
   switch (form) {
-    case 0: return launch_form<T, OutT, 0>(g, s);
-    case 1: return launch_form<T, OutT, 1>(g, s);
-    case 2: return launch_form<T, OutT, 2>(g, s);
-    case 3: return launch_form<T, OutT, 3>(g, s);
-    case 4: return launch_form<T, OutT, 4>(g, s);
-    case 5: return launch_form<T, OutT, 5>(g, s);
-    case 6: return launch_form<T, OutT, 6>(g, s);
+    case 0: return launch_form<T, OutT, kAnyRows, 0>(g, s);
+    case 1: return launch_form<T, OutT, kAnyRows, 1>(g, s);
+    case 2: return launch_form<T, OutT, kAnyRows, 2>(g, s);
+    case 3: return launch_form<T, OutT, kAnyRows, 3>(g, s);
+    case 4: return launch_form<T, OutT, kAnyRows, 4>(g, s);
+    case 5: return launch_form<T, OutT, kAnyRows, 5>(g, s);
+    case 6: return launch_form<T, OutT, kAnyRows, 6>(g, s);
   }
   return -1;
 }
 
-template <class T>
+template <class T, bool kAnyRows>
 int launch_out(const GemmArgs& g, int out_dtype, int form, hipStream_t s) {
-  return out_dtype == 0 ? launch_any<T, BF16>(g, form, s) : launch_any<T, F16>(g, form, s);
+  return out_dtype == 0 ? launch_any<T, BF16, kAnyRows>(g, form, s) : launch_any<T, F16, kAnyRows>(g, form, s);
 }
+
+bool on_this_route(const SlicesAlternative& other) { return other.streams || other.tile_rows <= 128; }
 
 }  // namespace
 
@@ -279,28 +360,48 @@ int launch_out(const GemmArgs& g, int out_dtype, int form, hipStream_t s) {
 // to the streaming kernel, which HBM bounds there as it would this one (M <= 16: 10-20 % faster here between 24 and 48 MiB, 4 % from
 // there to 90), and so is everything whose plan has tiles of 256 rows.  MI355_RING_TILE, which forces a tile for measurements,
 // keeps problems off this kernel as well.  Of the 800 problems, 17 are more than 2 % slower than on the other route.
-int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other) {
-  if (M <= 0 || N <= 0 || K <= 0 || (double)M * (double)N * (double)K > kSlicesMaxProducts) return -1;
-  if (!other.streams && other.tile_rows > 128) return -1;
-  if ((double)N * (double)K * elem_bytes > (M <= 16 ? 48.0 : 32.0) * 1048576.0 || std::getenv("MI355_RING_TILE")) return -1;
+int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other, double* route_us) {
   const int64_t steps = ceil_div(K * elem_bytes, kRowBytes);
-  int best = -1;
-  double us = 0.9 * other_us(other, M, N, steps);
-  for (int f = 0; f < (int)(sizeof(kForms) / sizeof(kForms[0])); ++f) {
-    const double e = form_us(kForms[f], M, N, steps, mx);
-    if (e < us) {
-      us = e;
-      best = f;
-    }
-  }
-  return best;
+  double us = 0;
+  const double limit = on_this_route(other) ? other_us(other, M, N, steps) : ring_shortest_us(M, N, K, elem_bytes);
+  if (route_us) *route_us = limit;
+  if (M <= 0 || N <= 0 || K <= 0 || (double)M * (double)N * (double)K > kSlicesMaxProducts || !on_this_route(other)) return -1;
+  if ((double)N * (double)K * elem_bytes > (M <= 16 ? 48.0 : 32.0) * 1048576.0 || std::getenv("MI355_RING_TILE")) return -1;
+  const int form = shortest_form(kForms, kFormCount, kDepth, M, N, steps, mx, 1.0, &us);
+  if (us >= 0.9 * limit) return -1;
+  if (route_us) *route_us = us;
+  return form;
+}
+
+// The other route of a product with rows of any alignment is `other` (or this kernel, whichever is shorter) behind a repacking of
+// `copied` bytes: us = 6.4 + 0.36 x MB + 0.75 x product + 0.25 x million outputs (296 problems, 11 % rms).  Taken from 0.97 of it:
+// 0.66 of the time before on average over those, as the better choice on each would leave, 4 of them 4-24 % slower.  Small 16-bit
+// products (copied == 0) have none but one thread or a sixteenth of a wave per output, which was slower on all of 124 problems.
+int slices_any_rows_config(int64_t M, int64_t N, int64_t K, int elem_bytes, int alignment, int64_t copied, const SlicesAlternative& other) {
+  if (M <= 0 || N <= 0 || K * elem_bytes < 16 || (double)M * (double)N * (double)K > kSlicesMaxProductsAnyRows) return -1;
+  if (std::getenv("MI355_RING_TILE")) return -1;
+  double us = 0, product = 0;
+  const int form = shortest_form(kAnyRowsForms, kAnyRowsFormCount, 1, M, N, ceil_div(K * elem_bytes, kRowBytes), false,
+                                 alignment % 4 == 0 ? 1.0 : alignment % 2 == 0 ? 1.25 : 1.6, &us);
+  if (copied == 0) return form;
+  slices_config(M, N, K, elem_bytes, false, other, &product);
+  return us < 0.97 * (6.44 + 0.357e-6 * (double)copied + 0.751 * product + 0.25e-6 * (double)M * (double)N) ? form : -1;
 }
 
 int launch_slices(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream) {
   switch (in_dtype) {
-    case 0: return launch_out<BF16>(g, out_dtype, config, stream);
-    case 1: return launch_out<F16>(g, out_dtype, config, stream);
-    case 2: return g.mx_a ? launch_out<MxE4M3>(g, out_dtype, config, stream) : launch_out<E4M3>(g, out_dtype, config, stream);
+    case 0: return launch_out<BF16, false>(g, out_dtype, config, stream);
+    case 1: return launch_out<F16, false>(g, out_dtype, config, stream);
+    case 2: return g.mx_a ? launch_out<MxE4M3, false>(g, out_dtype, config, stream) : launch_out<E4M3, false>(g, out_dtype, config, stream);
+  }
+  return -1;
+}
+
+int launch_slices_any_rows(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream) {
+  switch (in_dtype) {
+    case 0: return launch_out<BF16, true>(g, out_dtype, config, stream);
+    case 1: return launch_out<F16, true>(g, out_dtype, config, stream);
+    case 2: return launch_out<E4M3, true>(g, out_dtype, config, stream);
   }
   return -1;
 }

@@ -1,4 +1,5 @@
-// Small products whose operands have rows of any alignment: one wave per block of 4 x 4 outputs, K spread over its lanes.
+// Small products on fp32 sums whose operands have rows of any alignment: one wave per block of 4 x 4 outputs, K spread over its lanes.
+// For e4m3, whose sums on the matrix cores are coarser (16-bit products run on gemm_tn_slices, where their rows are in its reach).
 //
 // What the streaming and tile kernels cannot address (K*elem_bytes or a row stride not a multiple of 16, A or B misaligned)
 // and is too small to be worth repacking used to run one serial chain of K additions per thread, bound by the latency of

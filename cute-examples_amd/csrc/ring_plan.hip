@@ -151,6 +151,8 @@ constexpr double kSecondLaunchUs = 3.0;
 
 }  // namespace
 
+double ring_shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes) { return shortest_us(M, N, K, elem_bytes); }
+
 // One row (M <= 128) or one column (N <= 128) of 128 x 128 tiles on the nine-slot ring, K split as
 // uniform_splits says: every workgroup streams its own rows of B from HBM, and the ring that keeps
 // four k-steps in flight does that faster than the five-slot ring and than the streaming kernel's

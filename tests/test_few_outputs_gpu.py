@@ -5,7 +5,7 @@ import torch
 
 import gemm_kernels
 from tests import abi_ctypes as ac
-from tests.few_outputs_cases import MX, PLAIN
+from tests.few_outputs_cases import ANY_ROWS, MX, PLAIN
 
 pytestmark = pytest.mark.gpu
 DT = {ac.BF16: torch.bfloat16, ac.F16: torch.float16, ac.E4M3: torch.float8_e4m3fn}
@@ -50,3 +50,25 @@ def test_block_scaled(M, N, K):
         C = torch.full((M, N), float("nan"), dtype=out, device="cuda")
         gemm_kernels.gemm_tn_mxfp8(x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), sx, sw, C)
         assert torch.equal(C, want.to(torch.float32).to(out))
+
+
+@pytest.mark.parametrize("M,N,K,code,offset,gap", ANY_ROWS)
+def test_rows_of_any_alignment(M, N, K, code, offset, gap):
+    """What lies between the rows and around the operands is NaN."""
+    abi = ac.load()
+    x, w = integers(M, N, K)
+    want = x.double() @ w.double().T
+    views = []
+    for v in (x, w):
+        nan = torch.full((offset + v.shape[0] * (K + gap),), float("nan"), device="cuda").to(DT[code])
+        view = torch.as_strided(nan, v.shape, (K + gap, 1), offset)
+        view.copy_(v)
+        views.append(view)
+    A, B = views
+    ws = torch.empty(1 << 27, dtype=torch.uint8, device="cuda")
+    for pad in (0, 1, 2):
+        C = torch.full((M, N + pad), float("nan"), dtype=torch.bfloat16, device="cuda")
+        st = abi.mi355_gemm_tn(A.data_ptr(), B.data_ptr(), C.data_ptr(), M, N, K, K + gap, K + gap, N + pad, code, ac.BF16, 1.0, ac.AUTO,
+                               ws.data_ptr(), ws.numel(), torch.cuda.current_stream().cuda_stream)
+        assert st == ac.OK
+        assert torch.equal(C[:, :N], want.to(torch.float32).to(torch.bfloat16)) and bool(C[:, N:].isnan().all())
