@@ -546,6 +546,10 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
     p.M = m;
     p.N = n;
     p.c_streams = c_streams(m, n, K, 1);
+    if (m != M || n != N) {
+      const int form = few_outputs(m, n, K, 1, true, false);
+      if (form >= 0) return mi355::launch_slices(p, MI355_E4M3, out_dtype, form, s) == 0 ? (int)MI355_OK : (int)MI355_ERR_LAUNCH;
+    }
     int splits, tail_tiles, tail_splits;
     const size_t partial = mx_partial_bytes(m, n, K, &splits, &tail_tiles, &tail_splits);
     if (partial && workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= used + partial) {
@@ -557,11 +561,11 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
     const int tile = mi355::ring_tile_edge(m, n, K, 1, true);
     p.tiles_m = (m + mi355::ring_tile_rows(tile) - 1) / mi355::ring_tile_rows(tile);
     p.tiles_n = (n + mi355::ring_tile_cols(tile) - 1) / mi355::ring_tile_cols(tile);
-    return mi355::launch_tile_ring_mx(p, out_dtype, tile, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
+    return mi355::launch_tile_ring_mx(p, out_dtype, tile, s) == 0 ? (int)MI355_OK : (int)MI355_ERR_LAUNCH;
   };
-  // Two launches where a cut spares a partly filled last round of workgroups, as for plain operands (ring_first_piece).
+  // Two launches where a cut spares a partly filled last round of workgroups, as for plain operands.
   bool along_m = false;
-  const int64_t first = mi355::ring_first_piece(M, N, K, 1, &along_m);
+  const int64_t first = mi355::ring_cut(M, N, K, 1, &along_m);
   if (first <= 0) return tiles_of_piece(0, M, 0, N);
   st = along_m ? tiles_of_piece(0, first, 0, N) : tiles_of_piece(0, M, 0, first);
   if (st != MI355_OK) return st;
@@ -608,30 +612,34 @@ namespace {
 //   kRowsRagged      of any 2-byte alignment (GemmArgs::c_ragged; BASIC and SKINNY only)
 enum CRows { kRowsAligned, kRowsRagged };
 
-// One problem on the variant v (resolved, not AUTO).  from_auto: the caller left the choice to the library, which may then
+// Whose choice the variant is: the caller's, the library's, or the library's for a piece of a problem that it has cut in two.
+enum Choice { kExplicit, kAuto, kPiece };
+
+// One problem on the variant v (resolved, not AUTO).  kAuto: the caller left the choice to the library, which may then
 // cut the problem in two or leave the streaming kernel for the tile kernel.  The plan is that of N rounded up to 4.
 int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
-                int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, int v, bool from_auto,
+                int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, int v, Choice choice,
                 CRows c_rows, void* workspace, size_t workspace_bytes, hipStream_t s, WorkspaceMode mode) {
   const bool strict = mode != kLenient, dry = mode == kStrictDry;
   const int es = elem_bytes(in_dtype);
   const int64_t Np = mi355::partial_columns(N);
-  const int config = from_auto && (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_SKINNY) ? few_outputs(M, Np, K, es, false, v == MI355_VARIANT_SKINNY) : -1;
+  const bool from_auto = choice == kAuto;
+  const int config = choice != kExplicit && (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_SKINNY) ? few_outputs(M, Np, K, es, false, v == MI355_VARIANT_SKINNY) : -1;
   if (config < 0 && from_auto && v == MI355_VARIANT_BASIC) {
-    // Two launches where the planner finds a cut that spares a partly filled last round (ring_first_piece): each
+    // Two launches where the planner finds a cut that spares a partly filled last round (ring_cut): each
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
     // the other on the stream and through the same workspace.
     bool along_m = false;
-    const int64_t first = mi355::ring_first_piece(M, Np, K, es, &along_m);
+    const int64_t first = mi355::ring_cut(M, Np, K, es, &along_m);
     if (first > 0) {
       const int st = run_variant(A, B, C, along_m ? first : M, along_m ? N : first, K, lda, ldb, ldc, in_dtype, out_dtype, scale,
-                                 scale_a, scale_b, v, false, c_rows, workspace, workspace_bytes, s, mode);
+                                 scale_a, scale_b, v, kPiece, c_rows, workspace, workspace_bytes, s, mode);
       if (st != MI355_OK) return st;
       const uint8_t* a2 = (const uint8_t*)A + (along_m ? first * lda * es : 0);
       const uint8_t* b2 = (const uint8_t*)B + (along_m ? 0 : first * ldb * es);
       uint8_t* c2 = (uint8_t*)C + (along_m ? first * ldc : first) * 2;   // 16-bit output
       return run_variant(a2, b2, c2, along_m ? M - first : M, along_m ? N : N - first, K, lda, ldb, ldc, in_dtype, out_dtype,
-                         scale, scale_a, scale_b, v, false, c_rows, workspace, workspace_bytes, s, mode);
+                         scale, scale_a, scale_b, v, kPiece, c_rows, workspace, workspace_bytes, s, mode);
     }
   }
   mi355::GemmArgs g;
@@ -684,14 +692,14 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
       if (splits > 1) {
         const size_t need = (size_t)splits * (size_t)M * (size_t)Np * sizeof(float);
         if (usable(need)) g.splits = splits;
-        else if (strict) return MI355_ERR_SCRATCH;
+        else if (strict && choice != kPiece) return MI355_ERR_SCRATCH;
       } else {
         int tail_tiles, tail_splits;
         const size_t need = mi355::ring_tail(M, Np, K, es, &tail_tiles, &tail_splits);
         if (usable(need)) {
           g.tail_tiles = tail_tiles;
           g.tail_splits = tail_splits;
-        } else if (strict && need) {
+        } else if (strict && need && choice != kPiece) {   // a piece's split is no part of what the query counts on (ring_cut)
           return MI355_ERR_SCRATCH;
         }
       }
@@ -742,7 +750,7 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
                            size_t ws_bytes) {
     const CRows rows = padded || c_aligned ? kRowsAligned : kRowsRagged;
     return run_variant(a, b, c, M, N, Kp, ld_a, ld_b, ld_c, in_dtype, out_dtype, scale, scale_a, scale_b,
-                       rows == kRowsAligned ? v : v_ragged, true, rows, ws, ws_bytes, s, mode);
+                       rows == kRowsAligned ? v : v_ragged, kAuto, rows, ws, ws_bytes, s, mode);
   };
   // Small e4m3 products stay on fp32 sums (gemm_tn_small, the generic kernel): the matrix cores' fp8 sums are coarser.  Sums that
   // cancel, relative error behind the rounding to fp16: 1.8e-4 with either of the two at every K, 1.8e-4 / 2.4e-4 / 4.0e-4 / 6.9e-4
@@ -849,7 +857,7 @@ int run_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_
                        mode, &handled);
     if (handled) return st;
   }
-  return run_variant(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, out_dtype, scale, scale_a, scale_b, v, from_auto, kRowsAligned, workspace,
+  return run_variant(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, out_dtype, scale, scale_a, scale_b, v, from_auto ? kAuto : kExplicit, kRowsAligned, workspace,
                      workspace_bytes, s, mode);
 }
 

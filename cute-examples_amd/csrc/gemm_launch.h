@@ -78,6 +78,8 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
+// The cut that a call with MI355_VARIANT_AUTO makes: that one, or another that wants no more workspace.
+int64_t ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
 double ring_shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // estimate of the single-group kernel's plan
 // Whether MI355_VARIANT_AUTO computes a C whose rows start at odd 2-byte addresses into a padded copy that is then copied out (if
 // there is memory for it) instead of storing it directly.
@@ -121,6 +123,7 @@ struct SlicesAlternative {
 };
 constexpr double kSlicesMaxProducts = 1.5e10, kSlicesMaxProductsAnyRows = 3e10;   // M * N * K; the rules were fitted below
 int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other, double* route_us = nullptr);
+double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // the estimate of its shortest form, huge where the rule is not for
 int launch_slices(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);
 int slices_any_rows_config(int64_t M, int64_t N, int64_t K, int elem_bytes, int alignment, int64_t copied, const SlicesAlternative& other);
 int launch_slices_any_rows(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);

@@ -100,11 +100,12 @@ constexpr ShortTileCost kShort256 = {0.889, 5.38, 3.46}, kShort256x128 = {0.775,
 constexpr int64_t kShortSteps = 16;
 
 // k_loop_factor scales the k-step part of the small tile's estimate (not the fixed and reduction parts): see ring_tile_edge.
-double estimate_us(int tile, int64_t M, int64_t N, int64_t K, int elem_bytes, double k_loop_factor = 1.0) {
+// split: with the plan's K split or tail split.
+double estimate_us(int tile, int64_t M, int64_t N, int64_t K, int elem_bytes, double k_loop_factor = 1.0, bool split = true) {
   const int64_t rows = ring_tile_rows(tile), cols = ring_tile_cols(tile);
   const int64_t tm = (M + rows - 1) / rows, tn = (N + cols - 1) / cols, tiles = tm * tn;
   const int64_t steps = k_steps_of(K, elem_bytes);
-  const int s = uniform_splits(tiles, steps);
+  const int s = split ? uniform_splits(tiles, steps) : 1;
   const int64_t items = tiles * s;
   const double item_steps = (double)steps / s;
   double partial_mb = s > 1 ? (double)s * (double)M * (double)N * 4.0e-6 : 0.0;
@@ -124,7 +125,7 @@ double estimate_us(int tile, int64_t M, int64_t N, int64_t K, int elem_bytes, do
   const TileCost& c = tile == 256 ? kCost256 : kCost256x128;
   double rounds = (double)((items + kCuSlots - 1) / kCuSlots);
   double occupancy = (double)items / (rounds * (double)kCuSlots);
-  if (tile == 256 && s == 1) {
+  if (tile == 256 && s == 1 && split) {
     int tail_tiles, tail_splits;
     tail_plan(tiles, steps, &tail_tiles, &tail_splits);
     if (tail_tiles) {   // the last round takes 1/S of a round
@@ -144,6 +145,12 @@ double estimate_us(int tile, int64_t M, int64_t N, int64_t K, int elem_bytes, do
 double shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
   const double a = estimate_us(256, M, N, K, elem_bytes), b = estimate_us(kRingTile256x128, M, N, K, elem_bytes),
                c = estimate_us(128, M, N, K, elem_bytes);
+  return a < b ? (a < c ? a : c) : (b < c ? b : c);
+}
+
+double shortest_unsplit_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
+  const double a = estimate_us(256, M, N, K, elem_bytes, 1.0, false), b = estimate_us(kRingTile256x128, M, N, K, elem_bytes, 1.0, false),
+               c = estimate_us(128, M, N, K, elem_bytes, tiles_of(M, N, 128) <= kCuSlots && k_steps_of(K, elem_bytes) >= kShortSteps ? 0.82 : 1.0, false);
   return a < b ? (a < c ? a : c) : (b < c ? b : c);
 }
 
@@ -255,6 +262,40 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
       const double e = axis == 0 ? best_of(M, c * 256) + best_of(M, N - c * 256) : best_of(c * 256, N) + best_of(M - c * 256, N);
       if (e + kSecondLaunchUs < best) {
         best = e + kSecondLaunchUs;
+        extent = c * 256;
+        *along_m = axis == 1;
+      }
+    }
+  }
+  return extent;
+}
+
+// The cut that MI355_VARIANT_AUTO makes: ring_first_piece's (which the queries report), or one whose first piece is nearly whole
+// rounds -- as many tile columns (rows) as r rounds have room for -- and whose rest needs no workspace, where that is estimated to be
+// shorter, the second launch counted with 2 us.  Problems of a few tiles more than whole rounds have it, and of any number of k-steps:
+// bf16 1000 x 50257 x 768 (3.08 rounds) 118 -> 97 us, 1056 x 26704 x 2176 (2.05) 149 -> 117, e4m3 1509 x 11192 x 4864 (1.03) 93 -> 71.  Over 110
+// problems of 1.02...5 rounds and 2...40 k-steps 3.5 % less time on average (the best cut of each: 4.8 %), two of them 2 % more; of 90
+// others one is slower (fp16 1478 x 10784 x 768, 1.01 rounds, 28.3 -> 30.4 us).  Beyond 64 k-steps ring_first_piece's limit of rounds.
+int64_t ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m) {
+  int64_t extent = ring_first_piece(M, N, K, elem_bytes, along_m);
+  if (std::getenv("MI355_ONE_PIECE") || std::getenv("MI355_RING_TILE")) return extent;
+  const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, steps = k_steps_of(K, elem_bytes);
+  if (tm * tn <= kCuSlots || (tm * tn) % kCuSlots == 0 || tm * tn > 5 * kCuSlots || (steps > 64 && 10 * tm * tn > 34 * kCuSlots)) return extent;
+  double best = shortest_us(M, N, K, elem_bytes);
+  if (extent > 0) {
+    const int64_t rest_m = *along_m ? M - extent : M, rest_n = *along_m ? N : N - extent;
+    best = shortest_us(*along_m ? extent : M, *along_m ? N : extent, K, elem_bytes) + shortest_us(rest_m, rest_n, K, elem_bytes) + kSecondLaunchUs;
+  }
+  for (int axis = 0; axis < 2; ++axis) {
+    const int64_t across = axis == 0 ? tm : tn, along = axis == 0 ? tn : tm;   // axis 0: cut N, axis 1: cut M
+    for (int64_t r = tm * tn / kCuSlots; r > 0; --r) {
+      const int64_t c = r * kCuSlots / across;
+      if (c <= 0 || c >= along) continue;
+      const int64_t rest_m = axis == 0 ? M : M - c * 256, rest_n = axis == 0 ? N - c * 256 : N;
+      const double tiles = shortest_unsplit_us(rest_m, rest_n, K, elem_bytes), slices = slices_us(rest_m, rest_n, K, elem_bytes);
+      const double e = shortest_unsplit_us(axis == 0 ? M : c * 256, axis == 0 ? c * 256 : N, K, elem_bytes) + (tiles < slices ? tiles : slices) + 2.0;
+      if (e < best) {
+        best = e;
         extent = c * 256;
         *along_m = axis == 1;
       }

@@ -1,0 +1,41 @@
+"""Problems of a few tiles more than whole rounds: cut in two by a call, whatever the number of k-steps; what each half is, on the CPU."""
+import random
+
+import pytest
+
+from tests import abi_ctypes as ac
+from tests.test_dispatch_cpu import A, B, C, case, launches, matrix_core  # noqa: F401  (fixture)
+
+
+def covered(c, got, es):
+    """The products' rectangles of C make up all of it, each from its own rows of A and B."""
+    rects = []
+    for name, v in got:
+        if matrix_core(name):
+            m0, n0 = divmod((v["C"] - C) // 2, c["ldc"])
+            assert v["A"] == A + m0 * c["lda"] * es and v["B"] == B + n0 * c["ldb"] * es and v["K"] == c["K"]
+            rects.append((m0, n0, v["M"], v["N"]))
+    assert sum(m * n for _, _, m, n in rects) == c["M"] * c["N"]
+    assert all(m0 + m <= c["M"] and n0 + n <= c["N"] for m0, n0, m, n in rects)
+    assert len(rects) in (1, 2) and (len(rects) == 1 or rects[0][:2] == (0, 0) and rects[1][:2] in ((rects[0][2], 0), (0, rects[0][3])))
+    return len(rects)
+
+
+@pytest.mark.parametrize("M,N,K,in_dt", [(1000, 50257, 768, ac.BF16), (1000, 50260, 768, ac.F16), (1056, 26704, 2176, ac.BF16), (1509, 11192, 4864, ac.E4M3),
+                                         (6784, 2504, 2304, ac.BF16), (3748, 13208, 640, ac.BF16)])
+def test_cut(launches, M, N, K, in_dt):  # noqa: F811
+    es = 1 if in_dt == ac.E4M3 else 2
+    cases = [case(M, N, K, in_dt), case(M, N, K, in_dt, room=0) if N % 4 == 0 else case(M, N, K, in_dt, room=256), case(M, N, K, in_dt, noalloc=True)]
+    for c, (st, _, got) in zip(cases, launches(cases)):
+        assert st == ac.OK and covered(c, got, es) == 2, c
+
+
+def test_halves_cover_random_problems(launches):  # noqa: F811
+    rng = random.Random(3)
+    cases = []
+    for _ in range(300):
+        in_dt = rng.choice([ac.BF16, ac.E4M3])
+        M, N, K = int(2 ** rng.uniform(8, 13.2)), int(2 ** rng.uniform(9, 15.6)) // 4 * 4, int(2 ** rng.uniform(7, 13)) // 16 * 16
+        cases.append(case(M, N, K, in_dt, room=rng.choice([0, None])))
+    seen = {covered(c, got, 1 if c["in_dt"] == ac.E4M3 else 2) for c, (st, _, got) in zip(cases, launches(cases)) if st == ac.OK}
+    assert seen == {1, 2}
