@@ -9,6 +9,7 @@
 // (gemm_test.cu:82-85).  Every check that does not need a GPU runs before the first HIP call.
 #include <torch/extension.h>
 
+#include <ATen/hip/EmptyTensor.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
@@ -47,6 +48,13 @@ const char* variant_name(int v) {
     case MI355_VARIANT_ALTERNATE: return "alternate";
   }
   return "?";
+}
+
+// Uninitialised memory on a device from torch's caching allocator, so stream-ordered with the launches that use it, without the two
+// passes through the dispatcher that torch::empty makes: small calls are bound by the host (8 x 384, back to back: e4m3 quantiser 6.0 ->
+// 5.0 us, of which half is its scale as a 0-dim tensor without sa[0]; MXFP8 quantiser 5.4 -> 4.8; fp8 layer 9.8 -> 9.0).
+torch::Tensor device_empty(at::IntArrayRef sizes, at::ScalarType dtype, const torch::Tensor& like) {
+  return torch::Tensor(at::detail::empty_cuda(sizes, dtype, like.device(), std::nullopt));
 }
 
 // A scale given as a one-element tensor on the GEMM's device is passed by address (no host
@@ -96,8 +104,7 @@ torch::Tensor run(const torch::Tensor& A, const torch::Tensor& B, torch::Tensor 
   torch::Tensor ws;
   void* ws_ptr = nullptr;
   if (ws_bytes) {
-    // From torch's caching allocator, so the memory is stream-ordered with the launch below.
-    ws = torch::empty({(int64_t)ws_bytes}, A.options().dtype(torch::kUInt8));
+    ws = device_empty({(int64_t)ws_bytes}, at::kByte, A);
     ws_ptr = ws.data_ptr();
   }
   st = mi355_gemm_tn_scaled(A.const_data_ptr(), B.const_data_ptr(), C.mutable_data_ptr(), M, N, K, K, K,
@@ -158,15 +165,16 @@ std::pair<torch::Tensor, torch::Tensor> quantize_e4m3(const torch::Tensor x) {
   TORCH_CHECK(x.is_cuda(), "gemm_kernels runs on a HIP device only; got a tensor on ", x.device());
   c10::DeviceGuard guard(x.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-  torch::Tensor q = torch::empty(x.sizes(), x.options().dtype(at::kFloat8_e4m3fn));
+  torch::Tensor q = device_empty(x.sizes(), at::kFloat8_e4m3fn, x);
   // scale, amax, and behind them the quantiser's scratch memory
   const size_t scratch = mi355_quantize_e4m3_scratch_bytes(x.numel());
-  torch::Tensor sa = torch::empty({2 + (int64_t)(scratch / sizeof(float))}, x.options().dtype(at::kFloat));
+  torch::Tensor sa = device_empty({2 + (int64_t)(scratch / sizeof(float))}, at::kFloat, x);
   float* sa_ptr = sa.data_ptr<float>();
   int st = mi355_quantize_e4m3_scratch(x.const_data_ptr(), dt, x.numel(), q.mutable_data_ptr(), sa_ptr,
                                        scratch ? sa_ptr + 2 : nullptr, scratch, (void*)stream);
   TORCH_CHECK(st == MI355_OK, "gemm_kernels: ", mi355_gemm_strerror(st));
-  return {q, sa[0]};
+  sa.unsafeGetTensorImpl()->set_sizes_contiguous(at::IntArrayRef());   // the first element, as a 0-dim tensor
+  return {q, sa};
 }
 
 // Scale bytes of an MX operand: a uint8 (or float8_e8m0fnu) tensor (rows, K/32), rows contiguous.
@@ -224,7 +232,7 @@ torch::Tensor gemm_tn_mxfp8(const torch::Tensor A_q, const torch::Tensor B_q, co
   torch::Tensor ws;
   void* ws_ptr = nullptr;
   if (ws_bytes) {
-    ws = torch::empty({(int64_t)ws_bytes}, A_q.options().dtype(torch::kUInt8));
+    ws = device_empty({(int64_t)ws_bytes}, at::kByte, A_q);
     ws_ptr = ws.data_ptr();
   }
   st = mi355_gemm_tn_mxfp8(A_q.const_data_ptr(), B_q.const_data_ptr(), C.mutable_data_ptr(), M, N, K, K, K, ldc, sa,
@@ -246,7 +254,7 @@ torch::Tensor shuffle_mx_scales(const torch::Tensor scales) {
   TORCH_CHECK(scales.is_cuda(), "gemm_kernels runs on a HIP device only; got a tensor on ", scales.device());
   c10::DeviceGuard guard(scales.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(scales.device().index()).stream();
-  torch::Tensor out = torch::empty({(int64_t)mi355_mx_shuffled_bytes(rows, K)}, scales.options().dtype(at::kByte));
+  torch::Tensor out = device_empty({(int64_t)mi355_mx_shuffled_bytes(rows, K)}, at::kByte, scales);
   int st = mi355_mx_shuffle_scales((const uint8_t*)scales.const_data_ptr(), rows, K, rows > 1 ? scales.stride(0) : K / 32,
                                    out.data_ptr<uint8_t>(), (void*)stream);
   TORCH_CHECK(st == MI355_OK, "gemm_kernels: ", mi355_gemm_strerror(st));
@@ -270,10 +278,10 @@ std::pair<torch::Tensor, torch::Tensor> quantize_mxfp8(const torch::Tensor x, bo
   TORCH_CHECK(x.is_cuda(), "gemm_kernels runs on a HIP device only; got a tensor on ", x.device());
   c10::DeviceGuard guard(x.device());
   hipStream_t stream = c10::hip::getCurrentHIPStream(x.device().index()).stream();
-  torch::Tensor q = torch::empty({rows, K}, x.options().dtype(at::kFloat8_e4m3fn));
+  torch::Tensor q = device_empty({rows, K}, at::kFloat8_e4m3fn, x);
   TORCH_CHECK(!shuffled || K % 128 == 0, "shuffled scales need the last dimension to be a multiple of 128");
-  torch::Tensor sc = shuffled ? torch::empty({(int64_t)mi355_mx_shuffled_bytes(rows, K)}, x.options().dtype(at::kByte))
-                              : torch::empty({rows, K / 32}, x.options().dtype(at::kByte));
+  torch::Tensor sc = shuffled ? device_empty({(int64_t)mi355_mx_shuffled_bytes(rows, K)}, at::kByte, x)
+                              : device_empty({rows, K / 32}, at::kByte, x);
   int st = mi355_quantize_mxfp8(x.const_data_ptr(), dt, rows, K, K, q.mutable_data_ptr(), sc.data_ptr<uint8_t>(),
                                 shuffled ? 1 : 0, (void*)stream);
   TORCH_CHECK(st == MI355_OK, "gemm_kernels: ", mi355_gemm_strerror(st));
