@@ -57,10 +57,11 @@ __device__ __forceinline__ uint32_t to_e4m3(float f) {
 // codes in one word (a in the lowest byte): the hardware conversion (v_cvt_pk_fp8_f32, OCP e4m3 on this GPU, round to
 // nearest even).  A NaN comes out of it as a code whose low seven bits are all ones, as no number does; the sign of such
 // codes is cleared.
+__device__ __forceinline__ uint32_t to_e4m3x4_numbers(float a, float b, float c, float d) {   // without NaN
+  return (uint32_t)__builtin_amdgcn_cvt_pk_fp8_f32(c, d, __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false), true);
+}
 __device__ __forceinline__ uint32_t to_e4m3x4_bounded(float a, float b, float c, float d) {
-  int w = __builtin_amdgcn_cvt_pk_fp8_f32(a, b, 0, false);
-  w = __builtin_amdgcn_cvt_pk_fp8_f32(c, d, w, true);
-  const uint32_t u = (uint32_t)w;
+  const uint32_t u = to_e4m3x4_numbers(a, b, c, d);
   const uint32_t nan_sign = ((u & 0x7f7f7f7fu) + 0x01010101u) & 0x80808080u;   // bit 7 of the bytes that hold 0x7f or 0xff
   return u & ~nan_sign;
 }

@@ -8,12 +8,16 @@
 // and the GEMM reads it from there.  One launch for small tensors (bound by its latency: bf16 16 x 4096 9.1 -> 3.8 us), two
 // for larger ones, or three where the caller has no scratch memory for the maxima of the workgroups.  Large tensors are
 // bound by their two reads and one write: bf16 8192 x 8192 65.6 -> 53.6 us, 6.3 TB/s (the maximum 22.7 us; the rest was
-// 47.7 us long on its divisions, see codes_of).  The reference has no fp8 path;
+// 47.7 us long on its divisions, see codes4), but for those that the chip holds: 41.8 us (quantize_resident_kernel).  The reference
+// has no fp8 path;
 // the contract is the benchmark configuration's (operands quantised with per-tensor fp32 scales
 // amax/448) and is checked against torch's float8_e4m3fn cast and the C restatement in the tests.
 #include "cdna4_primitives.h"
 #include "gemm_launch.h"
 #include "quantize_convert.h"
+#include "ring_common.h"
+
+#include <cstdlib>
 
 namespace mi355 {
 namespace {
@@ -78,10 +82,10 @@ __device__ __forceinline__ float workgroup_max(float m) {
   return m;
 }
 
-// x / scale for eight elements -> eight codes, the same bits whichever way is taken.
-//   kDivide   the IEEE division: about a dozen instructions, one of them quarter rate, per element; alone it takes longer
+// x / scale for four elements -> four codes, the same bits whichever way is taken.
+//   kDivide     the IEEE division: about a dozen instructions, one of them quarter rate, per element; alone it takes longer
 //             than the memory traffic of the pass (bf16 8192 x 8192: 47.7 us of vector instructions)
-//   else      Markstein's correction (IBM J. Res. Dev. 34, 1990) of x * y, y = 1 / scale correctly rounded: with
+//   kCorrected  Markstein's correction (IBM J. Res. Dev. 34, 1990) of x * y, y = 1 / scale correctly rounded: with
 //             r = x - (x*y) * scale, which one fused multiply-add gives exactly, x*y + r*y is the correctly rounded quotient:
 //             three instructions.  It needs r free of underflow for every quotient that does not round to code 0 (from 2^-11 on
 //             r is a multiple of 2^-57 times scale), hence the range of `scale` in markstein_ok.  The sign is taken from x (a
@@ -89,21 +93,63 @@ __device__ __forceinline__ float workgroup_max(float m) {
 //             conversion rounds to 448: no clamp.  NaN stays NaN through all of it.
 __device__ __forceinline__ bool markstein_ok(float scale) { return scale >= 0x1p-60f && scale <= 0x1p100f; }
 
-template <bool kDivide>
-__device__ __forceinline__ u32x2 codes_of(const float (&v)[8], float scale, float inv) {
-  if constexpr (kDivide) {
-    return (u32x2){to_e4m3x4(v[0] / scale, v[1] / scale, v[2] / scale, v[3] / scale),
-                   to_e4m3x4(v[4] / scale, v[5] / scale, v[6] / scale, v[7] / scale)};
+//   kProduct, kTwoProducts  for 16-bit x without NaN, see factors_for
+enum Quotient { kDivide, kCorrected, kProduct, kTwoProducts };
+// inv: 1 / scale, or factors_for's first factor; `more` its second.
+template <Quotient kQuotient>
+__device__ __forceinline__ uint32_t codes4(const float* v, float scale, float inv, float more = 0.f) {
+  if constexpr (kQuotient == kProduct) {
+    return to_e4m3x4_numbers(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+  } else if constexpr (kQuotient == kTwoProducts) {
+    return to_e4m3x4_numbers(__builtin_fmaf(v[0], inv, v[0] * more), __builtin_fmaf(v[1], inv, v[1] * more),
+                             __builtin_fmaf(v[2], inv, v[2] * more), __builtin_fmaf(v[3], inv, v[3] * more));
+  } else if constexpr (kQuotient == kDivide) {
+    return to_e4m3x4(v[0] / scale, v[1] / scale, v[2] / scale, v[3] / scale);
   } else {
-    float q[8];
+    float q[4];
 #pragma unroll
-    for (int k = 0; k < 8; ++k) {
+    for (int k = 0; k < 4; ++k) {
       const float q0 = v[k] * inv;
       const float r = __builtin_fmaf(-q0, scale, v[k]);
       q[k] = __builtin_copysignf(__builtin_fmaf(r, inv, q0), v[k]);
     }
-    return (u32x2){to_e4m3x4_bounded(q[0], q[1], q[2], q[3]), to_e4m3x4_bounded(q[4], q[5], q[6], q[7])};
+    return to_e4m3x4_bounded(q[0], q[1], q[2], q[3]);
   }
+}
+template <bool kDivides>
+__device__ __forceinline__ u32x2 codes_of(const float (&v)[8], float scale, float inv) {
+  constexpr Quotient kQuotient = kDivides ? kDivide : kCorrected;
+  return (u32x2){codes4<kQuotient>(v, scale, inv), codes4<kQuotient>(v + 4, scale, inv)};
+}
+
+// The codes of 16-bit x without NaN from one or two products per element (x * first, or x * first + x * more, rounded once, where
+// first + more is 1 / scale to 48 bits) instead of the corrected quotient.  They are off the quotient by less than 2^-21.9 of it, which
+// changes a code only if one of the codes' midpoints (odd m up to 31 times a power of two) lies that close to x / scale, that is, m *
+// scale that close to a value of so few bits as x has: at most one value per m (they are 2^-11 apart), and which side of the midpoint
+// it falls on does not depend on its power of two.  So those sixteen values are tried against the corrected quotient, with four first
+// factors within two units of the last place of 1 / scale and with the two products; what agrees on all sixteen will do for every x.
+// (m = 7 always is such a case, amax / 448 being amax / 7 but for a power of two.  One of the four factors does for 94 % of all amax.)
+// markstein_ok keeps the factors normal; a quotient below that rounds to a zero of x's sign either way, since more is not negative.
+struct Factors {
+  float first, more;   // first == 0: none
+};
+template <class In>
+__device__ __forceinline__ Factors factors_for(float scale, float inv) {
+  constexpr uint32_t kDropped = 24 - (std::is_same<In, BF16>::value ? 8 : 11);   // bits of a significand that x does not have
+  const uint32_t lane = threadIdx.x & 63u, pick = lane >> 4;
+  const float p = (float)(int)(2 * (lane & 15u) + 1) * scale * 0x1p-10f;
+  const uint32_t near = (__builtin_bit_cast(uint32_t, p) + (1u << (kDropped - 1))) & ~((1u << kDropped) - 1);
+  const float x = __builtin_bit_cast(float, near);
+  const auto ulps = [&](int n) { return __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, inv) + (uint32_t)n); };
+  const auto candidate = [&](uint32_t c) { return ulps(c == 3 ? 2 : c == 2 ? -1 : (int)c); };
+  const float v[4] = {x, x, x, x};
+  const uint32_t want = codes4<kCorrected>(v, scale, inv);
+  const uint64_t agree = __ballot(codes4<kProduct>(v, scale, candidate(pick)) == want);
+  for (uint32_t c = 0; c < 4; ++c)
+    if ((agree >> (16 * c) & 0xffffu) == 0xffffu) return {candidate(c), 0.f};
+  const float below = __builtin_fmaf(-inv, scale, 1.0f) < 0.f ? ulps(-1) : inv;   // the largest number not above 1 / scale
+  const float more = __builtin_fmaf(-below, scale, 1.0f) * inv;
+  return {__all(codes4<kTwoProducts>(v, scale, below, more) == want) ? below : 0.f, more};
 }
 
 template <bool kStream>
@@ -208,12 +254,255 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(const void* x, int
   else quantize_groups<In, true>(x, n, q, scale, inv, thread, stride, thread);
 }
 
+// Tensors of kResidentFrom bytes to what the chip holds, read once.  One workgroup per CU keeps its pieces of 8 KiB on the chip
+// between the maximum and the codes, 48 in registers (192 of a lane's 256) and 16 in LDS: 512 KiB per CU, 128 MiB in all.  Between the
+// two halves every workgroup waits for the maxima of all others, one word each in `slots`.  That they all run at the same time is how
+// the chip fills when nothing else does; it is not relied on: the wait is bounded, and a workgroup that gives up leaves its pieces to
+// quantize_left_kernel behind it, which finds nothing to do otherwise.
+// bf16 8192 x 8192 (128 MiB) 53.4 -> 41.8 us, of which reading 20, waiting 4, codes 11 (19 with the corrected quotient, see factors_for),
+// the two small launches around it 5; 96 MiB 41.2 -> 34.6, 80 MiB 35.7 -> 31.1, 64 MiB 30.8 / 30.1, 32 MiB 16.6 / 23.8; fp32 128 MiB 52.7 ->
+// 40.3, 80 MiB 33.2 -> 30.2, 64 MiB 28.2 / 29.3; with a part of 224 MiB read twice 89.5 / 104.  fp8 layer 8192^3 421 -> 406 us.
+constexpr int kHeld = 48, kHeldInLds = 16, kResident = kHeld + kHeldInLds, kResidentThreads = 512, kResidentBlocks = 256;
+constexpr int64_t kResidentFrom = (int64_t)80 << 20;
+constexpr int64_t kWaitTicks = 20000;      // of the 100 MHz clock: 200 us
+constexpr uint32_t kUnset = 0xffffffffu;   // no maximum: those are numbers, this is the pattern of a NaN
+typedef __attribute__((ext_vector_type(32))) uint32_t u32x32;
+
+template <class In> struct Chunk {   // 16 bytes of x
+  static constexpr int kPer = 16 / sizeof(typename Load8<In>::Element);
+  static __device__ __forceinline__ void decode(u32x4 a, float* v) {
+    if constexpr (std::is_same<In, float>::value) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) v[k] = __builtin_bit_cast(float, (uint32_t)a[k] + 0u);   // (of an element itself, the first one's bits)
+    } else if constexpr (std::is_same<In, BF16>::value) {
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        v[2 * k] = __builtin_bit_cast(float, a[k] << 16);
+        v[2 * k + 1] = __builtin_bit_cast(float, a[k] & 0xffff0000u);
+      }
+    } else {
+      const f16x8 h = __builtin_bit_cast(f16x8, a);
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = (float)h[k];
+    }
+  }
+  static __device__ __forceinline__ float amax(u32x4 a, float m) {
+    float v[kPer];
+    decode(a, v);
+#pragma unroll
+    for (int k = 0; k < kPer; ++k) m = __builtin_fmaxf(m, __builtin_fabsf(v[k]));
+    return m;
+  }
+  // Chunk `tid` of piece `piece`: the piece's address is the workgroup's, the chunk's a lane's 32-bit offset.
+  static __device__ __forceinline__ u32x4 load(const void* x, int64_t piece, uint32_t tid) {
+    return ((const u32x4*)x + piece * kResidentThreads)[tid];
+  }
+  template <Quotient kQuotient>
+  static __device__ __forceinline__ void store(uint8_t* q, int64_t piece, uint32_t tid, u32x4 a, float scale, float inv, float more = 0.f) {
+    float v[kPer];
+    decode(a, v);
+    // Written through the L2s and past the Infinity Cache (nt sc1), at once: what the L2s still hold when the kernel ends, the next one
+    // waits for, and lines left in the Infinity Cache cost other passes 8 us (bf16 8192 x 8192 43.7 or 51.5 us, by what came before;
+    // written through 41.3).
+    const __amdgpu_buffer_rsrc_t to = make_raw_buffer(q + piece * (kResidentThreads * kPer), kResidentThreads * kPer);
+    const uint32_t low = codes4<kQuotient>(v, scale, inv, more);
+    if constexpr (kPer == 8) __builtin_amdgcn_raw_buffer_store_b64((u32x2){low, codes4<kQuotient>(v + 4, scale, inv, more)}, to, tid * 8, 0, 18);
+    else __builtin_amdgcn_raw_buffer_store_b32(low, to, tid * 4, 0, 18);
+  }
+};
+
+// The largest magnitude of chunks.  16-bit values by their bits, two at a time (for magnitudes the order of the bits is that of the
+// numbers, with NaN above infinity): half the instructions of the decoded ones.
+template <class In> struct Largest {
+  typedef __attribute__((ext_vector_type(2))) uint16_t u16x2;
+  u16x2 most = {0, 0};
+  __device__ __forceinline__ void add(u32x4 a) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) most = __builtin_elementwise_max(most, __builtin_bit_cast(u16x2, (uint32_t)(a[k] & 0x7fff7fffu)));
+  }
+  __device__ __forceinline__ uint16_t bits() const { return most[0] > most[1] ? most[0] : most[1]; }
+  __device__ __forceinline__ bool has_nan() const { return bits() > (std::is_same<In, BF16>::value ? 0x7f80 : 0x7c00); }
+  __device__ __forceinline__ float value() const {
+    const uint16_t b = bits();
+    return Decode<In>::run(&b, 0);
+  }
+};
+template <> struct Largest<float> {
+  float most = 0.f;
+  __device__ __forceinline__ void add(u32x4 a) { most = Chunk<float>::amax(a, most); }
+  __device__ __forceinline__ bool has_nan() const { return false; }   // ignored by add, put right by the conversion
+  __device__ __forceinline__ float value() const { return most; }
+};
+
+// Pieces of workgroup b of `blocks`: b, b + blocks, ...  Whole pieces only; the elements behind the last one are workgroup 0's.
+template <class In>
+__device__ __forceinline__ int64_t pieces_of(int64_t n, int64_t b, int64_t blocks) {
+  const int64_t pieces = n / (Chunk<In>::kPer * kResidentThreads);
+  return (pieces - b + blocks - 1) / blocks;
+}
+
+template <class In, Quotient kQuotient>
+__device__ __forceinline__ void quantize_pieces(const void* x, int64_t n, uint8_t* q, float scale, float inv, int64_t mine) {
+#pragma unroll 4
+  for (int64_t i = 0; i < mine; ++i) {
+    const int64_t piece = i * gridDim.x + blockIdx.x;
+    Chunk<In>::template store<kQuotient>(q, piece, threadIdx.x, Chunk<In>::load(x, piece, threadIdx.x), scale, inv);
+  }
+}
+template <class In>
+__device__ __forceinline__ void quantize_rest(const void* x, int64_t n, uint8_t* q, float scale) {
+  if (blockIdx.x != 0) return;
+  constexpr int64_t kPiece = Chunk<In>::kPer * kResidentThreads;
+  for (int64_t i = n / kPiece * kPiece + threadIdx.x; i < n; i += kResidentThreads) q[i] = (uint8_t)to_e4m3(Load8<In>::one(x, i) / scale);
+}
+
+__global__ __launch_bounds__(2 * kResidentBlocks) void resident_init(uint32_t* slots) { slots[threadIdx.x] = threadIdx.x < kResidentBlocks ? kUnset : 0u; }
+
+// slots: kResidentBlocks maxima, then as many words that say whose pieces are done.
+template <class In>
+__global__ __launch_bounds__(kResidentThreads, 2) void quantize_resident_kernel(const void* x, int64_t n, uint8_t* q, float* out,
+                                                                                uint32_t* slots, int64_t wait_ticks) {
+  __shared__ __attribute__((aligned(1024))) uint8_t kept[kHeldInLds * kResidentThreads * 16];
+  const int64_t b = blockIdx.x, blocks = gridDim.x, mine = pieces_of<In>(n, b, blocks);
+  const uint32_t tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const auto piece = [&](int64_t i) __attribute__((always_inline)) { return i * blocks + b; };
+
+  Largest<In> most;
+  // kResident pieces; past the workgroup's last one, that one again.
+  const int64_t step = blocks * (kResidentThreads * 16);   // bytes from one of the workgroup's pieces to its next
+  const uint8_t* from = (const uint8_t*)x + b * (kResidentThreads * 16);
+  int left = (int)mine - 1;
+  const auto next = [&]() __attribute__((always_inline)) {
+    const uint8_t* p = from;
+    from += left > 0 ? step : 0;
+    --left;
+    return p;
+  };
+  u32x32 held[kHeld / 8];
+#pragma unroll
+  for (int j = 0; j < kHeld; ++j) {
+    const u32x4 a = ((const u32x4*)next())[tid];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) held[j / 8][j % 8 * 4 + k] = a[k];
+  }
+#pragma unroll
+  for (int j = 0; j < kHeldInLds; ++j)
+    dma_16B_to_lds(__builtin_amdgcn_readfirstlane(lds_address(kept) + j * (kResidentThreads * 16) + wave * 1024), tid * 16,
+                   make_raw_buffer(next(), kResidentThreads * 16), 0);
+#pragma unroll
+  for (int g = 0; g < kHeld / 8; ++g) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+      most.add((u32x4){held[g][4 * j], held[g][4 * j + 1], held[g][4 * j + 2], held[g][4 * j + 3]});
+    asm volatile("" : "+v"(held[g]));   // what is kept are the chunks, not their elements
+  }
+  wait_vmcnt<0>();
+  const u32x4* const in_lds = (const u32x4*)kept + tid;   // a lane reads what its own copies brought
+#pragma unroll 4
+  for (int j = 0; j < kHeldInLds; ++j) most.add(in_lds[j * kResidentThreads]);
+  const bool numbers = !__syncthreads_or(most.has_nan());
+  float m = most.value();
+  if (!numbers) {   // the maximum of the numbers among them
+    m = 0.f;
+    for (int64_t i = 0; i < mine; ++i) m = Chunk<In>::amax(Chunk<In>::load(x, piece(i), tid), m);
+  }
+  if (b == 0) {
+    constexpr int64_t kPiece = Chunk<In>::kPer * kResidentThreads;
+    for (int64_t i = n / kPiece * kPiece + tid; i < n; i += kResidentThreads) m = __builtin_fmaxf(m, __builtin_fabsf(Load8<In>::one(x, i)));
+  }
+  m = workgroup_max<8>(m);
+  if (tid == 0) __hip_atomic_store(slots + b, __builtin_bit_cast(uint32_t, m), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+
+  // The values travel in the words themselves, so no order with other memory is needed.
+  uint32_t theirs = 0;
+  if (tid < blocks) {
+    const int64_t until = (int64_t)__builtin_amdgcn_s_memrealtime() + wait_ticks;
+    for (;;) {
+      theirs = __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (theirs != kUnset || (int64_t)__builtin_amdgcn_s_memrealtime() >= until) break;
+      __builtin_amdgcn_s_sleep(1);
+    }
+  }
+  if (!__syncthreads_and(theirs != kUnset)) return;
+  const float amax = workgroup_max<8>(__builtin_bit_cast(float, theirs)), scale = scale_of(amax), inv = 1.0f / scale;
+  if (tid == 0) {
+    slots[kResidentBlocks + b] = 1u;
+    if (b == 0) {
+      out[0] = scale;
+      out[1] = amax;
+    }
+  }
+  const auto store_all = [&](auto quotient, float inv, float more) __attribute__((always_inline)) {
+    constexpr Quotient kQuotient = decltype(quotient)::value;
+    // loops over registers by a scalar index: unrolled, these are tens of KB of code that run once
+#pragma unroll
+    for (int g = 0; g < kHeld / 8; ++g) {
+#pragma unroll 2
+      for (int j = 0; j < 8; ++j) {
+        const u32x4 a = {held[g][4 * j], held[g][4 * j + 1], held[g][4 * j + 2], held[g][4 * j + 3]};
+        if (8 * g + j < mine) Chunk<In>::template store<kQuotient>(q, piece(8 * g + j), tid, a, scale, inv, more);
+      }
+    }
+#pragma unroll 2
+    for (int j = 0; j < kHeldInLds; ++j)
+      if (kHeld + j < mine) Chunk<In>::template store<kQuotient>(q, piece(kHeld + j), tid, in_lds[j * kResidentThreads], scale, inv, more);
+  };
+  Factors f = {0.f, 0.f};
+  if constexpr (!std::is_same<In, float>::value)
+    if (numbers && markstein_ok(scale)) f = factors_for<In>(scale, inv);
+  if (!markstein_ok(scale)) {   // tiny or infinite scales
+    quantize_pieces<In, kDivide>(x, n, q, scale, inv, mine);
+  } else if constexpr (std::is_same<In, float>::value) {
+    store_all(std::integral_constant<Quotient, kCorrected>{}, inv, 0.f);
+  } else if (f.first != 0.f && f.more == 0.f) {
+    store_all(std::integral_constant<Quotient, kProduct>{}, f.first, 0.f);
+  } else if (f.first != 0.f) {
+    store_all(std::integral_constant<Quotient, kTwoProducts>{}, f.first, f.more);
+  } else {
+    quantize_pieces<In, kCorrected>(x, n, q, scale, inv, mine);
+  }
+  quantize_rest<In>(x, n, q, scale);
+}
+
+template <class In>
+__global__ __launch_bounds__(kResidentThreads) void quantize_left_kernel(const void* x, int64_t n, uint8_t* q, float* out, const uint32_t* slots) {
+  if (slots[kResidentBlocks + blockIdx.x]) return;
+  const float amax = workgroup_max<8>(threadIdx.x < gridDim.x ? __builtin_bit_cast(float, slots[threadIdx.x]) : 0.f);
+  const float scale = scale_of(amax), inv = 1.0f / scale;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    out[0] = scale;
+    out[1] = amax;
+  }
+  const int64_t mine = pieces_of<In>(n, blockIdx.x, gridDim.x);
+  if (markstein_ok(scale)) quantize_pieces<In, kCorrected>(x, n, q, scale, inv, mine);
+  else quantize_pieces<In, kDivide>(x, n, q, scale, inv, mine);
+  quantize_rest<In>(x, n, q, scale);
+}
+
+
+template <class In>
+int run_resident(const void* x, int64_t n, void* q, float* out, uint32_t* slots, hipStream_t stream) {
+  const char* wait = std::getenv("MI355_QUANTIZE_WAIT_US");   // for tests: 0 has the second kernel do what is left
+  const int64_t ticks = wait ? std::atoll(wait) * 100 : kWaitTicks;
+  const dim3 grid((unsigned)compute_units());   // at most kResidentBlocks (run)
+  hipLaunchKernelGGL(resident_init, dim3(1), dim3(2 * kResidentBlocks), 0, stream, slots);
+  hipLaunchKernelGGL((quantize_resident_kernel<In>), grid, dim3(kResidentThreads), 0, stream, x, n, (uint8_t*)q, out, slots, ticks);
+  hipLaunchKernelGGL((quantize_left_kernel<In>), grid, dim3(kResidentThreads), 0, stream, x, n, (uint8_t*)q, out, (const uint32_t*)slots);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
 template <class In>
 int run(const void* x, int64_t n, void* q, float* out, float* partial, int64_t partials, hipStream_t stream) {
   if (n * (int64_t)sizeof(typename Load8<In>::Element) <= kSmallBytes) {
     const int64_t want = (n / 8 + 1023) / 1024;
     hipLaunchKernelGGL((quantize_small_kernel<In>), dim3((unsigned)(want < 1 ? 1 : want)), dim3(1024), 0, stream, x, n, (uint8_t*)q, out);
     return hipGetLastError() == hipSuccess ? 0 : -1;
+  }
+  const int64_t bytes = n * (int64_t)sizeof(typename Load8<In>::Element);
+  if (bytes >= kResidentFrom && partial && partials >= 2 * kResidentBlocks) {
+    const int64_t cus = compute_units();
+    if (cus <= kResidentBlocks && bytes < cus * kResident * kResidentThreads * 16 + kResidentThreads * 16)   // whole pieces fit
+      return run_resident<In>(x, n, q, out, (uint32_t*)partial, stream);
   }
   const int64_t want = (n / 8 + 255) / 256;
   const int64_t most = n * (int64_t)sizeof(typename Load8<In>::Element) <= kL2Bytes ? kQuantizeBlocksInL2 : kQuantizeBlocks;

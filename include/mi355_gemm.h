@@ -161,7 +161,8 @@ int mi355_gemm_tn_noalloc(const void *A, const void *B, void *C,
  *
  * mi355_quantize_e4m3_scratch is the same with scratch memory (4-byte aligned, contents need not be
  * initialised, not shared with calls that may overlap) of mi355_quantize_e4m3_scratch_bytes(n) bytes,
- * which spares one of the three launches; with less, or NULL, it runs as mi355_quantize_e4m3 does.
+ * which spares one of the three launches, or for tensors that the chip holds (80 to 128 MiB) the second read of x; with less,
+ * or NULL, it runs as mi355_quantize_e4m3 does.
  */
 int mi355_quantize_e4m3(const void *x, int x_dtype, int64_t n, void *x_q,
                         float *scale_amax, void *stream);
