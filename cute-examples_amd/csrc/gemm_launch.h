@@ -122,6 +122,7 @@ struct SlicesAlternative {
   int64_t tile_rows, tile_cols, splits;
 };
 constexpr double kSlicesMaxProducts = 1.5e10, kSlicesMaxProductsAnyRows = 3e10;   // M * N * K; the rules were fitted below
+constexpr double kSlicesMaxOutputs = 2.5e6, kSlicesMaxOutputsAnyRows = 4e6;       // M * N, likewise
 int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other, double* route_us = nullptr);
 double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // the estimate of its shortest form, huge where the rule is not for
 int launch_slices(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);

@@ -360,7 +360,7 @@ bool on_this_route(const SlicesAlternative& other) { return other.streams || oth
 // one (M <= 16: 10-20 % faster here between 24 and 48 MiB, 4 % from there to 90).  MI355_RING_TILE, which forces a tile for
 // measurements, keeps problems off this kernel as well.
 double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
-  if (M <= 0 || N <= 0 || K <= 0 || (double)M * (double)N * (double)K > kSlicesMaxProducts) return 1e30;
+  if (M <= 0 || N <= 0 || K <= 0 || (double)M * (double)N * (double)K > kSlicesMaxProducts || (double)M * (double)N > kSlicesMaxOutputs) return 1e30;
   if ((double)N * (double)K * elem_bytes > (M <= 16 ? 48.0 : 32.0) * 1048576.0 || std::getenv("MI355_RING_TILE")) return 1e30;
   double us = 0;
   shortest_form(kForms, kFormCount, kDepth, M, N, ceil_div(K * elem_bytes, kRowBytes), false, 1.0, &us);
@@ -383,7 +383,8 @@ int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, cons
 
 // The other route of a product with rows of any alignment is `other` (or this kernel, whichever is shorter) behind a repacking of
 // `copied` bytes: us = 6.4 + 0.36 x MB + 0.75 x product + 0.25 x million outputs (296 problems, 11 % rms).  Taken from 0.97 of it:
-// 0.66 of the time before on average over those, as the better choice on each would leave, 4 of them 4-24 % slower.  Small 16-bit
+// 0.66 of the time before on average over those, as the better choice on each would leave, 4 of them 4-24 % slower; with more than four
+// million outputs, whose stores the estimate does not know, not at all (e4m3 4150 x 4115 x 174 32.5 us repacked, 40.9 as it is).  Small 16-bit
 // products (copied == 0) have none but one thread or a sixteenth of a wave per output, which was slower on all of 124 problems.
 int slices_any_rows_config(int64_t M, int64_t N, int64_t K, int elem_bytes, int alignment, int64_t copied, const SlicesAlternative& other) {
   if (M <= 0 || N <= 0 || K * elem_bytes < 16 || (double)M * (double)N * (double)K > kSlicesMaxProductsAnyRows) return -1;
@@ -392,6 +393,7 @@ int slices_any_rows_config(int64_t M, int64_t N, int64_t K, int elem_bytes, int 
   const int form = shortest_form(kAnyRowsForms, kAnyRowsFormCount, 1, M, N, ceil_div(K * elem_bytes, kRowBytes), false,
                                  alignment % 4 == 0 ? 1.0 : alignment % 2 == 0 ? 1.25 : 1.6, &us);
   if (copied == 0) return form;
+  if ((double)M * (double)N > kSlicesMaxOutputsAnyRows) return -1;
   slices_config(M, N, K, elem_bytes, false, other, &product);
   return us < 0.97 * (6.44 + 0.357e-6 * (double)copied + 0.751 * product + 0.25e-6 * (double)M * (double)N) ? form : -1;
 }
