@@ -565,7 +565,7 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
   };
   // Two launches where a cut spares a partly filled last round of workgroups, as for plain operands.
   bool along_m = false;
-  const int64_t first = mi355::ring_cut(M, N, K, 1, &along_m);
+  const int64_t first = mi355::ring_cut(M, N, K, 1, false, &along_m);
   if (first <= 0) return tiles_of_piece(0, M, 0, N);
   st = along_m ? tiles_of_piece(0, first, 0, N) : tiles_of_piece(0, M, 0, first);
   if (st != MI355_OK) return st;
@@ -630,7 +630,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
     // the other on the stream and through the same workspace.
     bool along_m = false;
-    const int64_t first = mi355::ring_cut(M, Np, K, es, &along_m);
+    const int64_t first = mi355::ring_cut(M, Np, K, es, true, &along_m);
     if (first > 0) {
       const int st = run_variant(A, B, C, along_m ? first : M, along_m ? N : first, K, lda, ldb, ldc, in_dtype, out_dtype, scale,
                                  scale_a, scale_b, v, kPiece, c_rows, workspace, workspace_bytes, s, mode);

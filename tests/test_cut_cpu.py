@@ -21,13 +21,26 @@ def covered(c, got, es):
     return len(rects)
 
 
-@pytest.mark.parametrize("M,N,K,in_dt", [(1000, 50257, 768, ac.BF16), (1000, 50260, 768, ac.F16), (1056, 26704, 2176, ac.BF16), (1509, 11192, 4864, ac.E4M3),
-                                         (6784, 2504, 2304, ac.BF16), (3748, 13208, 640, ac.BF16)])
+@pytest.mark.parametrize("M,N,K,in_dt", [(1000, 50257, 768, ac.BF16), (1000, 50260, 768, ac.F16), (2123, 8032, 1408, ac.BF16), (1509, 11192, 3200, ac.E4M3),
+                                         (6784, 2504, 1792, ac.BF16), (3748, 13208, 640, ac.BF16)])
 def test_cut(launches, M, N, K, in_dt):  # noqa: F811
     es = 1 if in_dt == ac.E4M3 else 2
     cases = [case(M, N, K, in_dt), case(M, N, K, in_dt, room=0) if N % 4 == 0 else case(M, N, K, in_dt, room=256), case(M, N, K, in_dt, noalloc=True)]
     for c, (st, _, got) in zip(cases, launches(cases)):
         assert st == ac.OK and covered(c, got, es) == 2, c
+
+
+def test_what_the_queries_call_one_launch_with_a_tail_split_is_one(launches):  # noqa: F811
+    """Its result is the tile variant's to the bit."""
+    abi, rng, tails = ac.load(), random.Random(4), 0
+    problems = [(4352, 4352, 4096), (1056, 26704, 2176), (6784, 2504, 2304)]
+    problems += [(rng.randint(1000, 7000), 4 * rng.randint(500, 3000), 64 * rng.randint(32, 90)) for _ in range(300)]
+    cases = [case(*p) for p in problems]
+    for p, c, (st, _, got) in zip(problems, cases, launches(cases)):
+        if abi.mi355_gemm_pieces(*p, ac.BF16, ac.AUTO, None, None) == 1 and ac.plan(abi, *p, ac.BF16)[4] > 0:
+            tails += 1
+            assert st == ac.OK and covered(c, got, 2) == 1, p
+    assert tails >= 20
 
 
 def test_halves_cover_random_problems(launches):  # noqa: F811
