@@ -257,14 +257,18 @@ __global__ __launch_bounds__(1024) void quantize_small_kernel(const void* x, int
 // Tensors of kResidentFrom bytes to what the chip holds, read once.  One workgroup per CU keeps its pieces of 8 KiB on the chip
 // between the maximum and the codes, 48 in registers (192 of a lane's 256) and 16 in LDS: 512 KiB per CU, 128 MiB in all.  Between the
 // two halves every workgroup waits for the maxima of all others, one word each in `slots`.  That they all run at the same time is how
-// the chip fills when nothing else does; it is not relied on: the wait is bounded, and a workgroup that gives up leaves its pieces to
-// quantize_left_kernel behind it, which finds nothing to do otherwise.
+// the chip fills when nothing else does; it is not relied on: the wait is bounded by about what the second read costs (40 us, ten
+// times the usual wait), and a workgroup that gives up leaves its pieces to quantize_left_kernel behind it, which finds nothing to do
+// otherwise.  A stream with a CU mask, where workgroups would always be waiting for others that cannot start, reads twice (has_all_cus;
+// bf16 8192 x 8192 on 255, 224 or 128 CUs 53 us, 115...119 this way, 275 with a bound of 200 us).  Beside other work, this against two
+// reads (us): two such quantisers on two streams 74 / 99 the pair, two beside a bf16 4096^3 product 170 / 190 in all, six beside products
+// of several rounds (8192^3, 8192^2 x 1024, 4352^2 x 4096, 8192 x 16384 x 256) 0.90...1.02 of the time in all, 2048 x 14336 x 4096 1.06...1.12.
 // bf16 8192 x 8192 (128 MiB) 53.4 -> 41.8 us, of which reading 20, waiting 4, codes 11 (19 with the corrected quotient, see factors_for),
 // the two small launches around it 5; 96 MiB 41.2 -> 34.6, 80 MiB 35.7 -> 31.1, 64 MiB 30.8 / 30.1, 32 MiB 16.6 / 23.8; fp32 128 MiB 52.7 ->
 // 40.3, 80 MiB 33.2 -> 30.2, 64 MiB 28.2 / 29.3; with a part of 224 MiB read twice 89.5 / 104.  fp8 layer 8192^3 421 -> 406 us.
 constexpr int kHeld = 48, kHeldInLds = 16, kResident = kHeld + kHeldInLds, kResidentThreads = 512, kResidentBlocks = 256;
 constexpr int64_t kResidentFrom = (int64_t)80 << 20;
-constexpr int64_t kWaitTicks = 20000;      // of the 100 MHz clock: 200 us
+constexpr int64_t kWaitTicks = 4000;       // of the 100 MHz clock: 40 us
 constexpr uint32_t kUnset = 0xffffffffu;   // no maximum: those are numbers, this is the pattern of a NaN
 typedef __attribute__((ext_vector_type(32))) uint32_t u32x32;
 
@@ -479,11 +483,22 @@ __global__ __launch_bounds__(kResidentThreads) void quantize_left_kernel(const v
   quantize_rest<In>(x, n, q, scale);
 }
 
+// Whether the stream's kernels may run on all `cus` compute units; false where that cannot be told.
+bool has_all_cus(hipStream_t stream, int64_t cus) {
+  uint32_t mask[32] = {};
+  if (hipExtStreamGetCUMask(stream, 32, mask) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  int64_t on = 0;
+  for (const uint32_t word : mask) on += __builtin_popcount(word);
+  return on >= cus;
+}
 
 template <class In>
 int run_resident(const void* x, int64_t n, void* q, float* out, uint32_t* slots, hipStream_t stream) {
-  const char* wait = std::getenv("MI355_QUANTIZE_WAIT_US");   // for tests: 0 has the second kernel do what is left
-  const int64_t ticks = wait ? std::atoll(wait) * 100 : kWaitTicks;
+  const char* wait = std::getenv("MI355_QUANTIZE_WAIT_US");   // for tests, up to the bound: 0 has the second kernel do what is left
+  const int64_t asked = wait ? std::atoll(wait) : kWaitTicks / 100, ticks = asked < kWaitTicks / 100 ? asked * 100 : kWaitTicks;
   const dim3 grid((unsigned)compute_units());   // at most kResidentBlocks (run)
   hipLaunchKernelGGL(resident_init, dim3(1), dim3(2 * kResidentBlocks), 0, stream, slots);
   hipLaunchKernelGGL((quantize_resident_kernel<In>), grid, dim3(kResidentThreads), 0, stream, x, n, (uint8_t*)q, out, slots, ticks);
@@ -501,7 +516,8 @@ int run(const void* x, int64_t n, void* q, float* out, float* partial, int64_t p
   const int64_t bytes = n * (int64_t)sizeof(typename Load8<In>::Element);
   if (bytes >= kResidentFrom && partial && partials >= 2 * kResidentBlocks) {
     const int64_t cus = compute_units();
-    if (cus <= kResidentBlocks && bytes < cus * kResident * kResidentThreads * 16 + kResidentThreads * 16)   // whole pieces fit
+    if (cus <= kResidentBlocks && bytes < cus * kResident * kResidentThreads * 16 + kResidentThreads * 16 &&   // whole pieces fit
+        has_all_cus(stream, cus))
       return run_resident<In>(x, n, q, out, (uint32_t*)partial, stream);
   }
   const int64_t want = (n / 8 + 255) / 256;
