@@ -535,7 +535,8 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
   }
   // The tile kernel on rows [m0, m0 + m) of A and rows [n0, n0 + n) of B (multiples of 256 but for the last).
   // K split or tail split when the rest of the workspace holds the partial results (optional, as
-  // for the other tiled kernels: without it the tiles run unsplit).
+  // for the other tiled kernels: without it the tiles run unsplit), and not where the cut is one of unsplit pieces.
+  const mi355::RingCut cut = mi355::ring_cut(M, N, K, 1, false);
   const auto tiles_of_piece = [&](int64_t m0, int64_t m, int64_t n0, int64_t n) {
     mi355::GemmArgs p = g;
     p.A = (const uint8_t*)A_q + m0 * lda;
@@ -552,7 +553,7 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
     }
     int splits, tail_tiles, tail_splits;
     const size_t partial = mx_partial_bytes(m, n, K, &splits, &tail_tiles, &tail_splits);
-    if (partial && workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= used + partial) {
+    if (!cut.unsplit && partial && workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= used + partial) {
       p.partial = (float*)((uint8_t*)workspace + used);  // used is a multiple of 1024
       p.splits = splits;
       p.tail_tiles = tail_tiles;
@@ -564,12 +565,11 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
     return mi355::launch_tile_ring_mx(p, out_dtype, tile, s) == 0 ? (int)MI355_OK : (int)MI355_ERR_LAUNCH;
   };
   // Two launches where a cut spares a partly filled last round of workgroups, as for plain operands.
-  bool along_m = false;
-  const int64_t first = mi355::ring_cut(M, N, K, 1, false, &along_m);
+  const int64_t first = cut.extent;
   if (first <= 0) return tiles_of_piece(0, M, 0, N);
-  st = along_m ? tiles_of_piece(0, first, 0, N) : tiles_of_piece(0, M, 0, first);
+  st = cut.along_m ? tiles_of_piece(0, first, 0, N) : tiles_of_piece(0, M, 0, first);
   if (st != MI355_OK) return st;
-  return along_m ? tiles_of_piece(first, M - first, 0, N) : tiles_of_piece(0, M, first, N - first);
+  return cut.along_m ? tiles_of_piece(first, M - first, 0, N) : tiles_of_piece(0, M, first, N - first);
 }
 
 int mi355_gemm_tn(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K,
@@ -612,8 +612,9 @@ namespace {
 //   kRowsRagged      of any 2-byte alignment (GemmArgs::c_ragged; BASIC and SKINNY only)
 enum CRows { kRowsAligned, kRowsRagged };
 
-// Whose choice the variant is: the caller's, the library's, or the library's for a piece of a problem that it has cut in two.
-enum Choice { kExplicit, kAuto, kPiece };
+// Whose choice the variant is: the caller's, the library's, or the library's for a piece of a problem that it has cut in two (with
+// kUnsplitPiece one that is not to split K, see RingCut).
+enum Choice { kExplicit, kAuto, kPiece, kUnsplitPiece };
 
 // One problem on the variant v (resolved, not AUTO).  kAuto: the caller left the choice to the library, which may then
 // cut the problem in two or leave the streaming kernel for the tile kernel.  The plan is that of N rounded up to 4.
@@ -629,17 +630,19 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     // Two launches where the planner finds a cut that spares a partly filled last round (ring_cut): each
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
     // the other on the stream and through the same workspace.
-    bool along_m = false;
-    const int64_t first = mi355::ring_cut(M, Np, K, es, true, &along_m);
+    const mi355::RingCut cut = mi355::ring_cut(M, Np, K, es, true);
+    const int64_t first = cut.extent;
+    const bool along_m = cut.along_m;
+    const Choice piece = cut.unsplit ? kUnsplitPiece : kPiece;
     if (first > 0) {
       const int st = run_variant(A, B, C, along_m ? first : M, along_m ? N : first, K, lda, ldb, ldc, in_dtype, out_dtype, scale,
-                                 scale_a, scale_b, v, kPiece, c_rows, workspace, workspace_bytes, s, mode);
+                                 scale_a, scale_b, v, piece, c_rows, workspace, workspace_bytes, s, mode);
       if (st != MI355_OK) return st;
       const uint8_t* a2 = (const uint8_t*)A + (along_m ? first * lda * es : 0);
       const uint8_t* b2 = (const uint8_t*)B + (along_m ? 0 : first * ldb * es);
       uint8_t* c2 = (uint8_t*)C + (along_m ? first * ldc : first) * 2;   // 16-bit output
       return run_variant(a2, b2, c2, along_m ? M - first : M, along_m ? N : N - first, K, lda, ldb, ldc, in_dtype, out_dtype,
-                         scale, scale_a, scale_b, v, kPiece, c_rows, workspace, workspace_bytes, s, mode);
+                         scale, scale_a, scale_b, v, piece, c_rows, workspace, workspace_bytes, s, mode);
     }
   }
   mi355::GemmArgs g;
@@ -681,7 +684,7 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     rc = mi355::launch_stream(g, in_dtype, out_dtype, splits, workspace, s);
   } else if (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_PINGPONG) {
     const int tile = v == MI355_VARIANT_PINGPONG ? 256 : mi355::ring_tile_edge(M, Np, K, es);
-    if (v == MI355_VARIANT_BASIC) {
+    if (v == MI355_VARIANT_BASIC && choice != kUnsplitPiece) {
       // Both kinds of K split are optional for this kernel: without a (large enough, aligned)
       // workspace a lenient call runs the same tiles unsplit, slower but with the same result contract.
       const auto usable = [&](size_t need) {
@@ -692,14 +695,14 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
       if (splits > 1) {
         const size_t need = (size_t)splits * (size_t)M * (size_t)Np * sizeof(float);
         if (usable(need)) g.splits = splits;
-        else if (strict && choice != kPiece) return MI355_ERR_SCRATCH;
+        else if (strict) return MI355_ERR_SCRATCH;
       } else {
         int tail_tiles, tail_splits;
         const size_t need = mi355::ring_tail(M, Np, K, es, &tail_tiles, &tail_splits);
         if (usable(need)) {
           g.tail_tiles = tail_tiles;
           g.tail_splits = tail_splits;
-        } else if (strict && need && choice != kPiece) {   // a piece's split is no part of what the query counts on (ring_cut)
+        } else if (strict && need) {
           return MI355_ERR_SCRATCH;
         }
       }

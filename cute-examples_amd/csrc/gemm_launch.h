@@ -78,9 +78,14 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
-// The cut that a call with MI355_VARIANT_AUTO makes: that one, or another that wants no more workspace (tail_splits: not where one
+// The cut that a call with MI355_VARIANT_AUTO makes: that one, or another whose pieces want no workspace (tail_splits: not where one
 // launch would have a tail split).
-int64_t ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits, bool* along_m);
+struct RingCut {
+  int64_t extent;      // the first piece's, 0 for one launch
+  bool along_m;
+  bool unsplit;        // not ring_first_piece's: the workspace query knows nothing of the pieces, which run without splits of K
+};
+RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits);
 double ring_shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // estimate of the single-group kernel's plan
 // Whether MI355_VARIANT_AUTO computes a C whose rows start at odd 2-byte addresses into a padded copy that is then copied out (if
 // there is memory for it) instead of storing it directly.

@@ -271,26 +271,27 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
 }
 
 // The cut that MI355_VARIANT_AUTO makes: ring_first_piece's (which the queries report), or one whose first piece is nearly whole
-// rounds -- as many tile columns (rows) as r rounds have room for -- and whose rest needs no workspace, where that is estimated to be
-// shorter, the second launch counted as there.  Problems of a few tiles more than whole rounds have it, and of any number of k-steps:
-// bf16 1000 x 50257 x 768 (3.08 rounds) 118 -> 97 us, 2123 x 8032 x 1408 (1.13) 64 -> 48, e4m3 1509 x 11192 x 3200 (1.03) 66 -> 53.  Of 90
+// rounds -- as many tile columns (rows) as r rounds have room for -- and whose pieces run without splits of K, whatever the workspace, where
+// that is estimated to be shorter, the second launch counted as there.  Problems of a few tiles more than whole rounds have it, and of
+// any number of k-steps: bf16 1000 x 50257 x 768 (3.08 rounds) 118 -> 97 us, 2123 x 8032 x 1408 (1.13) 64 -> 48, e4m3 1509 x 11192 x 3200 (1.03) 66 -> 53.  Of 90
 // random problems of 1.03...5 rounds and 2...64 k-steps 11 are cut so, in 0.94 of the time on average, none slower by more than 1 %
 // (counted with 2 us 17 are, one of them 3 % slower: bf16 2523 x 20680 x 448 69 -> 71 us).  A plain problem that the queries describe
 // as one launch with a tail split (tail_splits) stays one: its result is MI355_VARIANT_BASIC's to the bit, and the cut would add in
 // another order (a price: bf16 1056 x 26704 x 2176 149 us, cut 117).  Beyond 64 k-steps ring_first_piece's limit of rounds.
-int64_t ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits, bool* along_m) {
-  int64_t extent = ring_first_piece(M, N, K, elem_bytes, along_m);
-  if (std::getenv("MI355_ONE_PIECE") || std::getenv("MI355_RING_TILE")) return extent;
-  if (tail_splits && extent == 0) {
+RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits) {
+  RingCut cut = {0, false, false};
+  cut.extent = ring_first_piece(M, N, K, elem_bytes, &cut.along_m);
+  if (std::getenv("MI355_ONE_PIECE") || std::getenv("MI355_RING_TILE")) return cut;
+  if (tail_splits && cut.extent == 0) {
     int tiles, splits;
-    if (ring_tail(M, N, K, elem_bytes, &tiles, &splits) > 0) return 0;
+    if (ring_tail(M, N, K, elem_bytes, &tiles, &splits) > 0) return cut;
   }
   const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, steps = k_steps_of(K, elem_bytes);
-  if (tm * tn <= kCuSlots || (tm * tn) % kCuSlots == 0 || tm * tn > 5 * kCuSlots || (steps > 64 && 10 * tm * tn > 34 * kCuSlots)) return extent;
+  if (tm * tn <= kCuSlots || (tm * tn) % kCuSlots == 0 || tm * tn > 5 * kCuSlots || (steps > 64 && 10 * tm * tn > 34 * kCuSlots)) return cut;
   double best = shortest_us(M, N, K, elem_bytes);
-  if (extent > 0) {
-    const int64_t rest_m = *along_m ? M - extent : M, rest_n = *along_m ? N : N - extent;
-    best = shortest_us(*along_m ? extent : M, *along_m ? N : extent, K, elem_bytes) + shortest_us(rest_m, rest_n, K, elem_bytes) + kSecondLaunchUs;
+  if (cut.extent > 0) {
+    const int64_t rest_m = cut.along_m ? M - cut.extent : M, rest_n = cut.along_m ? N : N - cut.extent;
+    best = shortest_us(cut.along_m ? cut.extent : M, cut.along_m ? N : cut.extent, K, elem_bytes) + shortest_us(rest_m, rest_n, K, elem_bytes) + kSecondLaunchUs;
   }
   for (int axis = 0; axis < 2; ++axis) {
     const int64_t across = axis == 0 ? tm : tn, along = axis == 0 ? tn : tm;   // axis 0: cut N, axis 1: cut M
@@ -302,12 +303,11 @@ int64_t ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_spli
       const double e = shortest_unsplit_us(axis == 0 ? M : c * 256, axis == 0 ? c * 256 : N, K, elem_bytes) + (tiles < slices ? tiles : slices) + kSecondLaunchUs;
       if (e < best) {
         best = e;
-        extent = c * 256;
-        *along_m = axis == 1;
+        cut = {c * 256, axis == 1, true};
       }
     }
   }
-  return extent;
+  return cut;
 }
 
 // Rows of C that start at odd 2-byte addresses are stored directly (tile_store.h), but for a region where they go through a padded

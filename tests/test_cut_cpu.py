@@ -52,3 +52,23 @@ def test_halves_cover_random_problems(launches):  # noqa: F811
         cases.append(case(M, N, K, in_dt, room=rng.choice([0, None])))
     seen = {covered(c, got, 1 if c["in_dt"] == ac.E4M3 else 2) for c, (st, _, got) in zip(cases, launches(cases)) if st == ac.OK}
     assert seen == {1, 2}
+
+
+def launched(got):
+    """What was launched, wherever the workspace lies."""
+    return [(name, [v[k] for k in ("M", "N", "K", "lda", "ldb", "ldc", "A", "B", "C", "c_ragged", "splits", "tail_tiles")] if "gemm_tn_" in name else None) for name, v in got]
+
+
+def test_halves_do_not_depend_on_the_workspace(launches):  # noqa: F811
+    """The same kernels and splits, so the same sums, with the room that the query asks for, with more, and without allocation."""
+    rng = random.Random(6)
+    problems = [(3518, 14380, 7168, ac.BF16), (2167, 21868, 9792, ac.BF16), (3094, 16012, 12928, ac.BF16), (4139, 12620, 12224, ac.E4M3)]
+    problems += [(int(2 ** rng.uniform(9, 13.2)), int(2 ** rng.uniform(9, 15.6)) // 4 * 4, int(2 ** rng.uniform(10, 13.8)) // 16 * 16, rng.choice([ac.BF16, ac.E4M3]))
+                 for _ in range(800)]
+    answers = [launches([case(*p, room=room, noalloc=noalloc) for p in problems]) for room, noalloc in ((None, False), (1 << 30, False), (None, True))]
+    cut = 0
+    for p, (st, _, got), more, without in zip(problems, *answers):
+        assert (st, more[0], without[0]) == (ac.OK, ac.OK, ac.OK)
+        assert launched(got) == launched(more[2]) == launched(without[2]), p
+        cut += sum(matrix_core(name) for name, _ in got) > 1
+    assert cut >= 60
