@@ -535,8 +535,9 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
   }
   // The tile kernel on rows [m0, m0 + m) of A and rows [n0, n0 + n) of B (multiples of 256 but for the last).
   // K split or tail split when the rest of the workspace holds the partial results (optional, as
-  // for the other tiled kernels: without it the tiles run unsplit), and not where the cut is one of unsplit pieces.
-  const mi355::RingCut cut = mi355::ring_cut(M, N, K, 1, false);
+  // for the other tiled kernels: without it the tiles run unsplit).
+  const size_t room = mi355_gemm_mx_workspace_bytes(M, N, K, 1);
+  const mi355::RingCut cut = mi355::ring_cut(M, N, K, 1, false, true, room);
   const auto tiles_of_piece = [&](int64_t m0, int64_t m, int64_t n0, int64_t n) {
     mi355::GemmArgs p = g;
     p.A = (const uint8_t*)A_q + m0 * lda;
@@ -547,19 +548,26 @@ int mi355_gemm_tn_mxfp8(const void* A_q, const void* B_q, void* C, int64_t M, in
     p.M = m;
     p.N = n;
     p.c_streams = c_streams(m, n, K, 1);
+    mi355::CutPiece piece = {};
+    if (cut.own) piece = mi355::cut_piece(m, n, K, 1, true, room);
     if (m != M || n != N) {
-      const int form = few_outputs(m, n, K, 1, true, false);
+      const int form = cut.own ? piece.slices : few_outputs(m, n, K, 1, true, false);
       if (form >= 0) return mi355::launch_slices(p, MI355_E4M3, out_dtype, form, s) == 0 ? (int)MI355_OK : (int)MI355_ERR_LAUNCH;
     }
     int splits, tail_tiles, tail_splits;
-    const size_t partial = mx_partial_bytes(m, n, K, &splits, &tail_tiles, &tail_splits);
-    if (!cut.unsplit && partial && workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= used + partial) {
+    size_t partial = mx_partial_bytes(m, n, K, &splits, &tail_tiles, &tail_splits);
+    if (cut.own) {
+      splits = piece.splits;
+      tail_tiles = 0;
+      partial = splits > 1 ? (size_t)splits * (size_t)m * (size_t)n * sizeof(float) : 0;
+    }
+    if (partial && workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= used + partial) {
       p.partial = (float*)((uint8_t*)workspace + used);  // used is a multiple of 1024
       p.splits = splits;
       p.tail_tiles = tail_tiles;
       p.tail_splits = tail_splits;
     }
-    const int tile = mi355::ring_tile_edge(m, n, K, 1, true);
+    const int tile = cut.own ? piece.tile : mi355::ring_tile_edge(m, n, K, 1, true);
     p.tiles_m = (m + mi355::ring_tile_rows(tile) - 1) / mi355::ring_tile_rows(tile);
     p.tiles_n = (n + mi355::ring_tile_cols(tile) - 1) / mi355::ring_tile_cols(tile);
     return mi355::launch_tile_ring_mx(p, out_dtype, tile, s) == 0 ? (int)MI355_OK : (int)MI355_ERR_LAUNCH;
@@ -613,8 +621,8 @@ namespace {
 enum CRows { kRowsAligned, kRowsRagged };
 
 // Whose choice the variant is: the caller's, the library's, or the library's for a piece of a problem that it has cut in two (with
-// kUnsplitPiece one that is not to split K, see RingCut).
-enum Choice { kExplicit, kAuto, kPiece, kUnsplitPiece };
+// kOwnPiece as cut_piece says, without splits of K).
+enum Choice { kExplicit, kAuto, kPiece, kOwnPiece };
 
 // One problem on the variant v (resolved, not AUTO).  kAuto: the caller left the choice to the library, which may then
 // cut the problem in two or leave the streaming kernel for the tile kernel.  The plan is that of N rounded up to 4.
@@ -625,7 +633,9 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
   const int es = elem_bytes(in_dtype);
   const int64_t Np = mi355::partial_columns(N);
   const bool from_auto = choice == kAuto;
-  const int config = choice != kExplicit && (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_SKINNY) ? few_outputs(M, Np, K, es, false, v == MI355_VARIANT_SKINNY) : -1;
+  mi355::CutPiece piece = {};
+  if (choice == kOwnPiece) piece = mi355::cut_piece(M, Np, K, es, false, 0);
+  const int config = choice == kOwnPiece ? piece.slices : choice != kExplicit && (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_SKINNY) ? few_outputs(M, Np, K, es, false, v == MI355_VARIANT_SKINNY) : -1;
   if (config < 0 && from_auto && v == MI355_VARIANT_BASIC) {
     // Two launches where the planner finds a cut that spares a partly filled last round (ring_cut): each
     // piece is the single-group kernel's problem of its own, with its own tile, splits and store policy, one after
@@ -633,16 +643,16 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     const mi355::RingCut cut = mi355::ring_cut(M, Np, K, es, true);
     const int64_t first = cut.extent;
     const bool along_m = cut.along_m;
-    const Choice piece = cut.unsplit ? kUnsplitPiece : kPiece;
+    const Choice half = cut.own ? kOwnPiece : kPiece;
     if (first > 0) {
       const int st = run_variant(A, B, C, along_m ? first : M, along_m ? N : first, K, lda, ldb, ldc, in_dtype, out_dtype, scale,
-                                 scale_a, scale_b, v, piece, c_rows, workspace, workspace_bytes, s, mode);
+                                 scale_a, scale_b, v, half, c_rows, workspace, workspace_bytes, s, mode);
       if (st != MI355_OK) return st;
       const uint8_t* a2 = (const uint8_t*)A + (along_m ? first * lda * es : 0);
       const uint8_t* b2 = (const uint8_t*)B + (along_m ? 0 : first * ldb * es);
       uint8_t* c2 = (uint8_t*)C + (along_m ? first * ldc : first) * 2;   // 16-bit output
       return run_variant(a2, b2, c2, along_m ? M - first : M, along_m ? N : N - first, K, lda, ldb, ldc, in_dtype, out_dtype,
-                         scale, scale_a, scale_b, v, piece, c_rows, workspace, workspace_bytes, s, mode);
+                         scale, scale_a, scale_b, v, half, c_rows, workspace, workspace_bytes, s, mode);
     }
   }
   mi355::GemmArgs g;
@@ -683,8 +693,8 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
     g.tiles_m = g.tiles_n = 0;
     rc = mi355::launch_stream(g, in_dtype, out_dtype, splits, workspace, s);
   } else if (v == MI355_VARIANT_BASIC || v == MI355_VARIANT_PINGPONG) {
-    const int tile = v == MI355_VARIANT_PINGPONG ? 256 : mi355::ring_tile_edge(M, Np, K, es);
-    if (v == MI355_VARIANT_BASIC && choice != kUnsplitPiece) {
+    const int tile = v == MI355_VARIANT_PINGPONG ? 256 : choice == kOwnPiece ? piece.tile : mi355::ring_tile_edge(M, Np, K, es);
+    if (v == MI355_VARIANT_BASIC && choice != kOwnPiece) {
       // Both kinds of K split are optional for this kernel: without a (large enough, aligned)
       // workspace a lenient call runs the same tiles unsplit, slower but with the same result contract.
       const auto usable = [&](size_t need) {

@@ -78,14 +78,23 @@ int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scal
 // Whether MI355_VARIANT_AUTO runs the problem as two launches of the single-group kernel: the first piece's extent
 // along N (along M with *along_m set), or 0 for one launch.  Pure host heuristic; plain operands only.
 int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* along_m);
-// The cut that a call with MI355_VARIANT_AUTO makes: that one, or another whose pieces want no workspace (tail_splits: not where one
-// launch would have a tail split).
+// The cut that a call with MI355_VARIANT_AUTO makes: that one, or one of its own, whose pieces run as cut_piece says.  tail_splits: no
+// cut of its own where one launch would have a tail split.  room: bytes of workspace that the query counts on all the same, which the
+// pieces of its own may use for a split of K.
 struct RingCut {
-  int64_t extent;      // the first piece's, 0 for one launch
+  int64_t extent;   // the first piece's, 0 for one launch
   bool along_m;
-  bool unsplit;        // not ring_first_piece's: the workspace query knows nothing of the pieces, which run without splits of K
+  bool own;         // not ring_first_piece's
 };
-RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits);
+RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits, bool block_scaled = false, size_t room = 0);
+// What a piece of such a cut runs on, and the estimate of it that the cut was made by.
+struct CutPiece {
+  int tile;      // as ring_tile_edge's
+  int splits;    // of K
+  int slices;    // the form of gemm_tn_slices instead of it, or -1
+  double us;
+};
+CutPiece cut_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scaled, size_t room);
 double ring_shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // estimate of the single-group kernel's plan
 // Whether MI355_VARIANT_AUTO computes a C whose rows start at odd 2-byte addresses into a padded copy that is then copied out (if
 // there is memory for it) instead of storing it directly.
@@ -130,7 +139,7 @@ struct SlicesAlternative {
 constexpr double kSlicesMaxProducts = 1.5e10, kSlicesMaxProductsAnyRows = 3e10;   // M * N * K; the rules were fitted below
 constexpr double kSlicesMaxOutputs = 2.5e6, kSlicesMaxOutputsAnyRows = 4e6;       // M * N, likewise
 int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, const SlicesAlternative& other, double* route_us = nullptr);
-double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // the estimate of its shortest form, huge where the rule is not for
+double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, int* form);   // its shortest form's estimate, huge (and -1) where the rule is not for
 int launch_slices(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);
 int slices_any_rows_config(int64_t M, int64_t N, int64_t K, int elem_bytes, int alignment, int64_t copied, const SlicesAlternative& other);
 int launch_slices_any_rows(const GemmArgs& g, int in_dtype, int out_dtype, int config, hipStream_t stream);

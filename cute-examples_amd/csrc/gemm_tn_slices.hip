@@ -359,11 +359,12 @@ bool on_this_route(const SlicesAlternative& other) { return other.streams || oth
 // Rows of B of more than 32 MiB (48 MiB up to 16 rows of A) are left to the streaming kernel, which HBM bounds there as it would this
 // one (M <= 16: 10-20 % faster here between 24 and 48 MiB, 4 % from there to 90).  MI355_RING_TILE, which forces a tile for
 // measurements, keeps problems off this kernel as well.
-double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
+double slices_us(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, int* form) {
+  *form = -1;
   if (M <= 0 || N <= 0 || K <= 0 || (double)M * (double)N * (double)K > kSlicesMaxProducts || (double)M * (double)N > kSlicesMaxOutputs) return 1e30;
   if ((double)N * (double)K * elem_bytes > (M <= 16 ? 48.0 : 32.0) * 1048576.0 || std::getenv("MI355_RING_TILE")) return 1e30;
   double us = 0;
-  shortest_form(kForms, kFormCount, kDepth, M, N, ceil_div(K * elem_bytes, kRowBytes), false, 1.0, &us);
+  *form = shortest_form(kForms, kFormCount, kDepth, M, N, ceil_div(K * elem_bytes, kRowBytes), mx, 1.0, &us);
   return us;
 }
 
@@ -373,9 +374,9 @@ int slices_config(int64_t M, int64_t N, int64_t K, int elem_bytes, bool mx, cons
   const int64_t steps = ceil_div(K * elem_bytes, kRowBytes);
   const double limit = on_this_route(other) ? other_us(other, M, N, steps) : ring_shortest_us(M, N, K, elem_bytes);
   if (route_us) *route_us = limit;
-  if (!on_this_route(other) || slices_us(M, N, K, elem_bytes) >= 1e30) return -1;
-  double us = 0;
-  const int form = shortest_form(kForms, kFormCount, kDepth, M, N, steps, mx, 1.0, &us);
+  if (!on_this_route(other)) return -1;
+  int form;
+  const double us = slices_us(M, N, K, elem_bytes, mx, &form);
   if (us >= 0.85 * limit) return -1;
   if (route_us) *route_us = us;
   return form;

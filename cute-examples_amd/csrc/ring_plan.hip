@@ -148,12 +148,6 @@ double shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
   return a < b ? (a < c ? a : c) : (b < c ? b : c);
 }
 
-double shortest_unsplit_us(int64_t M, int64_t N, int64_t K, int elem_bytes) {
-  const double a = estimate_us(256, M, N, K, elem_bytes, 1.0, false), b = estimate_us(kRingTile256x128, M, N, K, elem_bytes, 1.0, false),
-               c = estimate_us(128, M, N, K, elem_bytes, tiles_of(M, N, 128) <= kCuSlots && k_steps_of(K, elem_bytes) >= kShortSteps ? 0.82 : 1.0, false);
-  return a < b ? (a < c ? a : c) : (b < c ? b : c);
-}
-
 constexpr double kSecondLaunchUs = 3.0;
 
 }  // namespace
@@ -270,15 +264,44 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
   return extent;
 }
 
+// The tile of the shortest estimate without splits of K, a larger one being preferred within 2 % as in ring_tile_edge; or that
+// function's tile with its splits where there is room for them and they are shorter; or gemm_tn_slices where its own rule takes it
+// instead of the tile or its estimate is the shortest.
+CutPiece cut_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scaled, size_t room) {
+  const int64_t steps = k_steps_of(K, elem_bytes);
+  const int split_tile = ring_tile_edge(M, N, K, elem_bytes, block_scaled), splits = uniform_splits(tiles_of(M, N, split_tile), steps);
+  const bool may_split = splits > 1 && (size_t)splits * (size_t)M * (size_t)N * sizeof(float) <= room;
+  const bool single_round = tiles_of(M, N, 128) <= kCuSlots && steps >= kShortSteps;
+  // (Block scales have no nine-slot ring; beside a split that there is room for, the factor would keep the small tile ahead wrongly.)
+  const double e256 = estimate_us(256, M, N, K, elem_bytes, 1.0, false), e2 = estimate_us(kRingTile256x128, M, N, K, elem_bytes, 1.0, false),
+               e128 = estimate_us(128, M, N, K, elem_bytes, single_round && !(block_scaled && may_split) ? 0.82 : 1.0, false);
+  CutPiece p = {0, 1, -1, e256 < e128 ? (e256 < e2 ? e256 : e2) : (e128 < e2 ? e128 : e2)};
+  p.tile = e256 <= 1.02 * p.us ? 256 : e2 <= 1.02 * p.us ? kRingTile256x128 : single_round && !block_scaled ? kRingTile128DeepPlain : 128;
+  if (may_split) {
+    const double e = estimate_us(split_tile, M, N, K, elem_bytes);
+    if (e < p.us) p = {split_tile, splits, -1, e};
+  }
+  int form;
+  const double us = slices_us(M, N, K, elem_bytes, block_scaled, &form);
+  if (us < p.us || slices_config(M, N, K, elem_bytes, block_scaled, {false, ring_tile_rows(p.tile), ring_tile_cols(p.tile), p.splits}) >= 0) {
+    p.slices = form;
+    p.us = us < p.us ? us : p.us;   // what its rule takes is no longer than the tile
+  }
+  return p;
+}
+
 // The cut that MI355_VARIANT_AUTO makes: ring_first_piece's (which the queries report), or one whose first piece is nearly whole
-// rounds -- as many tile columns (rows) as r rounds have room for -- and whose pieces run without splits of K, whatever the workspace, where
-// that is estimated to be shorter, the second launch counted as there.  Problems of a few tiles more than whole rounds have it, and of
-// any number of k-steps: bf16 1000 x 50257 x 768 (3.08 rounds) 118 -> 97 us, 2123 x 8032 x 1408 (1.13) 64 -> 48, e4m3 1509 x 11192 x 3200 (1.03) 66 -> 53.  Of 90
-// random problems of 1.03...5 rounds and 2...64 k-steps 11 are cut so, in 0.94 of the time on average, none slower by more than 1 %
-// (counted with 2 us 17 are, one of them 3 % slower: bf16 2523 x 20680 x 448 69 -> 71 us).  A plain problem that the queries describe
-// as one launch with a tail split (tail_splits) stays one: its result is MI355_VARIANT_BASIC's to the bit, and the cut would add in
-// another order (a price: bf16 1056 x 26704 x 2176 149 us, cut 117).  Beyond 64 k-steps ring_first_piece's limit of rounds.
-RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits) {
+// rounds -- as many tile columns (rows) as r rounds have room for -- and whose pieces run as cut_piece says, where that is estimated to
+// be shorter, the second launch counted as there.  Problems of a few tiles more than whole rounds have it, and of any number of k-steps:
+// bf16 1000 x 50257 x 768 (3.08 rounds) 118 -> 97 us, 2123 x 8032 x 1408 (1.13) 64 -> 48, e4m3 1509 x 11192 x 3200 (1.03) 66 -> 53.
+// Of 12000 random plain problems of 1.03...5 rounds 18 % are cut at all, 5 % by ring_first_piece alone.  70 of them took 0.88 of the time on average,
+// five 3-8 % more (bf16 2524 x 6793 x 528 34.5 -> 37.3 us, 1591 x 40960 x 2176 229 -> 246).  60 block-scaled ones 0.94, one 2 % more.
+// While the price was of other tiles than those launched (whose plan had counted on splits of K), 85 plain problems took 0.91 of the
+// uncut time, now 0.865; 60 block-scaled ones 0.97, now 0.92, four of them up to 5 % slower than with splits in room meant for others.
+// A plain problem that the queries describe as one launch with a tail split (tail_splits) stays one: its result is
+// MI355_VARIANT_BASIC's to the bit, and the cut would add in another order (a price: bf16 1056 x 26704 x 2176 149 us, cut 117).
+// Beyond 64 k-steps ring_first_piece's limit of rounds.
+RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits, bool block_scaled, size_t room) {
   RingCut cut = {0, false, false};
   cut.extent = ring_first_piece(M, N, K, elem_bytes, &cut.along_m);
   if (std::getenv("MI355_ONE_PIECE") || std::getenv("MI355_RING_TILE")) return cut;
@@ -286,6 +309,7 @@ RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_spli
     int tiles, splits;
     if (ring_tail(M, N, K, elem_bytes, &tiles, &splits) > 0) return cut;
   }
+  const RingCut reported = cut;
   const int64_t tm = (M + 255) / 256, tn = (N + 255) / 256, steps = k_steps_of(K, elem_bytes);
   if (tm * tn <= kCuSlots || (tm * tn) % kCuSlots == 0 || tm * tn > 5 * kCuSlots || (steps > 64 && 10 * tm * tn > 34 * kCuSlots)) return cut;
   double best = shortest_us(M, N, K, elem_bytes);
@@ -299,11 +323,12 @@ RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_spli
       const int64_t c = r * kCuSlots / across;
       if (c <= 0 || c >= along) continue;
       const int64_t rest_m = axis == 0 ? M : M - c * 256, rest_n = axis == 0 ? N - c * 256 : N;
-      const double tiles = shortest_unsplit_us(rest_m, rest_n, K, elem_bytes), slices = slices_us(rest_m, rest_n, K, elem_bytes);
-      const double e = shortest_unsplit_us(axis == 0 ? M : c * 256, axis == 0 ? c * 256 : N, K, elem_bytes) + (tiles < slices ? tiles : slices) + kSecondLaunchUs;
+      const double e = cut_piece(axis == 0 ? M : c * 256, axis == 0 ? c * 256 : N, K, elem_bytes, block_scaled, room).us +
+                       cut_piece(rest_m, rest_n, K, elem_bytes, block_scaled, room).us + kSecondLaunchUs;
       if (e < best) {
         best = e;
-        cut = {c * 256, axis == 1, true};
+        if (c * 256 != reported.extent || (axis == 1) != reported.along_m) cut = {c * 256, axis == 1, true};
+        else cut = reported;
       }
     }
   }

@@ -1,5 +1,6 @@
 """Problems of a few tiles more than whole rounds: cut in two by a call, whatever the number of k-steps; what each half is, on the CPU."""
 import random
+import re
 
 import pytest
 
@@ -72,3 +73,21 @@ def test_halves_do_not_depend_on_the_workspace(launches):  # noqa: F811
         assert launched(got) == launched(more[2]) == launched(without[2]), p
         cut += sum(matrix_core(name) for name, _ in got) > 1
     assert cut >= 60
+
+
+def test_a_half_without_splits_has_tiles_for_that(launches):  # noqa: F811
+    """Not the large tiles of a plan that would have cut K, on less than half of the compute units."""
+    rng = random.Random(8)
+    problems = [(3094, 16012, 12928, ac.BF16), (5436, 9524, 9920, ac.BF16), (4139, 12620, 12224, ac.E4M3), (565, 23296, 3712, ac.BF16)]
+    problems += [(int(2 ** rng.uniform(9, 13.2)), int(2 ** rng.uniform(9, 15.6)) // 4 * 4, int(2 ** rng.uniform(12, 13.8)) // 16 * 16, rng.choice([ac.BF16, ac.E4M3]))
+                 for _ in range(1500)]
+    seen = 0
+    for p, (st, _, got) in zip(problems, launches([case(*p) for p in problems])):
+        products = [(name, v) for name, v in got if matrix_core(name)]
+        for name, v in products if len(products) == 2 else []:
+            tile = re.search(r"gemm_tn_tile_ring\w*?Li(\d+)ELi\d+ELi(\d+)E", name)
+            if tile and v["splits"] == 1 and v["tail_tiles"] == 0:
+                rows, cols = int(tile.group(1)), int(tile.group(2))
+                seen += 1
+                assert rows == 128 or -(-v["M"] // rows) * -(-v["N"] // cols) > 128, (p, name, v)
+    assert seen >= 100

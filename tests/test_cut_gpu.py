@@ -30,3 +30,15 @@ def test_block_scaled(M, N, K):
     C = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device="cuda")
     gemm_kernels.gemm_tn_mxfp8(x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn), sx, sw, C)
     assert torch.equal(C, want.to(torch.bfloat16))
+
+
+# pieces that run on other tiles than a plan with splits of K has, on the kernel for few outputs, or split in the room that the query asks for
+@pytest.mark.parametrize("M,N,K,dt", [(565, 23296, 3712, torch.bfloat16), (4113, 8023, 880, torch.bfloat16), (3094, 16012, 4096, torch.float16),
+                                      (2302, 22144, 2048, torch.float8_e4m3fn)])
+def test_plain_pieces(M, N, K, dt):
+    test_plain(M, N, K, dt)
+
+
+@pytest.mark.parametrize("M,N,K", [(4143, 4096, 1920), (1480, 12160, 8320), (670, 23916, 2432), (3031, 6112, 7296)])
+def test_block_scaled_pieces(M, N, K):
+    test_block_scaled(M, N, K)
