@@ -194,7 +194,8 @@ int mi355_quantize_e4m3_scratch(const void *x, int x_dtype, int64_t n, void *x_q
  * (MI355_VARIANT_BASIC) with the planner's choice of tile and splits among the tiles this kernel
  * has: what mi355_gemm_plan reports for MI355_E4M3 operands of this shape and that variant,
  * except where plain operands get the nine-slot ring of 128 x 128 tiles (one row or column of
- * tiles, or tiles that make a single round), which the block-scaled kernel does not have.
+ * tiles, or tiles that make a single round), which the block-scaled kernel does not have, and
+ * where the call cuts the problem in two (mi355_gemm_pieces).
  * Counterpart in the reference: none (it has no fp8 path); same launcher contract as
  * mi355_gemm_tn (kernels/gemm_kernels/sm90a/gemm_test.cu:12-92), block format per the OCP
  * Microscaling Formats (MX) specification v1.0.
@@ -207,7 +208,9 @@ int mi355_gemm_tn_mxfp8(const void *A_q, const void *B_q, void *C,
                         int scales_shuffled, int out_dtype,
                         void *workspace, size_t workspace_bytes, void *stream);
 
-/* Workspace mi355_gemm_tn_mxfp8 wants: shuffled scales (unless already shuffled) + split partials. */
+/* Workspace mi355_gemm_tn_mxfp8 wants: shuffled scales (unless already shuffled) + split partials of what
+ * mi355_gemm_plan and mi355_gemm_pieces describe (a call that launches something else needs no more, and may
+ * leave this part unused). */
 size_t mi355_gemm_mx_workspace_bytes(int64_t M, int64_t N, int64_t K, int scales_shuffled);
 
 /* Argument check of mi355_gemm_tn_mxfp8 without pointers; runs without a GPU. */
@@ -258,8 +261,11 @@ int mi355_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int variant,
  * the rest runs as a problem of its own (mi355_gemm_plan then describes the first piece; the second is what
  * MI355_VARIANT_BASIC plans for its shape).  *first_rows x *first_cols receive the first piece's extent (M x N for one
  * launch); either may be NULL.  Explicit variants never cut; mi355_gemm_tn_mxfp8 cuts where this function says so for
- * MI355_E4M3 operands (and M > 64).  A call may also cut where this function reports one launch and mi355_gemm_plan no tail split,
- * or elsewhere than it reports, into a first piece of nearly whole rounds and a rest that needs no workspace.  Returns a negative
+ * MI355_E4M3 operands (and M > 64).  A call may also cut elsewhere than this function reports, or where it reports one launch, into
+ * a first piece of nearly whole rounds and a rest, both on tiles that neither this function nor mi355_gemm_plan describes:
+ * mi355_gemm_tn only where mi355_gemm_plan reports no tail split, mi355_gemm_tn_mxfp8 also where it reports one.  The same pieces
+ * are launched whatever the workspace: those of mi355_gemm_tn need none, those of mi355_gemm_tn_mxfp8 split K only in what
+ * mi355_gemm_mx_workspace_bytes asks for (the room of the launch that they replace).  Returns a negative
  * mi355_status for bad arguments.
  * Pure host function.  Counterpart in the reference: none (its Scheduler walks one tile grid per launch,
  * kernels/gemm_kernels/sm90a/gemm.cuh:168-212). */

@@ -61,3 +61,16 @@ def test_halves_cover_the_problem_and_stay_in_the_room(mx_launches):
                 assert (v["A"], v["B"]) == ((1 << 44) + m0 * K, (2 << 44) + n0 * K) and m0 + v["M"] <= M and n0 + v["N"] <= N
                 if v["splits"] > 1 and M > 64:
                     assert 4 * v["splits"] * v["M"] * v["N"] <= (need if room is None else 0), p
+
+
+def test_what_is_cut_besides_what_the_queries_report(mx_launches):
+    """As the header says: also problems that they give a tail split, and never more room than the query's."""
+    abi, tails, cut_tails = ac.load(), 0, 0
+    problems = [(6144, 4096, 4096)] + problems_of(1200, 9)
+    for p, (st, need, got) in zip(problems, mx_launches(problems)):
+        products = [v for name, v in got if matrix_core(name)]
+        if ac.plan(abi, *p, ac.E4M3)[4] > 0 and abi.mi355_gemm_pieces(*p, ac.E4M3, ac.AUTO, None, None) == 1:
+            tails += 1
+            cut_tails += len(products) == 2
+            assert need > 0 and len(products) <= 2, p
+    assert tails >= 20 and cut_tails >= 10
