@@ -270,7 +270,8 @@ def check_hazard_distances(asm_path, kernel_filter=None):
 def check_no_scratch(asm_path):
     """The ring kernels count the vector-memory instructions in flight by hand (s_waitcnt vmcnt(N) with N
     derived from the copies they issue); a register spill would add loads and stores of its own to
-    that count.  No kernel of the file may use scratch memory or spill a vector register.  Returns
+    that count.  The quantiser that keeps its tensor in registers would read and write them again
+    through memory.  No kernel of the file may use scratch memory or spill a vector register.  Returns
     the number of kernels checked."""
     src = open(asm_path).read()
     sizes = [int(x) for x in re.findall(r'^\s*\.private_segment_fixed_size:\s*(\d+)', src, re.M)]

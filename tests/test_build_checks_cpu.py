@@ -269,3 +269,11 @@ def test_fallback_build_of_the_block_scaled_kernel_passes_the_hazard_checks(tmp_
     assert len(loads) > 100
     for i in loads:
         assert text[i + 1].strip().startswith("s_waitcnt vmcnt(0)"), text[i:i + 2]
+
+
+def test_kernels_whose_registers_are_counted_on_are_checked_for_scratch_memory():
+    """The tile kernels count their loads in flight, and the quantiser that reads a tensor once keeps it in registers."""
+    import build
+    csrc = os.path.join(PKG, "csrc")
+    holds = [f for f in build.HIP_SOURCES if "wait_vmcnt<" in open(os.path.join(csrc, f)).read()]
+    assert "quantize_e4m3.hip" in holds and set(holds) <= set(build.NO_SCRATCH_SOURCES)
