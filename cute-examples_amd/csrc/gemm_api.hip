@@ -739,8 +739,9 @@ int run_variant(const void* A, const void* B, void* C, int64_t M, int64_t N, int
 // only C is in the way (N or ldc not a multiple of 4, C not 8-byte aligned), with A and B repacked when they are (and C padded
 // when its rows are out of reach) and the workspace holds the copies; few outputs on gemm_tn_slices as they are, where the workspace
 // would hold the copies or none are made.  *handled says whether it was done.  Measured, both
-// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 116 us; fp16 515 x 2050 x 4100 repacked
-// 30 us (37 on another box), as it is 26.
+// sides: bf16 1000 x 50257 x 768 with a padded copy of B and of C 174 us, direct 116 us; rows of C at odd addresses under tiles of 256
+// rows and 32 k-steps and more, 80 sizes, 3-21 % shorter directly than by a padded copy (bf16 4096 x 14337 x 2048 231 -> 194 us, fp16 8192 x
+// 8193 x 4096 432 -> 398); fp16 515 x 2050 x 4100 repacked 30 us (37 on another box), as it is 26.
 int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc,
                   int in_dtype, int out_dtype, float scale, const float* scale_a, const float* scale_b, void* workspace,
                   size_t workspace_bytes, hipStream_t s, WorkspaceMode mode, bool* handled) {
@@ -753,10 +754,9 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   const bool large = repack_plan(A, B, C, M, N, K, lda, ldb, ldc, in_dtype, &r);
   if (large && (!workspace || (uintptr_t)workspace % 256 != 0)) return MI355_OK;   // the contract: the generic kernel then
   const bool ab_aligned = (uintptr_t)A % 16 == 0 && (uintptr_t)B % 16 == 0;
-  const bool c_aligned = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 8 == 0, odd = ldc % 2 != 0 || (uintptr_t)C % 4 != 0;
+  const bool c_aligned = N % 4 == 0 && ldc % 4 == 0 && (uintptr_t)C % 8 == 0;
   const int v = auto_variant(M, Np, Kp, in_dtype);
   const int v_ragged = v == MI355_VARIANT_ALTERNATE ? MI355_VARIANT_BASIC : v;   // the two kernels that take rows of any alignment
-  const bool pads_odd = !c_aligned && odd && v_ragged == MI355_VARIANT_BASIC && mi355::ring_odd_rows_padded(M, Np, Kp, (int)es);
   // The product on operands that the tiled kernels can address, with what is left of the workspace: into the caller's C, or
   // (padded) into a copy of it whose rows are aligned and have room for Np columns.
   const auto product = [&](const void* a, const void* b, int64_t ld_a, int64_t ld_b, void* c, int64_t ld_c, bool padded, void* ws,
@@ -817,33 +817,29 @@ int run_unaligned(const void* A, const void* B, void* C, int64_t M, int64_t N, i
   // What the repacked (aligned) problem wants for its own splits.  The streaming kernel insists
   // on the workspace of its K split, so a lenient call repacks only when the rest covers it.
   const size_t inner = mi355_gemm_workspace_bytes(M, Np, Kp, in_dtype, MI355_VARIANT_AUTO);
-  for (const bool pads_c : {true, false}) {
-    if (pads_c ? in_reach && !pads_odd : !in_reach) continue;
-    if (pads_c && !(r.c && tile256_ok(M, Np, Kp, ld_a, ld_b, r.ld_c, in_dtype))) continue;
-    const size_t bytes_c = pads_c ? r.bytes_c : 0, packed = r.bytes_a + bytes_b + bytes_c;
-    const bool fits = !packed || (workspace_bytes >= packed && (workspace_bytes - packed >= inner || (!strict && v != MI355_VARIANT_SKINNY)));
-    *handled = *handled || strict;   // refused unless one of them fits
-    if (!fits) continue;
-    *handled = true;
-    if (r.a || copies_b) {
-      const int form = slices_form((r.a ? M * K * es : 0) + (copies_b ? N * K * es : 0));
-      if (form >= 0) return on_slices(form);
-    }
-    if (packed && mode == kStrictDry) return MI355_OK;
-    uint8_t* wa = (uint8_t*)workspace;
-    uint8_t* wb = wa + r.bytes_a;
-    uint8_t* wc = wb + bytes_b;
-    uint8_t* rest = wc + bytes_c;
-    const size_t rest_bytes = workspace_bytes - packed;
-    const mi355::RepackOperand pack_a = {(const uint8_t*)A, r.a ? M : 0, lda * es, wa, r.ld_ab * es};
-    const mi355::RepackOperand pack_b = {(const uint8_t*)B, copies_b ? N : 0, ldb * es, wb, r.ld_ab * es};
-    if (mi355::launch_repack_rows(pack_a, pack_b, K * es, (int)es, s) != 0) return MI355_ERR_LAUNCH;
-    const int st = product(r.a ? wa : A, copies_b ? wb : B, ld_a, ld_b, pads_c ? (void*)wc : C, pads_c ? r.ld_c : ldc, pads_c,
-                           rest_bytes ? rest : nullptr, rest_bytes);
-    if (st != MI355_OK || !pads_c) return st;
-    return mi355::launch_copy_out(wc, M, N, r.ld_c, C, ldc, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
+  const bool pads_c = !in_reach;
+  if (pads_c && !(r.c && tile256_ok(M, Np, Kp, ld_a, ld_b, r.ld_c, in_dtype))) return MI355_OK;
+  const size_t bytes_c = pads_c ? r.bytes_c : 0, packed = r.bytes_a + bytes_b + bytes_c;
+  const bool fits = !packed || (workspace_bytes >= packed && (workspace_bytes - packed >= inner || (!strict && v != MI355_VARIANT_SKINNY)));
+  *handled = fits || strict;
+  if (!fits) return strict ? MI355_ERR_SCRATCH : MI355_OK;
+  if (r.a || copies_b) {
+    const int form = slices_form((r.a ? M * K * es : 0) + (copies_b ? N * K * es : 0));
+    if (form >= 0) return on_slices(form);
   }
-  return *handled ? MI355_ERR_SCRATCH : MI355_OK;
+  if (packed && mode == kStrictDry) return MI355_OK;
+  uint8_t* wa = (uint8_t*)workspace;
+  uint8_t* wb = wa + r.bytes_a;
+  uint8_t* wc = wb + bytes_b;
+  uint8_t* rest = wc + bytes_c;
+  const size_t rest_bytes = workspace_bytes - packed;
+  const mi355::RepackOperand pack_a = {(const uint8_t*)A, r.a ? M : 0, lda * es, wa, r.ld_ab * es};
+  const mi355::RepackOperand pack_b = {(const uint8_t*)B, copies_b ? N : 0, ldb * es, wb, r.ld_ab * es};
+  if (mi355::launch_repack_rows(pack_a, pack_b, K * es, (int)es, s) != 0) return MI355_ERR_LAUNCH;
+  const int st = product(r.a ? wa : A, copies_b ? wb : B, ld_a, ld_b, pads_c ? (void*)wc : C, pads_c ? r.ld_c : ldc, pads_c,
+                         rest_bytes ? rest : nullptr, rest_bytes);
+  if (st != MI355_OK || !pads_c) return st;
+  return mi355::launch_copy_out(wc, M, N, r.ld_c, C, ldc, s) == 0 ? MI355_OK : MI355_ERR_LAUNCH;
 }
 
 int run_gemm(const void* A, const void* B, void* C, int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb,

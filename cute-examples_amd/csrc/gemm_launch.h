@@ -96,9 +96,6 @@ struct CutPiece {
 };
 CutPiece cut_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scaled, size_t room);
 double ring_shortest_us(int64_t M, int64_t N, int64_t K, int elem_bytes);   // estimate of the single-group kernel's plan
-// Whether MI355_VARIANT_AUTO computes a C whose rows start at odd 2-byte addresses into a padded copy that is then copied out (if
-// there is memory for it) instead of storing it directly.
-bool ring_odd_rows_padded(int64_t M, int64_t N, int64_t K, int elem_bytes);
 // C = rne(scale * sum_s partial[s]) for partial laid out [splits][M][partial_columns(N)] in fp32.
 int launch_splitk_reduce(const float* partial, const GemmArgs& g, int out_dtype, hipStream_t stream);
 int launch_tile_ring(const GemmArgs& g, int in_dtype, int out_dtype, int tile, hipStream_t stream);

@@ -335,27 +335,6 @@ RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_spli
   return cut;
 }
 
-// Rows of C that start at odd 2-byte addresses are stored directly (tile_store.h), but for a region where they go through a padded
-// copy: from 32 k-steps on, where tiles of 256 rows and the copy (0.1 us per MB moved and 10 us) are estimated to take no longer
-// than the 128 x 128 tiles do.  Storing directly has become the shorter way there too (bf16 4096 x 14337 x 2048 239 us by the copy,
-// 201 directly; fp16 8192 x 8193 x 4096 489, 450; e4m3 2048 x 4097 x 8192 79, 74), as on all of 50 problems of M = 360...9335, N =
-// 800...50257 and 4...110 k-steps (13 % on average against the copy or 128 x 128 tiles, none slower by more than 0.6 %), so the
-// region is as narrow as what is relied on about this route (test_dispatch_cpu.py) lets it be.
-bool ring_odd_rows_padded(int64_t M, int64_t N, int64_t K, int elem_bytes) {
-  if (k_steps_of(K, elem_bytes) < 2 * kShortSteps) return false;
-  bool along_m = false;
-  const int64_t first = ring_first_piece(M, N, K, elem_bytes, &along_m);
-  const int64_t m1 = along_m ? first : M, n1 = along_m ? N : first, m2 = along_m ? M - first : M, n2 = along_m ? N : N - first;
-  const auto tall_unsplit = [&](int64_t m, int64_t n) {   // sums of a K split are rounded and stored by another kernel
-    return ring_tile_rows(ring_tile_edge(m, n, K, elem_bytes)) == 256 && ring_splits(m, n, K, elem_bytes) == 1;
-  };
-  if (first > 0 ? !tall_unsplit(m1, n1) && !tall_unsplit(m2, n2) : !tall_unsplit(M, N)) return false;
-  const double plan_us = first > 0 ? shortest_us(m1, n1, K, elem_bytes) + shortest_us(m2, n2, K, elem_bytes) + kSecondLaunchUs
-                                   : shortest_us(M, N, K, elem_bytes);
-  const double copy_mb = (double)M * (double)N * 4e-6;
-  return plan_us + 0.1 * copy_mb + 10.0 < 1.03 * estimate_us(128, M, N, K, elem_bytes);
-}
-
 // K splits for the single-group kernel on the tile ring_tile_edge picks.
 int ring_splits(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scaled) {
   return uniform_splits(tiles_of(M, N, ring_tile_edge(M, N, K, elem_bytes, block_scaled)), k_steps_of(K, elem_bytes));

@@ -76,9 +76,9 @@ enum mi355_status {
  *             problem the tiled kernels cannot address (K*elem_bytes % 16, strides, pointers);
  *             without it such a problem, or a large one with N or ldc % 4 != 0, runs on the slow
  *             generic kernel.  With it, an output whose rows only its element type aligns is stored
- *             by the tiled kernels directly, or computed in a padded copy of it that the workspace
- *             holds and copied out, whichever is shorter (mi355_gemm_select_variant still reports
- *             SIMPLE)
+ *             by the tiled kernels directly, or where its rows are out of their reach computed in a
+ *             padded copy of it that the workspace holds and copied out (mi355_gemm_select_variant
+ *             still reports SIMPLE)
  *             A product of few outputs that MI355_VARIANT_AUTO would stream or tile runs on a kernel
  *             for those instead where that is estimated to be faster, without a workspace
  *             (mi355_gemm_select_variant, mi355_gemm_plan and the workspace query still report the

@@ -165,9 +165,9 @@ def test_streaming_kernel_has_a_form_for_each_kind_of_rows(launches, M, N, K, sp
         assert "Lb1E" not in got[0][0]
 
 
-# What the padded copy of C is for besides: rows at odd 2-byte addresses under a plan with tiles of 256 rows (the planner's choice
-# is held here at sizes where it is clear; everything else is the same product).
-@pytest.mark.parametrize("M,N,K,in_dt,padded", [(4096, 14337, 2048, ac.BF16, True), (8192, 8193, 4096, ac.F16, True), (2048, 4097, 8192, ac.E4M3, True),
+# Rows at odd 2-byte addresses under a plan with tiles of 256 rows are stored directly, with or without room for a padded copy of C
+# (which took 3-21 % longer on 80 sizes).
+@pytest.mark.parametrize("M,N,K,in_dt,padded", [(4096, 14337, 2048, ac.BF16, False), (8192, 8193, 4096, ac.F16, False), (2048, 4097, 8192, ac.E4M3, False),
                                                 (1000, 50257, 768, ac.BF16, False), (8192, 8193, 512, ac.BF16, False), (9335, 9969, 1536, ac.BF16, False)])
 def test_rows_of_c_at_odd_addresses(launches, M, N, K, in_dt, padded):
     cases = [case(M, N, K, in_dt), case(M, N, K, in_dt, c=C + 2), case(M, N, K, in_dt, room=256), case(M, N, K, in_dt, noalloc=True),

@@ -111,7 +111,7 @@ def test_tail_split_and_two_pieces(abi, M, N, K, dt, pieces):
     assert pieces == 2 or ac.plan(abi, M, Np, K, code)[4] > 0
     A, B = operand(M, K, dt, 3), operand(N, K, dt, 4)
     inner = max(abi.mi355_gemm_workspace_bytes(M, Np, K, code, ac.AUTO), 256)
-    # rows at even 2-byte addresses; at odd ones with room for the split's planes only (stored directly), and with a padded copy of C
+    # rows at even 2-byte addresses; at odd ones with room for the split's planes only, and with more
     for offset, pad, ws_bytes in ((0, 0, inner), (1, 0, inner), (0, 1, inner), (1, 1, None)):
         C, kept = run(abi, A, B, offset, N + pad, ws_bytes=ws_bytes)
         assert kept
@@ -129,7 +129,7 @@ def test_aligned_rows_with_a_partial_last_column(abi, M, N, K, dt):
         close_everywhere(C, A, B)
 
 
-# Rows of C at odd 2-byte addresses where the library computes into a padded copy: one launch, a tail split, two launches.
+# Rows of C at odd 2-byte addresses under plans with tiles of 256 rows: one launch, a tail split, two launches.
 @pytest.mark.parametrize("M,N,K,dt", [(2049, 2051, 4096, torch.bfloat16), (513, 8195, 4096, torch.float16), (2049, 6145, 4096, torch.float8_e4m3fn),
                                       (2049, 6145, 2056, torch.bfloat16), (2049, 8195, 4096, torch.bfloat16), (4096, 4111, 4096, torch.bfloat16),
                                       (1025, 6147, 4090, torch.float16)])
