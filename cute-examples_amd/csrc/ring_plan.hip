@@ -269,7 +269,11 @@ int64_t ring_first_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool* 
 // instead of the tile or its estimate is the shortest.
 CutPiece cut_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_scaled, size_t room) {
   const int64_t steps = k_steps_of(K, elem_bytes);
-  const int split_tile = ring_tile_edge(M, N, K, elem_bytes, block_scaled), splits = uniform_splits(tiles_of(M, N, split_tile), steps);
+  int split_tile = 0, splits = 1;
+  if (room > 0) {
+    split_tile = ring_tile_edge(M, N, K, elem_bytes, block_scaled);
+    splits = uniform_splits(tiles_of(M, N, split_tile), steps);
+  }
   const bool may_split = splits > 1 && (size_t)splits * (size_t)M * (size_t)N * sizeof(float) <= room;
   const bool single_round = tiles_of(M, N, 128) <= kCuSlots && steps >= kShortSteps;
   // (Block scales have no nine-slot ring; beside a split that there is room for, the factor would keep the small tile ahead wrongly.)
@@ -283,7 +287,7 @@ CutPiece cut_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_s
   }
   int form;
   const double us = slices_us(M, N, K, elem_bytes, block_scaled, &form);
-  if (us < p.us || slices_config(M, N, K, elem_bytes, block_scaled, {false, ring_tile_rows(p.tile), ring_tile_cols(p.tile), p.splits}) >= 0) {
+  if (form >= 0 && (us < p.us || slices_config(M, N, K, elem_bytes, block_scaled, {false, ring_tile_rows(p.tile), ring_tile_cols(p.tile), p.splits}) >= 0)) {
     p.slices = form;
     p.us = us < p.us ? us : p.us;   // what its rule takes is no longer than the tile
   }
