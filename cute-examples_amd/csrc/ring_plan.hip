@@ -303,8 +303,7 @@ CutPiece cut_piece(int64_t M, int64_t N, int64_t K, int elem_bytes, bool block_s
 // While the price was of other tiles than those launched (whose plan had counted on splits of K), 85 plain problems took 0.91 of the
 // uncut time, now 0.865; 60 block-scaled ones 0.97, now 0.92, four of them up to 5 % slower than with splits in room meant for others.
 // A plain problem that the queries describe as one launch with a tail split (tail_splits) stays one: its result is
-// MI355_VARIANT_BASIC's to the bit, and the cut would add in another order (a price: bf16 1056 x 26704 x 2176 149 us, cut 117).
-// Beyond 64 k-steps ring_first_piece's limit of rounds.
+// MI355_VARIANT_BASIC's to the bit, and the cut would add in another order.  Beyond 64 k-steps ring_first_piece's limit of rounds.
 RingCut ring_cut(int64_t M, int64_t N, int64_t K, int elem_bytes, bool tail_splits, bool block_scaled, size_t room) {
   RingCut cut = {0, false, false};
   cut.extent = ring_first_piece(M, N, K, elem_bytes, &cut.along_m);

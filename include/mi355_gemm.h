@@ -259,7 +259,7 @@ int mi355_gemm_plan(int64_t M, int64_t N, int64_t K, int in_dtype, int variant,
 /* How many launches of the GEMM kernel a call makes for this problem: 1, or 2 where MI355_VARIANT_AUTO cuts a
  * problem of the tiled kernel along N or M so that the first piece fills a whole number of rounds of workgroups and
  * the rest runs as a problem of its own (mi355_gemm_plan then describes the first piece; the second is what
- * MI355_VARIANT_BASIC plans for its shape).  *first_rows x *first_cols receive the first piece's extent (M x N for one
+ * MI355_VARIANT_BASIC plans for its shape, or the kernel for few outputs).  *first_rows x *first_cols receive the first piece's extent (M x N for one
  * launch); either may be NULL.  Explicit variants never cut; mi355_gemm_tn_mxfp8 cuts where this function says so for
  * MI355_E4M3 operands (and M > 64).  A call may also cut elsewhere than this function reports, or where it reports one launch, into
  * a first piece of nearly whole rounds and a rest, both on tiles that neither this function nor mi355_gemm_plan describes:
